@@ -16,8 +16,8 @@
 //            FP32 output layer and the masked data gradients (the same
 //            kernel on flipped, transposed weights, ReLU mask of the forward
 //            input fused); bias + ReLU fused in both
-//   k_wgrad  weight gradient, pixels as the K dimension, split-K with FP32
-//            atomics
+//   k_wgrad  weight and bias gradients, pixels as the K dimension, split-K
+//            with partial sums added in order (k_wgrad_sum)
 // Concatenations cost no copies: producers write into channel slices of the
 // concatenated tensor (row stride "ld").
 #include "kf_internal.h"
@@ -93,7 +93,7 @@ struct PackSrc {
 // stay in LDS while consecutive steps need the same ones (one input chunk
 // and the same output channels).
 // Cin must be a multiple of 32; ldx, ldy multiples of 8.
-constexpr int CBK = 32, CLD = CBK + 8;
+constexpr int CBK = 32;
 // LDS rows of the convolution tiles: 32 halves (64 bytes) per pixel or
 // weight row, 16-byte group q of row r stored at group q ^ ((r / 2) % 4), so
 // that the 16-byte reads of an MFMA operand (16 consecutive rows, one group)
@@ -710,69 +710,224 @@ __global__ __launch_bounds__(PackShape<TYP>::kThreads) void k_conv2_pack(const u
                       relu, nullptr);
 }
 
-// dW[tap, co, ci] += sum_p dY[p, co] * X[p + off(tap), ci] over one pixel chunk.
-// Tile 64 co x 64 ci, K step 32 pixels; LDS tiles are stored channel-major
-// (pixels contiguous) so each lane's 8 K values are one 16-byte read.
-__global__ __launch_bounds__(TB) void k_wgrad(const uint16_t* __restrict__ X, int ldx, int Cin,
-                                              const uint16_t* __restrict__ dY, int ldy, int Cout, int N, int H,
-                                              int W, int chunk, float* __restrict__ dW) {
-    __shared__ __attribute__((aligned(16))) uint16_t As[64 * CLD];  // [co][px]
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[64 * CLD];  // [ci][px]
-    const int P = N * H * W;
-    const int tap = blockIdx.y;
-    const int n_ci_t = (Cin + 63) / 64;
-    const int co0 = (blockIdx.z / n_ci_t) * 64, ci0 = (blockIdx.z % n_ci_t) * 64;
-    const int pbeg = blockIdx.x * chunk, pend = min(P, pbeg + chunk);
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-    f32x4 acc[4];
-    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const int lr = t >> 3, lc = (t & 7) * 8;  // pixel row 0..31, channel chunk
-    const int fr = lane & 15, fk = (lane >> 4) * 8;
-    for (int pk = pbeg; pk < pend; pk += 32) {
-        const int p = pk + lr;
-        uint16_t av[8], bv[8];
-        bool pv = p < pend;
-        uint4 a4 = make_uint4(0, 0, 0, 0), b4 = make_uint4(0, 0, 0, 0);
-        if (pv && co0 + lc < Cout) a4 = *(const uint4*)(dY + (size_t)p * ldy + co0 + lc);
-        if (pv && ci0 + lc < Cin) {
-            int n_ = p / (H * W), rem = p - n_ * H * W, y = rem / W, x = rem - y * W;
-            int yy = y + dy, xx = x + dx;
-            if (yy >= 0 && yy < H && xx >= 0 && xx < W)
-                b4 = *(const uint4*)(X + (size_t)((n_ * H + yy) * W + xx) * ldx + ci0 + lc);
-        }
-        memcpy(av, &a4, 16);
-        memcpy(bv, &b4, 16);
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            As[(lc + j) * CLD + lr] = av[j];
-            Bs[(lc + j) * CLD + lr] = bv[j];
-        }
-        __syncthreads();
-        bf16x8 a = __builtin_bit_cast(bf16x8, *(const uint4*)&As[(wv * 16 + fr) * CLD + fk]);
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-            bf16x8 b = __builtin_bit_cast(bf16x8, *(const uint4*)&Bs[(nb * 16 + fr) * CLD + fk]);
-            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[nb], 0, 0, 0);
-        }
+// ---------------------------------------------------------- weight gradient
+// dW[tap, co, ci] = sum_p dY[p, co] * X[p + off(tap), ci] and db[co] =
+// sum_p dY[p, co], with the pixels as the MFMA's K dimension.
+//
+// One wave owns a 32 co x 32 ci tile for all 9 taps (144 accumulator
+// registers) and walks strips of 32 pixels x `rows` rows downwards.  An MFMA
+// operand wants 8 consecutive K values (pixels) of one channel per lane while
+// the tensors are NHWC: lane (l, g) loads channels 2l, 2l + 1 of the 8
+// pixels 8g .. 8g + 7 of dY's row as dwords, and of pixels 8g - 1 .. 8g + 8
+// of X's row, and joins pixel pairs with byte permutes: even pairs serve tap
+// offset dx = 0, odd pairs dx = -1 and +1, so X is loaded once for all three.
+// X row y then meets dY rows y - 1, y, y + 1, which stay in registers: per
+// row 18 loads of 256 bytes, 26 permutes and 36 MFMAs, and nothing goes
+// through LDS.  Every row is read through a buffer resource of that row
+// alone, so pixels off either end of it are offsets out of range (zeros).
+// The four waves of a block add their tiles in LDS, in order, and the block
+// writes one partial sum; k_wgrad_sum adds those, in order as well, so a
+// gradient has the same bits on every run.
+//
+// Bound: at full resolution (32 -> 32 channels) the reads of X and dY, in
+// the wide layers the matrix cores.  8 x 256x256 images, all 19 layers with
+// the bias gradients: 7.16 ms (64 x 64 tiles per tap, operands transposed by
+// 2-byte LDS stores, FP32 atomics; one thread per channel for the biases)
+// -> 0.61 ms (k_wgrad 0.52, k_wgrad_sum 0.09).
+constexpr int kWgTile = 32, kWgSums = 9 * kWgTile * kWgTile;  // floats of one tile's partial sum
+constexpr int kWgBlocks = 512;  // 2 blocks per CU: 2 waves per SIMD (their registers allow no more)
+
+// How a layer's weight gradient is split: strips of 32 pixels x rows, and
+// `splits` blocks per tile, each adding up every splits-th group of four
+// strips.  rows is halved from the image height until the blocks fill the
+// chip twice over (2 per CU), not below 4 rows: a strip reads two rows of X
+// beyond its own.
+struct WgradPlan {
+    int rows, nseg, nyb, strips, splits, tiles;
+    size_t part;  // floats of one split's partial sums (weights, then biases)
+    WgradPlan(int N, int H, int W, int Cin, int Cout) {
+        tiles = (Cin / kWgTile) * (Cout / kWgTile);
+        nseg = (W + 31) / 32;
+        const int64_t want = 4 * (int64_t)std::max(1, kWgBlocks / tiles);  // strips that fill the chip
+        rows = H;
+        while (rows > 4 && (int64_t)N * nseg * ((H + rows - 1) / rows) < want) rows = (rows + 1) / 2;
+        nyb = (H + rows - 1) / rows;
+        const int64_t n = (int64_t)N * nseg * nyb;
+        if (n >= (1 << 30)) throw Error("conv: too many strips");
+        strips = (int)n;
+        splits = (int)std::min<int64_t>((n + 3) / 4, want / 4);
+        part = (size_t)9 * Cin * Cout + Cout;
     }
+    size_t floats() const { return part * splits; }
+};
+
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_wgrad(
+    const uint16_t* __restrict__ X, int ldx, int Cin, const uint16_t* __restrict__ dY, int ldy, int Cout, int H, int W,
+    int rows, int nseg, int nyb, int strips, float* __restrict__ part) {
+    __shared__ __attribute__((aligned(16))) float red[kWgSums + kWgTile];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l = lane & 15, g = lane >> 4;
+    const int n_ci = Cin / kWgTile;
+    const int co0 = (int)(blockIdx.y / n_ci) * kWgTile, ci0 = (int)(blockIdx.y % n_ci) * kWgTile;
+    const bool bias = ci0 == 0;  // the tiles of the first input channels add up dY too
+    const int ldx2 = 2 * ldx, ldy2 = 2 * ldy;
+    f32x4 acc[9][2][2], accb[2];
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
+    for (int k = 0; k < 9; ++k)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) acc[k][f >> 1][f & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    accb[0] = accb[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const bf16x8 ones = {1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f};
+    struct Row {
+        uint32_t x[10], d[8];
+    };
+    struct Frag {  // 8 pixels of channels 2l (lo) and 2l + 1 (hi)
+        uint32_t lo[4], hi[4];
+    };
+    auto bf8 = [](const uint32_t (&v)[4]) __attribute__((always_inline)) {
+        return __builtin_bit_cast(bf16x8, make_uint4(v[0], v[1], v[2], v[3]));
+    };
+    auto join_lo = [](uint32_t a, uint32_t b) __attribute__((always_inline)) { return __builtin_amdgcn_perm(b, a, 0x05040100u); };
+    auto join_hi = [](uint32_t a, uint32_t b) __attribute__((always_inline)) { return __builtin_amdgcn_perm(b, a, 0x07060302u); };
+    for (int strip = (int)blockIdx.x * 4 + wv; strip < strips; strip += (int)gridDim.x * 4) {
+        const int x0 = (strip % nseg) * 32, rest = strip / nseg;
+        const int y0 = (rest % nyb) * rows, n = rest / nyb, y1 = min(H, y0 + rows);
+        const int vx = (x0 + 8 * g - 1) * ldx2 + 2 * (ci0 + 2 * l), vd = (x0 + 8 * g) * ldy2 + 2 * (co0 + 2 * l);
+        // slots of pixels past the row's end: their dY is zero, and X must
+        // be too (zero times infinity); only dx = -1 reads a pixel there
+        uint32_t keep[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int co = co0 + wv * 16 + (lane >> 4) * 4 + i;
-            const int ci = ci0 + nb * 16 + (lane & 15);
-            if (co < Cout && ci < Cin) atomicAdd(&dW[((size_t)tap * Cout + co) * Cin + ci], acc[nb][i]);
+            const int px = x0 + 8 * g + 2 * i;
+            keep[i] = px + 1 < W ? ~0u : (px < W ? 0xffffu : 0u);
         }
+        // X row y and dY row y + 1 (rows that do not exist or belong to
+        // another strip read zeros and touch no memory)
+        auto fetch = [&](int y, Row& r) __attribute__((always_inline)) {
+            const bool okx = y >= 0 && y <= y1 && y < H, okd = y + 1 >= y0 && y + 1 < y1;
+            const __amdgpu_buffer_rsrc_t rx =
+                buffer_rsrc(X + ((size_t)n * H + (okx ? y : 0)) * W * ldx, okx ? (uint32_t)W * ldx2 : 0u);
+            const __amdgpu_buffer_rsrc_t rd =
+                buffer_rsrc(dY + ((size_t)n * H + (okd ? y + 1 : 0)) * W * ldy, okd ? (uint32_t)W * ldy2 : 0u);
+#pragma unroll
+            for (int j = 0; j < 10; ++j) r.x[j] = __builtin_amdgcn_raw_buffer_load_b32(rx, (uint32_t)(vx + j * ldx2), 0, 0);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) r.d[j] = __builtin_amdgcn_raw_buffer_load_b32(rd, (uint32_t)(vd + j * ldy2), 0, 0);
+        };
+        auto pack_d = [&](const Row& r, Frag& a) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                a.lo[i] = join_lo(r.d[2 * i], r.d[2 * i + 1]);
+                a.hi[i] = join_hi(r.d[2 * i], r.d[2 * i + 1]);
+            }
+        };
+        Frag a[3];  // dY rows y - 1, y, y + 1
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[0].lo[i] = a[0].hi[i] = a[1].lo[i] = a[1].hi[i] = 0u;
+        Row cur;
+        fetch(y0 - 1, cur);
+#pragma unroll 1
+        for (int y = y0 - 1; y <= y1; ++y) {
+            pack_d(cur, a[2]);
+            Frag b[3];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                b[1].lo[i] = join_lo(cur.x[2 * i + 1], cur.x[2 * i + 2]);
+                b[1].hi[i] = join_hi(cur.x[2 * i + 1], cur.x[2 * i + 2]);
+                b[2].lo[i] = join_lo(cur.x[2 * i + 2], cur.x[2 * i + 3]);
+                b[2].hi[i] = join_hi(cur.x[2 * i + 2], cur.x[2 * i + 3]);
+            }
+            b[0].lo[0] = join_lo(cur.x[0], cur.x[1]) & keep[0];
+            b[0].hi[0] = join_hi(cur.x[0], cur.x[1]) & keep[0];
+#pragma unroll
+            for (int i = 1; i < 4; ++i) {
+                b[0].lo[i] = b[2].lo[i - 1] & keep[i];
+                b[0].hi[i] = b[2].hi[i - 1] & keep[i];
+            }
+            fetch(y + 1, cur);  // its registers are free: the next row comes in beside the MFMAs
+            const bf16x8 bl[3] = {bf8(b[0].lo), bf8(b[1].lo), bf8(b[2].lo)};
+            const bf16x8 bh[3] = {bf8(b[0].hi), bf8(b[1].hi), bf8(b[2].hi)};
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {  // tap row k meets dY row y + 1 - k
+                const int yd = y + 1 - k;
+                if (yd < y0 || yd >= y1) continue;
+                const bf16x8 al = bf8(a[2 - k].lo), ah = bf8(a[2 - k].hi);
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx) {
+                    acc[3 * k + dx][0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bl[dx], acc[3 * k + dx][0][0], 0, 0, 0);
+                    acc[3 * k + dx][0][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh[dx], acc[3 * k + dx][0][1], 0, 0, 0);
+                    acc[3 * k + dx][1][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl[dx], acc[3 * k + dx][1][0], 0, 0, 0);
+                    acc[3 * k + dx][1][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh[dx], acc[3 * k + dx][1][1], 0, 0, 0);
+                }
+            }
+            if (bias && y + 1 >= y0 && y + 1 < y1) {  // each of the strip's rows once
+                accb[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf8(a[2].lo), ones, accb[0], 0, 0, 0);
+                accb[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf8(a[2].hi), ones, accb[1], 0, 0, 0);
+            }
+            a[0] = a[1];
+            a[1] = a[2];
+        }
+    }
+    // tile[tap][co][ci]: an accumulator's element i is row (co) 4g + i, column
+    // (ci) l of its 16 x 16 block, whose channels are the even or odd ones
+#pragma unroll 1
+    for (int w = 0; w < 4; ++w) {
+        if (wv == w) {
+#pragma unroll
+            for (int k = 0; k < 9; ++k)
+#pragma unroll
+                for (int fa = 0; fa < 2; ++fa)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float2* at = (float2*)&red[(k * kWgTile + 2 * (4 * g + i) + fa) * kWgTile + 2 * l];
+                        const float2 old = w ? *at : make_float2(0.f, 0.f);
+                        *at = make_float2(old.x + acc[k][fa][0][i], old.y + acc[k][fa][1][i]);
+                    }
+            if (bias && l == 0)  // every column of the products with ones is the sum
+#pragma unroll
+                for (int fa = 0; fa < 2; ++fa)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        float* at = &red[kWgSums + 2 * (4 * g + i) + fa];
+                        *at = (w ? *at : 0.f) + accb[fa][i];
+                    }
+        }
+        __syncthreads();
+    }
+    float* out = part + blockIdx.x * ((size_t)9 * Cin * Cout + Cout);
+    for (int i = threadIdx.x; i < kWgSums / 4; i += TB) {
+        const int tap = i / (kWgTile * kWgTile / 4), r = i % (kWgTile * kWgTile / 4);
+        const int co = r / (kWgTile / 4), c4 = r % (kWgTile / 4);
+        *(float4*)&out[((size_t)tap * Cout + co0 + co) * Cin + ci0 + 4 * c4] = *(const float4*)&red[4 * i];
+    }
+    if (bias && threadIdx.x < kWgTile) out[(size_t)9 * Cin * Cout + co0 + threadIdx.x] = red[kWgSums + threadIdx.x];
 }
 
-__global__ void k_bias_grad(const uint16_t* __restrict__ dY, int ldy, int Cout, int P, int chunk, float* db) {
-    int pbeg = blockIdx.x * chunk, pend = min(P, pbeg + chunk);
-    for (int c = threadIdx.x; c < Cout; c += blockDim.x) {
-        float s = 0.0f;
-        for (int p = pbeg; p < pend; ++p) s += bf2f(dY[(size_t)p * ldy + c]);
-        atomicAdd(&db[c], s);
+// dW, db = the sum of the partial sums, in order.  16 columns of 4 floats per
+// block, 16 threads over the splits of each: a layer of 9216 weights has too
+// few columns to hide the reads of its 512 splits otherwise.
+__global__ __launch_bounds__(TB) void k_wgrad_sum(const float* __restrict__ part, int splits, uint32_t n4, uint32_t nw4,
+                                                 float* __restrict__ dW, float* __restrict__ db) {
+    __shared__ float4 red[16][16];
+    const uint32_t c = threadIdx.x & 15u, s0 = threadIdx.x >> 4, col = blockIdx.x * 16u + c;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (col < n4) {
+        const float4* p = (const float4*)part + col;
+#pragma unroll 8
+        for (int s = s0; s < splits; s += 16) {
+            const float4 v = p[(size_t)s * n4];
+            a = make_float4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w);
+        }
+    }
+    red[s0][c] = a;
+    __syncthreads();
+    if (s0 == 0 && col < n4) {
+        for (int s = 1; s < 16; ++s) {
+            const float4 v = red[s][c];
+            a = make_float4(a.x + v.x, a.y + v.y, a.z + v.z, a.w + v.w);
+        }
+        if (col < nw4) ((float4*)dW)[col] = a;
+        else ((float4*)db)[col - nw4] = a;
     }
 }
 
@@ -1094,15 +1249,18 @@ void conv_dgrad(const uint16_t* dY, int ldy, int Cout, const uint16_t* Wd, int C
                 int ldx, const uint16_t* Xf, int ldxf, hipStream_t st) {
     conv_launch(dY, ldy, Cout, Wd, nullptr, Cin, N, H, W, dX, ldx, nullptr, 0, Cin, Xf, ldxf, 0, st);
 }
+// dW (9 x Cout x Cin) and db of one layer, both overwritten; part: a
+// workspace of WgradPlan(...).floats() floats.  Channels are multiples of 32.
 void conv_wgrad(const uint16_t* X, int ldx, int Cin, const uint16_t* dY, int ldy, int Cout, int N, int H, int W,
-                float* dW, float* db, hipStream_t st) {
-    const int P = N * H * W;
-    int chunk = 2048;
-    while ((size_t)blocks(P, chunk) * 9 * blocks(Cout, 64) * blocks(Cin, 64) < 2048 && chunk > 64) chunk /= 2;
-    dim3 grid(blocks(P, chunk), 9, blocks(Cout, 64) * blocks(Cin, 64));
-    k_wgrad<<<grid, TB, 0, st>>>(X, ldx, Cin, dY, ldy, Cout, N, H, W, chunk, dW);
-    int bchunk = 1024;
-    k_bias_grad<<<blocks(P, bchunk), TB, 0, st>>>(dY, ldy, Cout, P, bchunk, db);
+                float* dW, float* db, float* part, hipStream_t st) {
+    if (Cin % kWgTile || Cout % kWgTile || ldx % 2 || ldy % 2) throw Error("conv: weight gradient of ragged channels");
+    if (2ull * W * std::max(ldx, ldy) >= (1u << 30)) throw Error("conv: image row too large for 32-bit indexing");
+    const WgradPlan p(N, H, W, Cin, Cout);
+    k_wgrad<<<dim3(p.splits, p.tiles), TB, 0, st>>>(X, ldx, Cin, dY, ldy, Cout, H, W, p.rows, p.nseg, p.nyb, p.strips,
+                                                    part);
+    const uint32_t nw4 = (uint32_t)(9 * Cin * Cout / 4), n4 = (uint32_t)(p.part / 4);
+    k_wgrad_sum<<<blocks(n4, 16), TB, 0, st>>>(part, p.splits, n4, nw4, dW, db);
+    KF_CHECK(hipGetLastError());
 }
 
 // ---------------------------------------------------------------- network
@@ -1129,6 +1287,12 @@ std::vector<ConvDef> unet_convs() {
     }
     c.push_back({kCh[0], 32});  // output conv, channels 0-2 used
     return c;
+}
+
+// Level (halvings of the resolution) of convolution k of that order.
+int conv_level(int k) {
+    if (k < 2 * kLevels) return k / 2;
+    return std::max(0, 2 * kLevels - 2 - k / 2);
 }
 
 struct Acts {
@@ -1200,6 +1364,8 @@ struct Unet {
     float *w32 = nullptr, *g32 = nullptr, *m32 = nullptr, *v32 = nullptr;
     std::vector<uint16_t*> wb, wd;
     float* d_loss = nullptr;
+    float* wg_part = nullptr;  // partial weight gradients of one layer
+    size_t wg_cap = 0;
     int step = 0;
     Acts act;
     float* rec_in = nullptr;
@@ -1229,8 +1395,8 @@ struct Unet {
     }
     ~Unet() {
         act.release();
-        for (void* p : {(void*)w32, (void*)g32, (void*)m32, (void*)v32, (void*)d_loss, (void*)rec_in, (void*)rec_tg,
-                        (void*)rec_out})
+        for (void* p : {(void*)w32, (void*)g32, (void*)m32, (void*)v32, (void*)d_loss, (void*)wg_part, (void*)rec_in,
+                        (void*)rec_tg, (void*)rec_out})
             if (p) (void)hipFree(p);
         for (auto p : wb) (void)hipFree(p);
         for (auto p : wd) (void)hipFree(p);
@@ -1340,28 +1506,38 @@ struct Unet {
         conv_fwd(act.u[0], kCh[0], kCh[0], wb[k], w32 + boff[k], 32, N, H(0), W(0), nullptr, 0, false, st, act.y, 4, 3);
     }
 
-    // backward from act.dy; accumulates into g32 (zeroed here)
+    // backward from act.dy; writes every gradient in g32
     void backward(hipStream_t st) {
         const int N = act.N;
         auto H = [&](int l) { return act.H >> l; };
         auto W = [&](int l) { return act.W >> l; };
-        k_zero_f32<<<blocks(nparams, TB), TB, 0, st>>>(g32, nparams);
+        // one workspace for the layers' partial sums, one after another on the
+        // stream (each at most about kWgBlocks tiles: 20 MB)
+        size_t need = 0;
+        for (size_t j = 0; j < defs.size(); ++j)
+            need = std::max(need, WgradPlan(N, H(conv_level((int)j)), W(conv_level((int)j)), defs[j].cin, defs[j].cout).floats());
+        if (need > wg_cap) {
+            if (wg_part) KF_CHECK(hipFree(wg_part));
+            wg_part = nullptr;
+            wg_cap = 0;
+            wg_part = dalloc<float>(need);
+            wg_cap = need;
+        }
         int k = (int)defs.size() - 1;
         // output conv
-        conv_wgrad(act.u[0], kCh[0], kCh[0], act.dy, 32, 32, N, H(0), W(0), g32 + woff[k], g32 + boff[k], st);
+        conv_wgrad(act.u[0], kCh[0], kCh[0], act.dy, 32, 32, N, H(0), W(0), g32 + woff[k], g32 + boff[k], wg_part, st);
         conv_dgrad(act.dy, 32, 32, wd[k], kCh[0], N, H(0), W(0), act.du[0], kCh[0], act.u[0], kCh[0], st);
         --k;
         for (int l = 0; l < kLevels - 1; ++l) {
             int ldc = kCh[l] + kCh[l + 1];
             // d_lb: input da[l], grad du[l]
             conv_wgrad(act.da[l], kCh[l], kCh[l], act.du[l], kCh[l], kCh[l], N, H(l), W(l), g32 + woff[k],
-                       g32 + boff[k], st);
+                       g32 + boff[k], wg_part, st);
             conv_dgrad(act.du[l], kCh[l], kCh[l], wd[k], kCh[l], N, H(l), W(l), act.dda[l], kCh[l], act.da[l], kCh[l],
                        st);
             --k;
             // d_la: input cat[l], grad dda[l]
-            conv_wgrad(act.cat[l], ldc, ldc, act.dda[l], kCh[l], kCh[l], N, H(l), W(l), g32 + woff[k], g32 + boff[k],
-                       st);
+            conv_wgrad(act.cat[l], ldc, ldc, act.dda[l], kCh[l], kCh[l], N, H(l), W(l), g32 + woff[k], g32 + boff[k], wg_part, st);
             conv_dgrad(act.dda[l], kCh[l], kCh[l], wd[k], ldc, N, H(l), W(l), act.dcat[l], ldc, act.cat[l], ldc, st);
             --k;
             // upsampled half of the concat -> gradient of the level below's output
@@ -1373,11 +1549,11 @@ struct Unet {
         }
         // bottleneck bb, ba
         int L = kLevels - 1;
-        conv_wgrad(act.t[L], kCh[L], kCh[L], act.dbt, kCh[L], kCh[L], N, H(L), W(L), g32 + woff[k], g32 + boff[k], st);
+        conv_wgrad(act.t[L], kCh[L], kCh[L], act.dbt, kCh[L], kCh[L], N, H(L), W(L), g32 + woff[k], g32 + boff[k], wg_part, st);
         conv_dgrad(act.dbt, kCh[L], kCh[L], wd[k], kCh[L], N, H(L), W(L), act.dt[L], kCh[L], act.t[L], kCh[L], st);
         --k;
         conv_wgrad(act.pl[L - 1], kCh[L - 1], kCh[L - 1], act.dt[L], kCh[L], kCh[L], N, H(L), W(L), g32 + woff[k],
-                   g32 + boff[k], st);
+                   g32 + boff[k], wg_part, st);
         conv_dgrad(act.dt[L], kCh[L], kCh[L], wd[k], kCh[L - 1], N, H(L), W(L), act.dpl[L - 1], kCh[L - 1], nullptr, 0,
                    st);
         --k;
@@ -1388,14 +1564,13 @@ struct Unet {
             k_pool_bwd<<<blocks(n8, TB), TB, 0, st>>>(act.dpl[l], kCh[l], act.cat[l], ldc, act.dcat[l], ldc, N, H(l),
                                                      W(l));
             // e_lb: input t[l], grad dcat[l][:, 0:C]
-            conv_wgrad(act.t[l], kCh[l], kCh[l], act.dcat[l], ldc, kCh[l], N, H(l), W(l), g32 + woff[k], g32 + boff[k],
-                       st);
+            conv_wgrad(act.t[l], kCh[l], kCh[l], act.dcat[l], ldc, kCh[l], N, H(l), W(l), g32 + woff[k], g32 + boff[k], wg_part, st);
             conv_dgrad(act.dcat[l], ldc, kCh[l], wd[k], kCh[l], N, H(l), W(l), act.dt[l], kCh[l], act.t[l], kCh[l], st);
             --k;
             // e_la: input pl[l-1] (or x0), grad dt[l]
             const uint16_t* in = l > 0 ? act.pl[l - 1] : act.x0;
             int cin = l > 0 ? kCh[l - 1] : kInCh;
-            conv_wgrad(in, cin, cin, act.dt[l], kCh[l], kCh[l], N, H(l), W(l), g32 + woff[k], g32 + boff[k], st);
+            conv_wgrad(in, cin, cin, act.dt[l], kCh[l], kCh[l], N, H(l), W(l), g32 + woff[k], g32 + boff[k], wg_part, st);
             if (l > 0)
                 conv_dgrad(act.dt[l], kCh[l], kCh[l], wd[k], cin, N, H(l), W(l), act.dpl[l - 1], cin, nullptr, 0, st);
             --k;
@@ -1775,17 +1950,16 @@ int kf_conv3x3_backward(const uint16_t* x, uint32_t cin, const uint16_t* w, uint
         KF_CHECK(hipMemcpyAsync(d_dy, dy, P * cout * 2, hipMemcpyHostToDevice, st));
         KF_CHECK(hipMemcpyAsync(d_w32, w32.data(), NW * 4, hipMemcpyHostToDevice, st));
         k_weights_bf16<<<blocks(NW, TB), TB, 0, st>>>(d_w32, (int)cin, (int)cout, d_wb, d_wd);
-        k_zero_f32<<<blocks(NW, TB), TB, 0, st>>>(d_dw, NW);
-        k_zero_f32<<<blocks(cout, TB), TB, 0, st>>>(d_db, cout);
+        float* d_part = dalloc<float>(WgradPlan((int)n, (int)h, (int)wd, (int)cin, (int)cout).floats());
         conv_dgrad(d_dy, cout, cout, d_wd, cin, n, h, wd, d_dx, cin, mask_by_x ? d_x : nullptr, cin, st);
-        conv_wgrad(d_x, cin, cin, d_dy, cout, cout, n, h, wd, d_dw, d_db, st);
+        conv_wgrad(d_x, cin, cin, d_dy, cout, cout, n, h, wd, d_dw, d_db, d_part, st);
         KF_CHECK(hipGetLastError());
         if (dx) KF_CHECK(hipMemcpyAsync(dx, d_dx, P * cin * 2, hipMemcpyDeviceToHost, st));
         if (dw) KF_CHECK(hipMemcpyAsync(dw, d_dw, NW * 4, hipMemcpyDeviceToHost, st));
         if (db) KF_CHECK(hipMemcpyAsync(db, d_db, cout * 4, hipMemcpyDeviceToHost, st));
         KF_CHECK(hipStreamSynchronize(st));
         for (void* q : {(void*)d_x, (void*)d_dy, (void*)d_dx, (void*)d_w32, (void*)d_wb, (void*)d_wd, (void*)d_dw,
-                        (void*)d_db})
+                        (void*)d_db, (void*)d_part})
             KF_CHECK(hipFree(q));
         return 0;
     } catch (const std::exception& e) {

@@ -56,6 +56,26 @@ def test_conv_backward(gpu, cin, cout, h, w):
     assert np.allclose(db, rdb, rtol=1e-5, atol=1e-4)
 
 
+# Strips of the weight-gradient kernel: 32 pixels wide and at least 4 rows
+# high, two pixels per register.  Widths around a strip and a pixel pair,
+# heights around one strip, and (last) a layer whose waves take several strips.
+@pytest.mark.parametrize("cin,cout,n,h,w", [(32, 32, 1, 1, 1), (32, 64, 2, 3, 31), (64, 32, 1, 4, 32), (96, 32, 3, 5, 33),
+                                            (32, 32, 1, 9, 65), (32, 32, 2, 2, 2), (160, 160, 2, 80, 65)])
+def test_weight_gradient_strips(gpu, cin, cout, n, h, w):
+    rng = np.random.default_rng(7 * cin + cout + h + w)
+    x = bf(rng.normal(0, 1, (n, h, w, cin)))
+    wt = bf(rng.normal(0, 0.1, (9, cout, cin)))
+    dy = bf(rng.normal(0, 1, (n, h, w, cout)))
+    _, dw, db = conv_backward(x, wt, dy, mask_by_x=False)
+    _, rdw, rdb = U.conv_bwd(x, wt, dy)
+    # FP32 sums of n h w exact products: each rounding is at most 2^-24 of a
+    # partial sum, and sqrt(n h w) of them in a random walk stay below 1e-5
+    assert np.linalg.norm(dw - rdw) <= 1e-5 * np.linalg.norm(rdw)
+    assert np.linalg.norm(db - rdb) <= 1e-5 * np.linalg.norm(rdb)
+    _, dw2, db2 = conv_backward(x, wt, dy, mask_by_x=False)
+    assert np.array_equal(dw, dw2) and np.array_equal(db, db2)
+
+
 def he_params(seed):
     rng = np.random.default_rng(seed)
     sl, n = U.param_slices()
