@@ -401,7 +401,7 @@ int kf_render_envs(kf_renderer* r, kf_scene* s, uint32_t num_envs, const kf_came
  * rendered with samples_per_batch = 0.  Images do not depend on the
  * schedule.  Renders into r's targets (frame_count 0). */
 typedef struct kf_tune_result {
-    uint32_t samples_per_batch, refill, grab;
+    uint32_t samples_per_batch, refill, grab; /* grab 0: reservations sized by what their queue has left */
     float frame_ms;    /* kernel time of a frame with the picked schedule */
     float default_ms;  /* ... with the built-in default */
     uint32_t trials;   /* frames timed */
@@ -414,9 +414,10 @@ typedef struct kf_tune_result {
 int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_envs, const kf_camera_ubo* cams,
                          const kf_push_constants* pc, kf_tune_result* out);
 /* Set the schedule directly (e.g. one kf_renderer_autotune picked earlier);
- * 0 keeps the built-in default of that parameter (for tail_bounce: the
- * wavefront runs every bounce; for grab0 and grab_shadow, the camera rays'
- * and the shadow rays' reservations: grab).  refill is clamped to [1, 64],
+ * 0 keeps the built-in default of that parameter (for grab: reservations
+ * sized by what their queue has left; for tail_bounce: the wavefront runs
+ * every bounce; for grab0 and grab_shadow, the camera rays' and the shadow
+ * rays' reservations: grab).  refill is clamped to [1, 64],
  * the reservations to [16, 4096]. */
 int kf_renderer_set_schedule(kf_renderer* r, uint32_t samples_per_batch, uint32_t refill, uint32_t grab,
                              uint32_t tail_bounce, uint32_t grab0, uint32_t grab_shadow);

@@ -33,21 +33,25 @@ constexpr int TB = 256;
 static_assert(TB == (int)kRingThreads, "traversal kernels index their LDS stack ring by a 256-thread block");
 
 // Device counters of one batch: per bounce b: [0] active paths, [1] shadow
-// rays, [2] next queue, [3..10] work chunks of k_extend, [11..18] work chunks
-// of k_shadow, [19] rays k_extend traces at bounce b.  Global, at the end:
-// primary / extension / shadow rays, BVH4 node records / triangle tests
+// rays, [2] next queue, [3] rays k_extend traces at bounce b.  Global, after
+// them: primary / extension / shadow rays, BVH4 node records / triangle tests
 // (closest-hit traversal), stack overflow, instance records, speculative
 // rays, TLAS node records (part of the node records), closest-hit rays
-// traced by k_tail (part of the extension rays).
+// traced by k_tail (part of the extension rays).  Then, per bounce, the work
+// chunks of k_extend and of k_shadow (8 each, kChunkStride apart).
 constexpr int kMaxBounces = 64;
-constexpr int kCntPerBounce = 20;
+constexpr int kCntPerBounce = 4;
 // throughput and depth of a path before its first bounce
 __device__ constexpr float4 kPathStart = {1.0f, 1.0f, 1.0f, 0.0f};  // .w: depth 0 as uint bits
-constexpr int kCntExtendChunks = 3;
-constexpr int kCntShadowChunks = 11;
-constexpr int kCntExtQueue = 19;
+constexpr int kCntExtQueue = 3;
 constexpr int kCntGlobal = kMaxBounces * kCntPerBounce;
-constexpr int kCntSize = kCntGlobal + 10;
+constexpr int kCntChunks = (kCntGlobal + 10 + (int)kChunkStride - 1) / (int)kChunkStride * (int)kChunkStride;
+constexpr int kChunksPerBounce = 2 * 8 * (int)kChunkStride;
+constexpr int kCntSize = kCntChunks + kMaxBounces * kChunksPerBounce;
+KF_DEV unsigned long long* extend_chunks(unsigned long long* cnt, int b) { return cnt + kCntChunks + b * kChunksPerBounce; }
+KF_DEV unsigned long long* shadow_chunks(unsigned long long* cnt, int b) {
+    return extend_chunks(cnt, b) + 8 * kChunkStride;
+}
 
 // Per-frame values the kernels read from device memory, so that a captured
 // frame graph replays with new seeds and running-mean weights.
@@ -112,9 +116,13 @@ KF_DEV uint32_t block_append(unsigned long long* counter, bool pred) {
     return r;
 }
 
-__global__ void k_zero(unsigned long long* c, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) c[i] = 0;
+// Clears the counters of bounces 0 .. nb (their work chunks: of 0 .. nb - 1),
+// and the global ones on the frame's first batch.
+__global__ void k_zero(unsigned long long* c, int nb, int globals) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int small = globals ? kCntGlobal + 10 : (nb + 1) * kCntPerBounce;
+    if (i < small) c[i] = 0;
+    else if (i - small < nb * 16) c[kCntChunks + (i - small) * (int)kChunkStride] = 0;
 }
 
 // ------------------------------------------------------------ camera-ray TLAS
@@ -472,7 +480,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_num_vgpr(52))) void k_ext
         hit[p] = make_float4(b.t, b.b1, b.b2, __uint_as_float(b.inst));
         hit_prim[p] = b.prim | (b.back << 31);
     };
-    trace_persistent<false, COUNT>(S, n, cnt + bounce * kCntPerBounce + kCntExtendChunks, refill, grab, S.any_alpha != 0u, load,
+    trace_persistent<false, COUNT>(S, n, extend_chunks(cnt, bounce), refill, grab, S.any_alpha != 0u, load,
                                    store, ovf, tot);
     if (COUNT) {
         wave_add(&cnt[kCntGlobal + 3], tot.nodes);
@@ -918,7 +926,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_num_vgpr(48))) void k_sha
     auto store = [&](uint32_t slot, THit, bool found) __attribute__((always_inline)) {
         if (!found) vis[slot] = 1;
     };
-    trace_persistent<true, false>(S, n, cnt + bounce * kCntPerBounce + kCntShadowChunks, refill, grab, false, load,
+    trace_persistent<true, false>(S, n, shadow_chunks(cnt, bounce), refill, grab, false, load,
                                   store, ovf, tot);
     if (ovf) atomicAdd(&cnt[kCntGlobal + 5], 1ull);
 }
@@ -1193,7 +1201,7 @@ __global__ __launch_bounds__(TB) void k_tail2(SceneView S, Frame F, const DevLig
             }
             if (second && pending) alive = start_shadow();
             while (__ballot(alive) != 0ull) {
-                const bool more = T.template step<true>(TS, stk, ovf, alive);
+                const bool more = T.step(TS, stk, ovf, alive);
                 if (alive && !more) {
                     alive = false;
                     if (!second) {
@@ -1567,7 +1575,8 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     const uint32_t grid_conn = (uint32_t)n_cu * 8;
     const uint32_t refill = std::min<uint32_t>(64u, std::max<uint32_t>(1u, r->tune_refill ? r->tune_refill
                                                                                          : traversal_refill()));
-    const uint32_t grab = std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grab ? r->tune_grab : kGrab));
+    // reservations per wave: 0 sizes each by what its queue has left
+    const uint32_t grab = r->tune_grab ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grab)) : 0u;
     // camera rays (bounce 0): one long, coherent queue that may want another
     // reservation than the scattered later bounces
     const uint32_t grab0 = r->tune_grab0 ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grab0)) : grab;
@@ -1591,8 +1600,8 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
         F.s0 = s0;
         F.nsamp = std::min(spb, pc->spp - s0);
         const uint32_t B = WH * F.nsamp;
-        const int nz = s0 == 0 ? kCntSize : kCntGlobal;
-        k_zero<<<(nz + TB - 1) / TB, TB, 0, st>>>(r->counters, nz);
+        const int nz = (s0 == 0 ? kCntGlobal + 10 : (int)(nb + 1) * kCntPerBounce) + (int)nb * 16;
+        k_zero<<<(nz + TB - 1) / TB, TB, 0, st>>>(r->counters, (int)nb, s0 == 0 ? 1 : 0);
         if (timed) KF_CHECK(hipEventRecord(r->ev[0], st));
         if (tiles && s0 == 0)
             k_tile_roots<<<(uint32_t)std::min<size_t>((n_tiles + TB / 64 - 1) / (TB / 64), 65535u), TB, 0, st>>>(
@@ -1655,7 +1664,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
                 // the last wavefront bounce's shadow rays run with nothing
                 // beside them and the tail waiting: small reservations, so
                 // that few waves are left holding the longest rays
-                const uint32_t gsh = b + 1 < b_tail ? grabs : std::min<uint32_t>(grabs, kLastShadowGrab);
+                const uint32_t gsh = b + 1 < b_tail || !grabs ? grabs : std::min<uint32_t>(grabs, kLastShadowGrab);
                 k_shadow<<<grid_sh, TB, 0, r->st2>>>(S, (int)b, B * K, r->sh_o, r->sh_d, r->sh_root, r->vis,
                                                      r->counters, refill, gsh);
                 if (timed) KF_CHECK(hipEventRecord(r->ev[2 + 4 * b + 3], r->st2));
@@ -1877,10 +1886,10 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
         const uint32_t spb_def = default_batch(p.spp, WH);
         if (std::find(spbs.begin(), spbs.end(), spb_def) == spbs.end()) spbs.push_back(spb_def);
         b_refill = std::min<uint32_t>(64u, std::max<uint32_t>(1u, traversal_refill()));
-        b_grab = kGrab;
+        b_grab = 0u;
         // the best refill threshold depends on the reservation size: the
         // reservation is swept before and after it
-        const std::vector<uint32_t> grabs = {64u, 128u, 256u, 512u, 1024u};
+        const std::vector<uint32_t> grabs = {0u, 64u, 128u, 256u, 512u, 1024u};
         std::vector<uint32_t> refills = {8u, 16u, 32u, 48u};
         if (std::find(refills.begin(), refills.end(), b_refill) == refills.end()) refills.push_back(b_refill);
         // the bounce from which k_tail finishes the paths: never (0), or from
@@ -1897,7 +1906,7 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
         // rays favour larger reservations than the scattered later bounces
         // (at 16 spp of the 1080p scene 512 against 256 for the later
         // bounces; one reservation for all of them is 6 % slower)
-        const std::vector<uint32_t> grab0s = {256u, 512u, 1024u};
+        const std::vector<uint32_t> grab0s = {0u, 256u, 512u, 1024u};
         uint32_t best_grab0 = b_grab;
         sweep(grab0s, best_grab0, 4);
         b_grab0 = best_grab0;

@@ -17,8 +17,10 @@ constexpr int TB = 256;
 static_assert(TB == (int)kRingThreads, "traversal kernels index their LDS stack ring by a 256-thread block");
 
 // Counters of a trace call: [0] node records, [1] triangle tests, [2] stack
-// overflow / malformed tree, [4..11] work-chunk counters of the persistent grid.
-constexpr int kTraceCnt = 12;
+// overflow / malformed tree, from [kTraceChunks] the work-chunk counters of
+// the persistent grid, each on a line of its own.
+constexpr int kTraceChunks = kChunkStride;
+constexpr int kTraceCnt = kTraceChunks + 8 * kChunkStride;
 
 // Fixed batches trace environment 0 (the whole TLAS of a scene without
 // environments).
@@ -49,7 +51,7 @@ __global__ __launch_bounds__(TB) void k_closest(SceneView S, const kf_ray* __res
         o.back = b.back;
         hits[q] = o;
     };
-    trace_persistent<false, COUNT>(S, n, cnt + 4, refill, kGrab, false, load, store, ovf, tot);
+    trace_persistent<false, COUNT>(S, n, cnt + kTraceChunks, refill, 0u, false, load, store, ovf, tot);
     if (COUNT) {
         atomicAdd(&cnt[0], (unsigned long long)tot.nodes);
         atomicAdd(&cnt[1], (unsigned long long)tot.tris);
@@ -64,7 +66,7 @@ __global__ __launch_bounds__(TB) void k_any(SceneView S, const kf_ray* __restric
     TCount tot{0, 0, 0, 0};
     auto load = [&](uint32_t q, TRay& t) __attribute__((always_inline)) { ray_of(S, rays[q], q, t); };
     auto store = [&](uint32_t q, THit, bool found) __attribute__((always_inline)) { occ[q] = found ? 1 : 0; };
-    trace_persistent<true, false>(S, n, cnt + 4, refill, kGrab, false, load, store, ovf, tot);
+    trace_persistent<true, false>(S, n, cnt + kTraceChunks, refill, 0u, false, load, store, ovf, tot);
     if (ovf) atomicAdd(&cnt[2], 1ull);
 }
 
@@ -160,7 +162,7 @@ extern "C" int kf_trace_closest(kf_scene* s, const kf_ray* rays, uint32_t n, kf_
         KF_CHECK(hipMemcpyAsync(d_r, rays, n * sizeof(kf_ray), hipMemcpyHostToDevice, st));
         k_closest<false><<<trace_grid(k_closest<false>), TB, 0, st>>>(s->view(), d_r, n, d_h, c, traversal_refill());
         KF_CHECK(hipGetLastError());
-        unsigned long long h[kTraceCnt];
+        unsigned long long h[4];
         KF_CHECK(hipMemcpyAsync(hits, d_h, n * sizeof(kf_hit), hipMemcpyDeviceToHost, st));
         KF_CHECK(hipMemcpyAsync(h, c, sizeof(h), hipMemcpyDeviceToHost, st));
         KF_CHECK(hipStreamSynchronize(st));
@@ -188,7 +190,7 @@ extern "C" int kf_trace_any(kf_scene* s, const kf_ray* rays, uint32_t n, uint8_t
         KF_CHECK(hipMemcpyAsync(d_r, rays, n * sizeof(kf_ray), hipMemcpyHostToDevice, st));
         k_any<<<trace_grid(k_any), TB, 0, st>>>(s->view(), d_r, n, d_o, c, traversal_refill());
         KF_CHECK(hipGetLastError());
-        unsigned long long h[kTraceCnt];
+        unsigned long long h[4];
         KF_CHECK(hipMemcpyAsync(occluded, d_o, n, hipMemcpyDeviceToHost, st));
         KF_CHECK(hipMemcpyAsync(h, c, sizeof(h), hipMemcpyDeviceToHost, st));
         KF_CHECK(hipStreamSynchronize(st));
@@ -209,10 +211,11 @@ extern "C" int kf_trace_any(kf_scene* s, const kf_ray* rays, uint32_t n, uint8_t
 // the name `scratch` is only a host-side stand-in: the device address comes
 // from hipGetSymbolAddress, once per device, and only that address is used.
 constexpr uint32_t kNoAllocMaxRays = KF_TRACE_NOALLOC_MAX_RAYS;
-constexpr size_t kNoAllocCntBytes = 256;
+constexpr size_t kNoAllocCntBytes = 1280;
 constexpr size_t kNoAllocRayBytes = (size_t)kNoAllocMaxRays * sizeof(kf_ray);
 constexpr size_t kNoAllocBytes = kNoAllocCntBytes + kNoAllocRayBytes + (size_t)kNoAllocMaxRays * sizeof(kf_hit);
-static_assert(kTraceCnt * sizeof(unsigned long long) <= kNoAllocCntBytes, "trace counters fit their slot");
+static_assert(kTraceCnt * sizeof(unsigned long long) <= kNoAllocCntBytes && kNoAllocCntBytes % 256 == 0,
+              "trace counters fit their slot");
 static_assert(kNoAllocRayBytes % 256 == 0, "hit staging stays 256-byte aligned");
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -263,7 +266,7 @@ extern "C" int kf_trace_closest_noalloc(kf_scene* s, const kf_ray* rays, uint32_
         KF_CHECK(hipMemcpyAsync(d_r, rays, n * sizeof(kf_ray), hipMemcpyHostToDevice, st));
         k_closest<false><<<trace_grid(k_closest<false>), TB, 0, st>>>(s->view(), d_r, n, d_h, c, traversal_refill());
         KF_CHECK(hipGetLastError());
-        unsigned long long h[kTraceCnt];
+        unsigned long long h[4];
         KF_CHECK(hipMemcpyAsync(hits, d_h, n * sizeof(kf_hit), hipMemcpyDeviceToHost, st));
         KF_CHECK(hipMemcpyAsync(h, c, sizeof(h), hipMemcpyDeviceToHost, st));
         KF_CHECK(hipStreamSynchronize(st));

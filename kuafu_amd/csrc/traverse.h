@@ -364,11 +364,7 @@ struct Trav {
     // action; the stack is updated once at the end.
     // live: the lane holds a query.  Lanes without one read the zero record
     // and have no side effects beyond their own (discarded) state.
-    // SKIP: skip the instance and triangle evaluations when no lane of the
-    // wave needs them (for waves that often run with few queries: shadow
-    // rays, one-thread traversals; the full waves of the closest-hit launch
-    // are 1 % faster without the branches).
-    template <bool SKIP, class Stack>
+    template <class Stack>
     KF_DEV bool step(const TravScene& S, Stack& stk, uint32_t& overflow, bool live) {
         enum { kNext, kPush, kPop, kDone };
         const uint32_t kind = cur >> 30, idx = cur & kIdxMask;
@@ -412,18 +408,20 @@ struct Trav {
                      "v"(below));
 
         // Every lane evaluates the record as a node, an instance and a
-        // triangle and keeps the result of its kind: in a full wave64 nearly
-        // every step has lanes of all three kinds, so per-lane branches would
-        // run all three anyway and would copy the traversal state at each
-        // join.  With SKIP the instance and triangle evaluations are skipped
-        // when no lane of the wave needs them (wave-uniform branches), which
-        // happens once few lanes still hold queries.  An instance record is a
-        // node as well (its BLAS root's children).
+        // triangle and keeps the result of its kind: per-lane branches would
+        // copy the traversal state at each join, and a full wave64 has lanes
+        // of all three kinds in nearly every step.  Waves with few queries
+        // left do not: the instance and triangle evaluations are skipped when
+        // no lane of the wave needs them (wave-uniform branches).  With the
+        // branches 2 M rays against the 256-icosphere scene take 1.09 ms
+        // instead of 1.13, 4096 rays 0.15 instead of 0.16 (whole calls), and
+        // the long launches of full waves are no slower.  An instance record
+        // is a node as well (its BLAS root's children).
         const bool is_node = kind != kTriangle && on;
         const bool is_inst = irec;
         const bool is_tri = kind == kTriangle && on;
-        const bool any_inst = !SKIP || __builtin_amdgcn_ballot_w64(is_inst) != 0;
-        const bool any_tri = !SKIP || __builtin_amdgcn_ballot_w64(is_tri) != 0;
+        const bool any_inst = __builtin_amdgcn_ballot_w64(is_inst) != 0;
+        const bool any_tri = __builtin_amdgcn_ballot_w64(is_tri) != 0;
 
         // instance: its BLAS is entered with the object-space ray, which this
         // step's node test already uses for the BLAS root's children (an
@@ -619,7 +617,7 @@ KF_DEV bool traverse(const SceneView& S, uint32_t root, v3 o, v3 d, float tmin, 
     r.payload = 0u;
     T.start(true, r, root, use_alpha);
     if (root != kEmptyItem)
-        while (T.template step<true>(TS, stk, overflow, true)) {
+        while (T.step(TS, stk, overflow, true)) {
         }
     best = T.result();
     cnt.nodes += T.cnt.nodes;
@@ -632,17 +630,32 @@ KF_DEV bool traverse(const SceneView& S, uint32_t root, v3 o, v3 d, float tmin, 
 // ------------------------------------------------------- persistent driver
 // Queries [0, n) are split into 8 contiguous chunks, one per XCD (workgroups
 // are dispatched to the 8 XCDs round-robin, so block b runs on XCD b % 8 and
-// neighbouring queries share that XCD's L2).  A wave reserves `grab` queries
-// at a time from its chunk's counter and refills its idle lanes from that
-// reserve once at least `refill` lanes are idle (or all are), so no lane
-// waits for the slowest ray of a fixed group.  When its chunk is used up the
-// wave moves on to the next one; a plain load of the counter tells a used-up
-// chunk without an atomic, which keeps the end of a launch (every wave
-// passing over every chunk) off the contended counters.
-//   ctr[8]: per-chunk counters, zero before the launch.
+// neighbouring queries share that XCD's L2).  A wave reserves queries from
+// its chunk's counter and refills its idle lanes from that reserve once at
+// least `refill` lanes are idle (or all are), so no lane waits for the
+// slowest ray of a fixed group.  When its chunk is used up the wave looks at
+// all eight counters at once and moves to the next chunk with queries left.
+//
+// Reservation size: `grab` queries, or with grab = 0 half an equal share of
+// what its chunk has left (kGuidedMin .. kGuidedMax), so that a long queue
+// takes few atomics and a launch still ends evenly; at most one query per
+// lane in launches with fewer queries than lanes.  A fixed size is right for
+// one queue length only, and the counters sit on lines of their own
+// (kChunkStride): with 128 queries per reservation and the eight counters on
+// one line, the atomics of all XCDs queued up behind each other and bounded
+// the long queues (whole frames: 128 environments of 512x512 at 8 spp 397 ->
+// 175 ms, 720p projector at 32 spp 57.4 -> 24.9 ms; 2 M rays 1.45 -> 1.05 ms).
+// Measured around it: a quarter or an eighth of the share 1-4 % slower on 2 M
+// rays and the projector, all of the share 18 % slower on 2 M rays; at least
+// 128 or 256 queries 2 and 4 % slower on 2 M rays and no faster by more than
+// 1 % elsewhere, at least 32 2 % slower on 128 environments; at most 4096, 3 %
+// slower there; the queries of short launches spread at 4, 16 or 32 per wave
+// instead of one per lane, 11, 5 and 4 % slower on a 256x256 frame.
+//   ctr[8 * kChunkStride]: per-chunk counters, zero before the launch.
 //   load(q, TRay&) fills the ray of query q and its payload;
 //   store(payload, best, found) writes a finished query.
-constexpr uint32_t kGrab = 128;  // default reservation
+constexpr uint32_t kGuidedMin = 64, kGuidedMax = 1024;
+constexpr uint32_t kChunkStride = 16;  // 8-byte counters per 128-byte line
 
 KF_DEV uint64_t chunk_begin(uint32_t n, uint32_t c) { return (uint64_t)n * c / 8u; }
 
@@ -660,13 +673,30 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
     stk.spill = spill;
     bool live = false;
     uint32_t payload = 0;
+    const uint32_t waves = gridDim.x * (kRingThreads / 64u);
+    const uint32_t most = n < 64u * waves ? 64u : ~0u;  // queries of one reservation
     uint32_t chunk = blockIdx.x & 7u;  // wave-uniform from here on
-    uint32_t moved = 0;                // chunks found used up
+    bool more = n > 0u;                // some chunk may have queries left
+    uint32_t seen = ~0u;               // queries of this chunk known to be taken (~0: not looked at yet)
     uint32_t res_q = 0, res_n = 0;     // reserved queries [res_q, res_q + res_n)
+    auto finish = [&](bool alive) __attribute__((always_inline)) {
+        if (live && !alive) {
+            live = false;
+            store(payload, T.result(), T.found);
+            if (COUNT) {
+                total.nodes += T.cnt.nodes;
+                total.tlas += T.cnt.tlas;
+                total.tris += T.cnt.tris;
+                total.insts += T.cnt.insts;
+            }
+        }
+    };
     while (true) {
+        // lane numbers by mbcnt: no per-lane mask to keep
+        const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
         const unsigned long long idle = __ballot(!live);
         const uint32_t nidle = (uint32_t)__popcll(idle);
-        if ((res_n > 0u || moved < 8u) && (nidle >= refill || nidle == 64u)) {
+        if ((res_n > 0u || more) && (nidle >= refill || nidle == 64u)) {
             bool fresh = false;
             TRay r;  // the ray this lane fetches, if any
             r.o = r.d = mk(0.0f, 0.0f, 0.0f);
@@ -674,28 +704,42 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
             r.tmax = 0.0f;
             r.root = kEmptyItem;
             r.alpha_seed = r.payload = 0u;
-            // idle lanes below this one (mbcnt: no per-lane mask to keep)
             const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
             const bool wants = !live;
             uint32_t got = 0;
-            while (got < nidle && (res_n > 0u || moved < 8u)) {
+            while (got < nidle && (res_n > 0u || more)) {
                 if (res_n == 0u) {
-                    const uint64_t c0 = chunk_begin(n, chunk), len = chunk_begin(n, chunk + 1u) - c0;
-                    unsigned long long base = 0;
-                    if (__builtin_amdgcn_mbcnt_lo(~0u, 0u) == 0u) {  // lane 0
-                        base = __hip_atomic_load(&ctr[chunk], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        if (base < len) base = atomicAdd(&ctr[chunk], (unsigned long long)grab);
+                    if (seen == ~0u) {  // lane c < 8 looks at chunk c
+                        const uint32_t c = lane & 7u;
+                        const uint32_t len = (uint32_t)(chunk_begin(n, c + 1u) - chunk_begin(n, c));
+                        const unsigned long long taken =
+                            __hip_atomic_load(&ctr[c * kChunkStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        const uint32_t open = (uint32_t)__ballot(taken < len) & 0xffu;
+                        if (open == 0u) {
+                            more = false;
+                            break;
+                        }
+                        // the first open chunk from this one on
+                        const uint32_t turned = ((open | (open << 8)) >> chunk) & 0xffu;
+                        chunk = (chunk + (uint32_t)__ffs((int)turned) - 1u) & 7u;
+                        seen = (uint32_t)__builtin_amdgcn_readlane((int)min(taken, (unsigned long long)len), (int)chunk);
                     }
-                    base = __shfl(base, 0);
+                    const uint64_t c0 = chunk_begin(n, chunk);
+                    const uint32_t len = (uint32_t)(chunk_begin(n, chunk + 1u) - c0);
+                    const uint32_t left = len - min(seen, len);
+                    const uint32_t take =
+                        min(most, grab ? grab : min(kGuidedMax, max(kGuidedMin, left / max(waves / 4u, 1u))));
+                    unsigned long long base = 0;
+                    if (lane == 0u) base = atomicAdd(&ctr[chunk * kChunkStride], (unsigned long long)take);
+                    base = (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base) |
+                           ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(base >> 32)) << 32);
                     if (base < len) {
                         res_q = (uint32_t)(c0 + base);
-                        res_n = (uint32_t)min((unsigned long long)grab, len - base);
+                        res_n = min(take, len - (uint32_t)base);
+                        seen = (uint32_t)base + res_n;
                     }
-                    if (base + grab >= len) {
-                        chunk = (chunk + 1u) & 7u;
-                        ++moved;
-                    }
+                    if (base + take >= len) seen = ~0u;  // used up: look at the others
                     continue;
                 }
                 const uint32_t take = min(nidle - got, res_n);
@@ -718,22 +762,12 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
                 live = live || (fresh && !empty);
             }
         }
-        if (__ballot(live) == 0ull && moved >= 8u && res_n == 0u) break;
+        if (!more && res_n == 0u && __ballot(live) == 0ull) break;
         // The step runs even when no lane holds a query (idle lanes read the
-        // zero record; this happens only while a wave runs out of work):
-        // a path that skipped it would make every step pay for merging the
-        // two paths' registers, and the refill state lives only in its branch.
-        const bool alive = T.template step<ANY>(TS, stk, overflow, live);
-        if (live && !alive) {
-            live = false;
-            store(payload, T.result(), T.found);
-            if (COUNT) {
-                total.nodes += T.cnt.nodes;
-                total.tlas += T.cnt.tlas;
-                total.tris += T.cnt.tris;
-                total.insts += T.cnt.insts;
-            }
-        }
+        // zero record): a path that skipped it would make every step pay for
+        // merging the two paths' registers, and the refill state lives only
+        // in its branch.
+        finish(T.step(TS, stk, overflow, live));
     }
 }
 

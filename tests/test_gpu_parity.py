@@ -61,6 +61,30 @@ def check_blas(gs, g):
     return depth
 
 
+# Batches around a chunk, a wave, one query per lane of the resident grid
+# (4 waves per SIMD on 256 CUs, 5 for shadow rays) and several refills of it:
+# a ray's hit does not depend on the batch it is traced in.
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 63, 64, 65, 513, 262143, 262145, 327680, 700001])
+def test_batch_sizes_give_the_same_hits(gpu, n):
+    gs = GpuScene(scenes.config1().data)
+    rng = np.random.default_rng(5)
+    base = np.zeros(1009, abi.RAY_DTYPE)
+    base["org"] = rng.uniform(-3, 3, (1009, 3)) + (0.0, 3.0, 0.0)
+    d = rng.normal(size=(1009, 3))
+    base["dir"] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    base["tmin"], base["tmax"] = 0.001, 1e4
+    base["tmax"][::97] = -1.0  # nothing to trace: a miss
+    hits = np.concatenate([gs.trace_closest(base[i:i + 64]) for i in range(0, 1009, 64)])
+    occ = np.concatenate([gs.trace_any(base[i:i + 64]) for i in range(0, 1009, 64)])
+    idx = np.arange(n) % 1009
+    got = gs.trace_closest(base[idx])
+    assert got.tobytes() == hits[idx].tobytes()
+    assert np.array_equal(gs.trace_any(base[idx]), occ[idx])
+    if n == 65:
+        ref = oracle.Scene(scenes.config1().data).trace_closest(base)
+        assert np.array_equal(hits["inst"], ref["inst"]) and np.array_equal(hits["prim"], ref["prim"])
+
+
 def test_blas_invariants(gpu):
     w = scenes.config1()
     gs = GpuScene(w.data)
