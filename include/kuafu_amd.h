@@ -401,29 +401,29 @@ int kf_render_envs(kf_renderer* r, kf_scene* s, uint32_t num_envs, const kf_came
  * rendered with samples_per_batch = 0.  Images do not depend on the
  * schedule.  Renders into r's targets (frame_count 0). */
 typedef struct kf_tune_result {
-    uint32_t samples_per_batch, refill, grab; /* grab 0: reservations sized by what their queue has left */
+    uint32_t samples_per_batch, refill, grab; /* grab: largest reservation per wave (smaller once its queue runs short) */
     float frame_ms;    /* kernel time of a frame with the picked schedule */
     float default_ms;  /* ... with the built-in default */
     uint32_t trials;   /* frames timed */
-    uint32_t tail_bounce; /* bounce from which one thread carries each path to its end (0: never) */
+    uint32_t tail_bounce; /* bounce from which one thread carries each path to its end (path_depth + 1: never) */
     uint32_t grab0;       /* queries reserved per wave for the camera rays (0: grab) */
     uint32_t grab_shadow; /* ... for the shadow rays (0: grab) */
-    uint32_t tail_pairs;  /* 1: two lanes per path carry the tail bounces while few paths remain (at most a
-                             quarter of the launch's threads; no soft light), 0: one lane per path */
+    uint32_t tail_pairs;  /* 1: two lanes per path carry the tail bounces while few paths remain (at most an
+                             eighth of the launch's threads; no soft light), 0: one lane per path */
 } kf_tune_result;
 int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_envs, const kf_camera_ubo* cams,
                          const kf_push_constants* pc, kf_tune_result* out);
 /* Set the schedule directly (e.g. one kf_renderer_autotune picked earlier);
- * 0 keeps the built-in default of that parameter (for grab: reservations
- * sized by what their queue has left; for tail_bounce: the wavefront runs
- * every bounce; for grab0 and grab_shadow, the camera rays' and the shadow
- * rays' reservations: grab).  refill is clamped to [1, 64],
+ * 0 keeps the built-in default of that parameter (for tail_bounce: chosen by
+ * the number of paths and lights; a value beyond the last bounce runs every
+ * bounce in the wavefront; for grab0 and grab_shadow, the camera rays' and
+ * the shadow rays' largest reservations: grab).  refill is clamped to [1, 64],
  * the reservations to [16, 4096]. */
 int kf_renderer_set_schedule(kf_renderer* r, uint32_t samples_per_batch, uint32_t refill, uint32_t grab,
                              uint32_t tail_bounce, uint32_t grab0, uint32_t grab_shadow);
 /* Choose the kernel that carries the bounces from tail_bounce on (cleared to
  * 1 by kf_renderer_set_schedule): 1 lets two lanes per path take them while
- * at most a quarter of the launch's threads' worth of paths is left and no
+ * at most an eighth of the launch's threads' worth of paths is left and no
  * light has a random perturbation (kf_tune_result.tail_pairs), 0 keeps one
  * lane per path.  Images do not depend on it. */
 int kf_renderer_set_tail_pairs(kf_renderer* r, uint32_t tail_pairs);

@@ -264,8 +264,7 @@ struct Renderer {
     uint2* d_jump = nullptr;                   // LCG jump-ahead per sample
     uint32_t jump_cap = 0;
     float4* d_acc = nullptr;                   // per-pixel running sample sum
-    float4* d_out = nullptr;                   // per-path final radiance of a batch
-    size_t out_cap = 0;
+    float4* d_out = nullptr;                   // per-path final radiance of a batch (cap paths)
     std::vector<hipEvent_t> ev;
     hipStream_t st2 = nullptr;                 // any-hit traversal, beside the main stream
     std::vector<hipEvent_t> sync_ev;           // per bounce: shading done, shadow rays done
@@ -283,7 +282,7 @@ struct Renderer {
     uint32_t tune_pairs = 1;  // 1: k_tail2 may carry the tail bounces of few paths, 0: k_tail only
     uint32_t n_env_last = 1;                   // environments of the last frame (the denoiser's batch)
     ~Renderer();
-    void ensure(size_t paths, uint32_t nslots, uint32_t spp);
+    bool ensure(size_t paths, uint32_t nslots, uint32_t spp);
 };
 
 }  // namespace kf

@@ -1116,7 +1116,7 @@ KF_DEV bool nee_slots(const SceneView& S, const DevLights* __restrict__ LT, cons
 // streams, light order and radiance are those of the wavefront and k_tail;
 // a path's chain of dependent traversals is about half as long, which pays
 // while few paths are left: the frame launches k_tail2 for at most max_n
-// paths (a quarter of its threads) and k_tail beyond (1080p, 16 spp: 33 k
+// paths (an eighth of its threads) and k_tail beyond (1080p, 16 spp: 33 k
 // paths at bounce 5; 1 spp: hundreds of thousands at bounce 3).
 __global__ __launch_bounds__(TB) void k_tail2(SceneView S, Frame F, const DevLights* __restrict__ LT, int b0,
                                               const uint32_t* __restrict__ queue, float4* __restrict__ ray_o,
@@ -1339,40 +1339,55 @@ Renderer::~Renderer() {
         if (p) (void)hipFree(p);
 }
 
-void Renderer::ensure(size_t paths, uint32_t nslots, uint32_t spp) {
+// Buffers for `paths` paths; false when they do not fit the free memory
+// (nothing is held then).
+bool Renderer::ensure(size_t paths, uint32_t nslots, uint32_t spp) {
     if (paths > cap || nslots > slots) {
-        void* ptrs[] = {ray_o, ray_d, thr, col, rw, em, hit, hit_prim, seed, queue_a, queue_b, queue_e,
-                        sh_o, sh_d, sh_root, nee_a, nee_b, vis};
-        for (void* p : ptrs)
-            if (p) KF_CHECK(hipFree(p));
-        cap = std::max(cap, paths);
-        slots = std::max(slots, std::max<uint32_t>(nslots, 1));
-        ray_o = dmalloc<float4>(cap);
-        ray_d = dmalloc<float4>(cap);
-        thr = dmalloc<float4>(cap);
-        col = dmalloc<float4>(cap);
-        rw = dmalloc<float4>(cap);
-        em = dmalloc<float4>(cap);
-        hit = dmalloc<float4>(cap);
-        hit_prim = dmalloc<uint32_t>(cap);
-        seed = dmalloc<uint32_t>(cap);
-        queue_a = dmalloc<uint32_t>(cap);
-        queue_b = dmalloc<uint32_t>(cap);
-        queue_e = dmalloc<uint32_t>(cap);
-        sh_o = dmalloc<float4>(cap * slots);
-        sh_d = dmalloc<float4>(cap * slots);
-        sh_root = dmalloc<uint32_t>(cap * slots);
-        nee_a = dmalloc<float4>(cap * slots);
-        nee_b = dmalloc<float4>(cap * slots);
-        vis = dmalloc<uint8_t>(cap * slots);
+        const size_t want = std::max(cap, paths);
+        const uint32_t wslots = std::max(slots, std::max<uint32_t>(nslots, 1));
+        struct Buf {
+            void** p;
+            size_t bytes;
+        };
+        const size_t f4 = want * sizeof(float4), u4 = want * sizeof(uint32_t), s4 = wslots * f4;
+        const Buf bufs[] = {{(void**)&ray_o, f4},   {(void**)&ray_d, f4},   {(void**)&thr, f4},
+                            {(void**)&col, f4},     {(void**)&rw, f4},      {(void**)&em, f4},
+                            {(void**)&hit, f4},     {(void**)&hit_prim, u4}, {(void**)&seed, u4},
+                            {(void**)&queue_a, u4}, {(void**)&queue_b, u4}, {(void**)&queue_e, u4},
+                            {(void**)&sh_o, s4},    {(void**)&sh_d, s4},    {(void**)&sh_root, wslots * u4},
+                            {(void**)&nee_a, s4},   {(void**)&nee_b, s4},   {(void**)&vis, wslots * want},
+                        {(void**)&d_out, f4}};
+        auto drop = [&] {
+            for (const Buf& b : bufs) {
+                if (*b.p) KF_CHECK(hipFree(*b.p));
+                *b.p = nullptr;
+            }
+            cap = 0;
+            slots = 0;
+        };
+        drop();
+        for (const Buf& b : bufs) {
+            const hipError_t e = hipMalloc(b.p, b.bytes);
+            if (e == hipSuccess) continue;
+            *b.p = nullptr;
+            (void)hipGetLastError();
+            drop();
+            if (e == hipErrorOutOfMemory) return false;
+            throw Error(std::string("kf_render: hipMalloc: ") + hipGetErrorString(e));
+        }
+        cap = want;
+        slots = wslots;
     }
     size_t sneed = (size_t)spp * W * H * 3;
     if (spp && sneed > samples_cap) {
         if (samples) KF_CHECK(hipFree(samples));
+        samples = nullptr;
+        samples_cap = 0;
         samples = dmalloc<float>(sneed);
         samples_cap = sneed;
     }
     if (!counters) counters = dmalloc<unsigned long long>(kCntSize);
+    return true;
 }
 
 // ------------------------------------------------------------------ frame
@@ -1390,12 +1405,34 @@ uint32_t resident_grid(Kernel kernel, int n_cu) {
 
 constexpr uint32_t kLastShadowGrab = 32;  // queries per wave reservation, last wavefront bounce's shadow rays
 
-// Default batch: up to 32M paths (16 spp at 1920x1080).  Each bounce's
-// traversal launch then holds tens of rays per lane, so the tail of the
-// slowest rays is a small part of it; the state costs about 200 B per path
-// (6.6 GB at 32M paths).
+// Default batch: up to 64M paths (2 spp of 128 environments of 512x512).
+// Each batch ends every bounce's launch on its slowest rays, about 3 ms in
+// all on that frame (batches of 32M, 64M, 128M, 256M paths: 175, 162, 156,
+// 153 ms); the state costs 200-300 B per path, 13-19 GB at 64M paths, and a
+// default that does not fit the free memory is halved (render_frame).
 uint32_t default_batch(uint32_t spp, uint32_t WH) {
-    return std::max<uint32_t>(1, std::min<uint32_t>(spp, (32u << 20) / std::max<uint32_t>(WH, 1)));
+    return std::max<uint32_t>(1, std::min<uint32_t>(spp, (64u << 20) / std::max<uint32_t>(WH, 1)));
+}
+
+// Default bounce from which the tail kernels carry the paths (nb: never).
+// They run each path as one chain of rays, so they win where a bounce's
+// launches cannot fill the chip and last as long as their slowest ray, and
+// where Russian roulette has thinned the paths; measured over three scenes
+// at 16 k - 30 M paths per batch, never / from bounce 1 / 2 / 3 / 5:
+//   262 k paths, 256 icospheres   2.25 / 1.45 / 1.69 / 1.83 / 2.23 ms
+//   1 M paths, projector          2.31 / 2.43 / 2.03 / 2.02 / 2.18 ms
+//   4 M paths, 256 icospheres     4.57 / 5.08 / 3.98 / 3.77 / 4.25 ms
+//   17 M paths, 256 icospheres    8.60 / 14.7 / 10.4 / 8.56 / 8.04 ms
+// The shadow rays of all lights are part of a path's chain.  256 k paths on
+// the config-1 spheres, never / from bounce 1 / 2: 1.48 / 1.07 / 1.09 ms with
+// 2 lights, 1.63 / 1.38 / 1.33 with 3, 1.69 / 1.71 / 1.61 with 4, 1.99 / 2.47
+// / 2.23 with 8, 3.18 / 7.84 / 7.48 with 32.
+uint32_t default_tail(const kf_push_constants& pc, uint64_t paths, uint32_t lights, uint32_t nb) {
+    if (lights > 4) return nb;
+    if (paths <= (3u << 17) && lights <= 3) return 1;
+    if (paths <= (3u << 19)) return 2;
+    if (!pc.russian_roulette) return nb;
+    return paths <= (8u << 20) ? 3 : pc.rr_min_bounces + 1;
 }
 
 void build_light_list(const Scene& s, DevLights& L, bool& inline_nee) {
@@ -1464,7 +1501,11 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     if (spb == 0) spb = default_batch(pc->spp, WH);
     spb = std::min(spb, pc->spp);
     uint32_t K = inline_nee ? 1u : (uint32_t)std::max(L.n_slots, 1);
-    r->ensure((size_t)WH * spb, K, o.keep_samples ? pc->spp : 0);
+    const bool spb_default = !o.samples_per_batch && !r->tune_spb;
+    while (!r->ensure((size_t)WH * spb, K, o.keep_samples ? pc->spp : 0)) {
+        if (!spb_default || spb == 1) throw Error("kf_render: out of GPU memory for the path state");
+        spb = (spb + 1) / 2;
+    }
     r->samples_spp = o.keep_samples ? pc->spp : 0;
     // device light list (per frame, like the UBO upload)
     if (!r->d_lights) KF_CHECK(hipMalloc(&r->d_lights, sizeof(DevLights)));
@@ -1491,11 +1532,6 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     KF_CHECK(hipMemcpyAsync(d_jump, jump.data(), pc->spp * sizeof(uint2), hipMemcpyHostToDevice, st));
     if (!r->d_acc) KF_CHECK(hipMalloc((void**)&r->d_acc, (size_t)WH * sizeof(float4)));
     float4* d_acc = r->d_acc;
-    if ((size_t)WH * spb > r->out_cap) {
-        if (r->d_out) KF_CHECK(hipFree(r->d_out));
-        KF_CHECK(hipMalloc((void**)&r->d_out, (size_t)WH * spb * sizeof(float4)));
-        r->out_cap = (size_t)WH * spb;
-    }
     float4* d_out = r->d_out;
 
     if (n_env > r->cams_cap) {
@@ -1575,8 +1611,8 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     const uint32_t grid_conn = (uint32_t)n_cu * 8;
     const uint32_t refill = std::min<uint32_t>(64u, std::max<uint32_t>(1u, r->tune_refill ? r->tune_refill
                                                                                          : traversal_refill()));
-    // reservations per wave: 0 sizes each by what its queue has left
-    const uint32_t grab = r->tune_grab ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grab)) : 0u;
+    // largest reservation per wave
+    const uint32_t grab = std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grab ? r->tune_grab : kGrab));
     // camera rays (bounce 0): one long, coherent queue that may want another
     // reservation than the scattered later bounces
     const uint32_t grab0 = r->tune_grab0 ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grab0)) : grab;
@@ -1589,7 +1625,9 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     const uint32_t nb = pc->path_depth + 1;
     // bounces from b_tail on run in k_tail (not in counting frames, whose
     // node counts come from the wavefront kernels)
-    const uint32_t b_tail = (o.count_traversal || r->tune_tail == 0 || r->tune_tail >= nb) ? nb : r->tune_tail;
+    const uint32_t tail = r->tune_tail ? r->tune_tail
+                                       : std::max(1u, default_tail(*pc, (uint64_t)WH * spb, (uint32_t)L.n_slots, nb));
+    const uint32_t b_tail = o.count_traversal ? nb : std::min(tail, nb);
 
     // One batch of samples [s0, s0 + nsamp).  timed: record the per-kernel
     // events (not while capturing a graph).  The first batch clears every
@@ -1635,9 +1673,11 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
         for (uint32_t b = 0; b < nb; ++b) {
             if (b == b_tail) {
                 // the path count is on the device: k_tail2 (two lanes per
-                // path) runs for at most a quarter of the grid's threads,
-                // k_tail beyond, and the other launch returns at once
-                const uint32_t pair_max = (inline_nee || !r->tune_pairs) ? 0u : grid * TB / 4u;
+                // path) runs for at most an eighth of the grid's threads,
+                // k_tail beyond, and the other launch returns at once (up to
+                // a quarter, 4 M paths from bounce 3 are 4 % slower: the
+                // pairs then compete for the same SIMDs)
+                const uint32_t pair_max = (inline_nee || !r->tune_pairs) ? 0u : grid * TB / 8u;
                 if (!inline_nee)
                     k_tail2<<<grid, TB, 0, st>>>(S, F, d_lights, (int)b, qa, r->ray_o, r->ray_d, r->thr, r->col,
                                                  r->hit, r->hit_prim, r->rw, r->em, r->seed, r->nee_a, r->nee_b,
@@ -1664,7 +1704,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
                 // the last wavefront bounce's shadow rays run with nothing
                 // beside them and the tail waiting: small reservations, so
                 // that few waves are left holding the longest rays
-                const uint32_t gsh = b + 1 < b_tail || !grabs ? grabs : std::min<uint32_t>(grabs, kLastShadowGrab);
+                const uint32_t gsh = b + 1 < b_tail ? grabs : std::min<uint32_t>(grabs, kLastShadowGrab);
                 k_shadow<<<grid_sh, TB, 0, r->st2>>>(S, (int)b, B * K, r->sh_o, r->sh_d, r->sh_root, r->vis,
                                                      r->counters, refill, gsh);
                 if (timed) KF_CHECK(hipEventRecord(r->ev[2 + 4 * b + 3], r->st2));
@@ -1843,9 +1883,6 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
             }
             return best;
         };
-        r->tune_tail = 0;
-        r->tune_grab0 = 0;
-        r->tune_grabs = 0;
         run(0, 0, 0);  // warm-up: buffers, code objects, clocks
         run(0, 0, 0);
         const float t_def = run(0, 0, 0);
@@ -1886,18 +1923,18 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
         const uint32_t spb_def = default_batch(p.spp, WH);
         if (std::find(spbs.begin(), spbs.end(), spb_def) == spbs.end()) spbs.push_back(spb_def);
         b_refill = std::min<uint32_t>(64u, std::max<uint32_t>(1u, traversal_refill()));
-        b_grab = 0u;
+        b_grab = kGrab;
         // the best refill threshold depends on the reservation size: the
         // reservation is swept before and after it
-        const std::vector<uint32_t> grabs = {0u, 64u, 128u, 256u, 512u, 1024u};
+        const std::vector<uint32_t> grabs = {64u, 128u, 256u, 512u, 1024u};
         std::vector<uint32_t> refills = {8u, 16u, 32u, 48u};
         if (std::find(refills.begin(), refills.end(), b_refill) == refills.end()) refills.push_back(b_refill);
-        // the bounce from which k_tail finishes the paths: never (0), or from
-        // bounce 2 up to the first bounces after Russian roulette starts (few
+        // the bounce from which k_tail finishes the paths: never (beyond the
+        // last bounce), or from bounce 1 up to the first bounces after Russian roulette starts (few
         // paths per frame favour an early tail: at 1 spp of the 1080p scene
         // bounce 3 beats bounce 5 by 8 %)
-        std::vector<uint32_t> tails = {0u};
-        for (uint32_t tb = 2u; tb < std::min<uint32_t>(p.path_depth + 1u, p.rr_min_bounces + 4u); ++tb)
+        std::vector<uint32_t> tails = {p.path_depth + 1u};
+        for (uint32_t tb = 1u; tb < std::min<uint32_t>(p.path_depth + 1u, p.rr_min_bounces + 4u); ++tb)
             tails.push_back(tb);
         sweep(spbs, b_spb, 0);
         sweep(grabs, b_grab, 2);
@@ -1906,12 +1943,12 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
         // rays favour larger reservations than the scattered later bounces
         // (at 16 spp of the 1080p scene 512 against 256 for the later
         // bounces; one reservation for all of them is 6 % slower)
-        const std::vector<uint32_t> grab0s = {0u, 256u, 512u, 1024u};
+        const std::vector<uint32_t> grab0s = {256u, 512u, 1024u};
         uint32_t best_grab0 = b_grab;
         sweep(grab0s, best_grab0, 4);
         b_grab0 = best_grab0;
         sweep(grabs, b_grab, 2);
-        uint32_t best_tail = 0;
+        uint32_t best_tail = tails[0];
         sweep(tails, best_tail, 3);
         b_tail = best_tail;
         // the tail kernel: two lanes per path while few paths remain, or one

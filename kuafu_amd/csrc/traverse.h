@@ -636,25 +636,25 @@ KF_DEV bool traverse(const SceneView& S, uint32_t root, v3 o, v3 d, float tmin, 
 // slowest ray of a fixed group.  When its chunk is used up the wave looks at
 // all eight counters at once and moves to the next chunk with queries left.
 //
-// Reservation size: `grab` queries, or with grab = 0 half an equal share of
-// what its chunk has left (kGuidedMin .. kGuidedMax), so that a long queue
-// takes few atomics and a launch still ends evenly; at most one query per
-// lane in launches with fewer queries than lanes.  A fixed size is right for
-// one queue length only, and the counters sit on lines of their own
-// (kChunkStride): with 128 queries per reservation and the eight counters on
-// one line, the atomics of all XCDs queued up behind each other and bounded
-// the long queues (whole frames: 128 environments of 512x512 at 8 spp 397 ->
-// 175 ms, 720p projector at 32 spp 57.4 -> 24.9 ms; 2 M rays 1.45 -> 1.05 ms).
-// Measured around it: a quarter or an eighth of the share 1-4 % slower on 2 M
-// rays and the projector, all of the share 18 % slower on 2 M rays; at least
-// 128 or 256 queries 2 and 4 % slower on 2 M rays and no faster by more than
-// 1 % elsewhere, at least 32 2 % slower on 128 environments; at most 4096, 3 %
-// slower there; the queries of short launches spread at 4, 16 or 32 per wave
-// instead of one per lane, 11, 5 and 4 % slower on a 256x256 frame.
+// Reservation size: half an equal share of what its chunk has left, from
+// kGrabMin queries up to `grab`, so that a launch ends evenly; at most one
+// query per lane in launches with fewer queries than lanes.  The counters sit
+// on lines of their own (kChunkStride): with all eight on one line and 128
+// queries per reservation the atomics of all XCDs queued up behind each other
+// and bounded the long queues (whole frames with the default schedule: 128
+// environments of 512x512 at 8 spp 397 -> 159 ms, with the batches and tail
+// bounce of render_frame; 720p projector at 32 spp 57.4 -> 24.9 ms; 2 M rays
+// 1.45 -> 1.03 ms).  Measured around it: at most 512 or 1024 queries 2 and 6 %
+// slower on the 1080p frame (17.2 ms), 128 1 % slower on the projector and
+// the environments; a quarter of the share 1-4 % slower on 2 M rays and the
+// projector, all of it 18 % on 2 M rays; at least 32 queries 1 % slower on the
+// 1080p frame, 4 % denoised at 1 spp; at least 256 3 % slower on 2 M rays; the
+// queries of short launches spread at 4, 16 or 32 per wave instead of one per
+// lane 11, 5 and 4 % slower on a 256x256 frame.
 //   ctr[8 * kChunkStride]: per-chunk counters, zero before the launch.
 //   load(q, TRay&) fills the ray of query q and its payload;
 //   store(payload, best, found) writes a finished query.
-constexpr uint32_t kGuidedMin = 64, kGuidedMax = 1024;
+constexpr uint32_t kGrab = 256, kGrabMin = 64;  // kGrab: default grab
 constexpr uint32_t kChunkStride = 16;  // 8-byte counters per 128-byte line
 
 KF_DEV uint64_t chunk_begin(uint32_t n, uint32_t c) { return (uint64_t)n * c / 8u; }
@@ -728,8 +728,7 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
                     const uint64_t c0 = chunk_begin(n, chunk);
                     const uint32_t len = (uint32_t)(chunk_begin(n, chunk + 1u) - c0);
                     const uint32_t left = len - min(seen, len);
-                    const uint32_t take =
-                        min(most, grab ? grab : min(kGuidedMax, max(kGuidedMin, left / max(waves / 4u, 1u))));
+                    const uint32_t take = min(min(most, grab), max(kGrabMin, left / max(waves / 4u, 1u)));
                     unsigned long long base = 0;
                     if (lane == 0u) base = atomicAdd(&ctr[chunk * kChunkStride], (unsigned long long)take);
                     base = (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)base) |

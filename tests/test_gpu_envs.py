@@ -287,3 +287,23 @@ def test_tail_kernel_beyond_pair_capacity(gpu):
     lane pairs for (a quarter of a launch's threads: 131072 on 256 CUs), so
     k_tail takes them although tail_pairs is 1."""
     _assert_tail_equals_wavefront(scenes.config1(480, 360, spp=3), (1, 2, 3), pairs=(1,))
+
+
+@pytest.mark.parametrize("w,h,spp,extra,rr", [(48, 32, 1, 0, True), (768, 512, 1, 0, True), (769, 512, 1, 0, True),
+                                              (769, 512, 1, 2, True), (1024, 768, 2, 0, False), (1025, 768, 2, 0, False),
+                                              (1025, 768, 2, 0, True), (64, 64, 1, 3, True)])
+def test_default_schedule_equals_wavefront(gpu, w, h, spp, extra, rr):
+    """A renderer's own choice of the tail bounce, on either side of the path
+    and light counts where it changes, against the wavefront for every bounce."""
+    wl = scenes.config1(w, h, spp=spp, path_depth=6)
+    for k in range(extra):  # 2 lights and these
+        wl.data.add_point_light((k - 1.0, 3.0, 2.0), (1, 1, 1), 4.0, radius=0.0)
+    wl.pc.russian_roulette = int(rr)
+    gs = GpuScene(wl.data)
+    ra, rb = Renderer(w, h), Renderer(w, h)
+    rb.set_schedule(tail_bounce=wl.pc.path_depth + 1)
+    sa = ra.render(gs, wl.cam, wl.pc, seed=3)
+    sb = rb.render(gs, wl.cam, wl.pc, seed=3)
+    for t in range(3):
+        assert np.array_equal(ra.read(t), rb.read(t))
+    assert (sa.primary_rays, sa.extension_rays, sa.shadow_rays) == (sb.primary_rays, sb.extension_rays, sb.shadow_rays)
