@@ -384,8 +384,19 @@ int kf_scene_create(const kf_scene_desc* d, kf_scene** out) {
         for (uint32_t g = 0; g < s->n_geom; ++g)
             if (s->h_voff[g + 1] < s->h_voff[g] || s->h_toff[g + 1] < s->h_toff[g])
                 throw Error("kf_scene_create: offsets must be non-decreasing");
-        // validate indices and material indices (every device read stays in bounds)
-        for (uint32_t g = 0; g < s->n_geom; ++g) {
+        // validate indices and material indices (every device read stays in
+        // bounds): the largest of each geometry first, a loop without
+        // branches; the triangle loop names the first one out of range
+        uint32_t worst_mat = 0;
+        for (size_t t = 0; t < s->n_tri; ++t) worst_mat = std::max(worst_mat, d->mat_index[t]);
+        bool bad = s->n_tri && worst_mat >= s->n_mat;
+        for (uint32_t g = 0; g < s->n_geom && !bad; ++g) {
+            uint32_t worst = 0;
+            const size_t i0 = 3 * (size_t)s->h_toff[g], i1 = 3 * (size_t)s->h_toff[g + 1];
+            for (size_t i = i0; i < i1; ++i) worst = std::max(worst, d->indices[i]);
+            bad = i1 > i0 && worst >= s->h_voff[g + 1] - s->h_voff[g];
+        }
+        for (uint32_t g = 0; g < s->n_geom && bad; ++g) {
             uint32_t nv = s->h_voff[g + 1] - s->h_voff[g];
             for (size_t t = s->h_toff[g]; t < s->h_toff[g + 1]; ++t) {
                 for (int k = 0; k < 3; ++k)
@@ -433,6 +444,7 @@ int kf_scene_create(const kf_scene_desc* d, kf_scene** out) {
         KF_CHECK(hipEventCreate(&e0));
         KF_CHECK(hipEventCreate(&e1));
         KF_CHECK(hipEventRecord(e0, st));
+        map_triangles(*s);
         share_geometry(*s, d->vertices, d->indices, d->separate_geometry != 0);
         build_blas(*s);
         build_tlas(*s, d->instances, d->num_instances);

@@ -43,7 +43,8 @@ inline uint32_t tea_host(uint32_t v0, uint32_t v1) {
 //   a = (L.lo.x, L.hi.x, L.lo.y, L.hi.y)
 //   b = (R.lo.x, R.hi.x, R.lo.y, R.hi.y)
 //   c = (L.lo.z, L.hi.z, R.lo.z, R.hi.z)
-//   d = (left_ref, right_ref, -, -)
+//   d = (left_ref, right_ref, first leaf, last leaf), the leaves in sorted
+//       order over all BLAS / TLAS arrays
 // A child ref >= 0 is an internal node index (global over all BLAS / TLAS
 // arrays); < 0 is a leaf: ~leaf where leaf is a triangle slot (BLAS) or an
 // instance index (TLAS).
@@ -203,16 +204,10 @@ struct Scene {
 void lbvh_build(uint32_t n, const float4* d_lo, const float4* d_hi, const uint32_t* d_seg, uint32_t n_seg,
                 const uint32_t* d_seg_off, const uint32_t* d_node_off, Node* d_nodes, uint32_t* d_order,
                 int* d_root, bool leaf_is_slot, hipStream_t st);
-// Collapse a BVH2 into a BVH4 (level by level on the GPU): each BVH4 node
-// takes the two children of a BVH2 node and then repeatedly opens its inner
-// child of largest surface area until it has four.  roots2[i] (BVH2 root
-// refs, host) -> roots4[i] (BVH4 root refs); leaf and empty roots pass
-// through.  Returns the number of BVH4 nodes written to out (capacity cap).
-uint32_t collapse_bvh4(const Node* d_b2, uint32_t n_b2, const std::vector<int>& roots2, std::vector<int>& roots4,
-                       Node4* d_out, uint32_t cap, uint32_t inner_kind, hipStream_t st);
 // Root refs of the TLAS trees of environments with instance offsets env_off
 // and BVH2 node offsets node_off (known by construction, no device read).
 void env_roots(const std::vector<uint32_t>& env_off, const std::vector<uint32_t>& node_off, std::vector<int>& roots);
+void map_triangles(Scene& s);
 void build_blas(Scene& s);
 void upload_trav_roots(Scene& s);
 void upload_mesh_sources(Scene& s);

@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 
 import oracle
-from kuafu_amd import abi, scenes
+from kuafu_amd import abi, api, scenes
 from kuafu_amd.api import GpuScene, Renderer, push_constants
 
 pytestmark = pytest.mark.gpu
@@ -104,6 +104,49 @@ def test_blas_invariants(gpu):
     check_blas(gs2, 2)
     info = gs2.bvh_info()
     assert info.triangles == 5120 + 2 + 1 and info.max_blas_depth == d
+
+
+# Triangles per geometry: around the runs of 512 leaves that one pyramid block
+# reduces, around sort tiles (2048 keys), many segments per wave (geometries of
+# one to three triangles) and a geometry after them.
+@pytest.mark.parametrize("counts", [(2,), (3,), (511,), (512,), (513,), (1025,), (2049, 1, 2, 3), (1,) * 100 + (2, 70, 3) * 30,
+                                    (5000, 262145)])
+def test_blas_boxes_are_the_unions_of_their_triangles(gpu, counts):
+    rng = np.random.default_rng(len(counts) + counts[0])
+    s = scenes.SceneData()
+    m = s.add_material(scenes.material())
+    for n in counts:
+        pos = (rng.uniform(-5, 5, (n, 1, 3)) + rng.normal(0, 0.1, (n, 3, 3))).reshape(-1, 3).astype(np.float32)
+        s.add_geometry(api.vertices(pos), np.arange(3 * n, dtype=np.uint32).reshape(n, 3), m)
+    for g in range(len(counts)):
+        s.add_instance(g)
+    gs = GpuScene(s)
+    moved = s.geoms[-1][0].copy()
+    moved["pos"] = moved["pos"][:, [1, 2, 0]] * np.float32(1.5)
+    for step in range(2):
+        for g in ([0, len(counts) // 2, len(counts) - 1] if step == 0 else [len(counts) - 1]):
+            pos = (moved if step else s.geoms[g][0])["pos"].reshape(-1, 3, 3)
+            nodes, root, order = gs.read_blas(g)
+            n = counts[g]
+            assert sorted(order.tolist()) == list(range(n))
+            lo, hi = pos.min(1)[order], pos.max(1)[order]
+            refs = nodes[:, 12:14].copy().view(np.int32)
+            # ranges of leaves, children before parents
+            todo, seen = [root] if n > 1 else [], []
+            while todo:
+                r = todo.pop()
+                seen.append(r)
+                todo += [int(c) for c in refs[r] if c >= 0]
+            assert len(seen) == n - 1 == len(set(seen))
+            box = {}
+            for r in reversed(seen):
+                L, R = node_boxes(nodes[r])
+                for ref, b in ((int(refs[r, 0]), L), (int(refs[r, 1]), R)):
+                    want = np.stack([lo[~ref], hi[~ref]]) if ref < 0 else box[ref]
+                    assert np.array_equal(b, want)
+                box[r] = np.stack([np.minimum(L[0], R[0]), np.maximum(L[1], R[1])])
+        if step == 0:
+            gs.update_geometry(len(counts) - 1, moved)
 
 
 EMPTY_ITEM = 0xFFFFFFFF
