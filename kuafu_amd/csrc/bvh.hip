@@ -96,6 +96,19 @@ __device__ __forceinline__ uint32_t spread10(uint32_t v) {
     return v;
 }
 
+// 30-bit Morton code of centroid c in the bounds [l, h]; 0 for an empty box.
+__device__ __forceinline__ uint32_t morton30(bool full, const float c[3], const float l[3], const float h[3]) {
+    if (!full) return 0u;
+    uint32_t q[3];
+    for (int k = 0; k < 3; ++k) {
+        float e = h[k] - l[k];
+        float u = e > 0.0f ? (c[k] - l[k]) / e : 0.5f;
+        u = fminf(fmaxf(u, 0.0f), 1.0f);
+        q[k] = min((uint32_t)(u * 1024.0f), 1023u);
+    }
+    return (spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]);
+}
+
 __global__ void k_morton(uint32_t n, const float4* __restrict__ lo, const float4* __restrict__ hi,
                          const uint32_t* __restrict__ seg, const int* __restrict__ sb,
                          unsigned long long* __restrict__ keys, uint32_t* __restrict__ vals) {
@@ -103,19 +116,13 @@ __global__ void k_morton(uint32_t n, const float4* __restrict__ lo, const float4
     if (i >= n) return;
     uint32_t s = seg[i];
     float4 a = lo[i], b = hi[i];
-    uint32_t q[3] = {0, 0, 0};
-    if (a.x <= b.x) {
-        float c[3] = {0.5f * (a.x + b.x), 0.5f * (a.y + b.y), 0.5f * (a.z + b.z)};
-        for (int k = 0; k < 3; ++k) {
-            float l = ord2f(sb[6 * s + k]), h = ord2f(sb[6 * s + 3 + k]);
-            float e = h - l;
-            float u = e > 0.0f ? (c[k] - l) / e : 0.5f;
-            u = fminf(fmaxf(u, 0.0f), 1.0f);
-            q[k] = min((uint32_t)(u * 1024.0f), 1023u);
-        }
+    const float c[3] = {0.5f * (a.x + b.x), 0.5f * (a.y + b.y), 0.5f * (a.z + b.z)};
+    float l[3], h[3];
+    for (int k = 0; k < 3; ++k) {
+        l[k] = ord2f(sb[6 * s + k]);
+        h[k] = ord2f(sb[6 * s + 3 + k]);
     }
-    uint32_t m = (spread10(q[0]) << 2) | (spread10(q[1]) << 1) | spread10(q[2]);
-    keys[i] = ((unsigned long long)s << 30) | m;
+    keys[i] = ((unsigned long long)s << 30) | morton30(a.x <= b.x, c, l, h);
     vals[i] = i;
 }
 
@@ -317,11 +324,37 @@ __global__ __launch_bounds__(kPyrThreads) void k_pyramid(Pyramid P, int k0, uint
 }
 
 // ---------------------------------------------------------------- Karras
-__device__ __forceinline__ int delta(const unsigned long long* k, int n, int a, int b) {
-    if (b < 0 || b >= n) return -1;
-    unsigned long long x = k[a] ^ k[b];
-    if (x) return __clzll(x);
-    return 64 + __clz((uint32_t)(a ^ b));
+// Node i of the hierarchy over n >= 2 sorted keys: its leaves first .. last,
+// the left child's being first .. split.
+struct KarrasNode {
+    int first, split, last;
+};
+template <class Key>
+KF_DEV_INLINE KarrasNode karras_node(Key key, int n, int i) {
+    auto delta = [&](int a, int b) {
+        if (b < 0 || b >= n) return -1;
+        const unsigned long long x = key(a) ^ key(b);
+        return x ? __clzll(x) : 64 + __clz((uint32_t)(a ^ b));
+    };
+    const int d = (delta(i, i + 1) - delta(i, i - 1)) >= 0 ? 1 : -1;
+    const int dmin = delta(i, i - d);
+    int lmax = 2;
+    while (delta(i, i + lmax * d) > dmin) lmax <<= 1;
+    int l = 0;
+    for (int t = lmax >> 1; t >= 1; t >>= 1)
+        if (delta(i, i + (l + t) * d) > dmin) l += t;
+    const int j = i + l * d;
+    const int dnode = delta(i, j);
+    int sp = 0;
+    int div = 2;
+    int t = (l + div - 1) / div;
+    while (true) {
+        if (delta(i, i + (sp + t) * d) > dnode) sp += t;
+        if (t == 1) break;
+        div <<= 1;
+        t = (l + div - 1) / div;
+    }
+    return {min(i, j), i + sp * d + min(d, 0), max(i, j)};
 }
 
 // A node from its range of leaves: child boxes, child refs and (d.zw) the
@@ -347,26 +380,8 @@ __global__ void k_karras(uint32_t n, const unsigned long long* __restrict__ keys
     int i = (int)(gi - so);
     if (i >= ns - 1) return;
     const unsigned long long* k = keys + so;
-    int d = (delta(k, ns, i, i + 1) - delta(k, ns, i, i - 1)) >= 0 ? 1 : -1;
-    int dmin = delta(k, ns, i, i - d);
-    int lmax = 2;
-    while (delta(k, ns, i, i + lmax * d) > dmin) lmax <<= 1;
-    int l = 0;
-    for (int t = lmax >> 1; t >= 1; t >>= 1)
-        if (delta(k, ns, i, i + (l + t) * d) > dmin) l += t;
-    int j = i + l * d;
-    int dnode = delta(k, ns, i, j);
-    int sp = 0;
-    int div = 2;
-    int t = (l + div - 1) / div;
-    while (true) {
-        if (delta(k, ns, i, i + (sp + t) * d) > dnode) sp += t;
-        if (t == 1) break;
-        div <<= 1;
-        t = (l + div - 1) / div;
-    }
-    const int gamma = i + sp * d + min(d, 0);
-    const int first = min(i, j), last = max(i, j), nb = (int)node_off[s];
+    const KarrasNode kn = karras_node([&](int a) { return k[a]; }, ns, i);
+    const int first = kn.first, gamma = kn.split, last = kn.last, nb = (int)node_off[s];
     auto leaf = [&](int q) { return ~(leaf_is_slot ? (int)so + q : (int)order[so + q]); };
     const int lref = first == gamma ? leaf(gamma) : nb + gamma;
     const int rref = last == gamma + 1 ? leaf(gamma + 1) : nb + gamma + 1;
@@ -394,8 +409,10 @@ template <class T> void dfree(T* p) {
 
 inline uint32_t blocks(uint32_t n, uint32_t b) { return (n + b - 1) / b; }
 
-// The pyramid over n > 0 leaves with the boxes lo / hi of order[0 .. n).
-Pyramid build_pyramid(uint32_t n, const uint32_t* order, const float4* lo, const float4* hi, hipStream_t st) {
+// The pyramid over n > 0 leaves with the boxes lo / hi of order[0 .. n), in
+// `at` (pyramid_size(n) boxes).
+size_t pyramid_size(uint32_t n) { return 2 * (size_t)n + kMaxLevels; }
+Pyramid build_pyramid(uint32_t n, const uint32_t* order, const float4* lo, const float4* hi, Box* at, hipStream_t st) {
     Pyramid P;
     uint32_t len[kMaxLevels], total = 0;
     for (uint32_t m = n;; m = (m + 1u) / 2u) {
@@ -404,7 +421,7 @@ Pyramid build_pyramid(uint32_t n, const uint32_t* order, const float4* lo, const
         total += m;
         if (m == 1u) break;
     }
-    P.at = dalloc<Box>(total);
+    P.at = at;
     for (int k = 0; k == 0 || k + 1 < P.levels; k += kPyrLevels)
         k_pyramid<<<blocks(len[k], kPyrItems), kPyrThreads, 0, st>>>(P, k, len[k], k == 0, order, lo, hi);
     return P;
@@ -499,52 +516,60 @@ __global__ void k_blas_box(uint32_t n_geom, const int* __restrict__ root, const 
     ghi[g] = hi;
 }
 
-// Instance records + padded world AABBs (corners transformed in double).
-// root: BVH4 root ref of each geometry (node index, ~triangle slot for a
-// BLAS of one triangle, kEmptyRef); blas4: the BVH4 nodes it indexes; mesh:
-// (voff, toff) of the arrays each geometry's shading reads; toff: each
-// geometry's own triangle offset.
-__global__ void k_instances(uint32_t n, const kf_instance* __restrict__ src, const float* __restrict__ w2o,
-                            uint32_t n_geom, const uint32_t* __restrict__ gflags, const int* __restrict__ root,
-                            const Node4* __restrict__ blas4, uint32_t n_blas4,
-                            const float4* __restrict__ glo, const float4* __restrict__ ghi,
-                            const uint2* __restrict__ mesh, const uint32_t* __restrict__ toff,
-                            const uint32_t* __restrict__ inst_env, Inst* __restrict__ out,
-                            float4* __restrict__ ilo, float4* __restrict__ ihi, uint32_t* __restrict__ iseg) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const kf_instance& in = src[i];
-    uint32_t g = in.geometry_index;
+// What an instance record is made from.  root: BVH4 root ref of each geometry
+// (node index, ~triangle slot for a BLAS of one triangle, kEmptyRef); blas4:
+// the BVH4 nodes it indexes; glo / ghi: its BLAS box; mesh: (voff, toff) of
+// the arrays each geometry's shading reads; toff: each geometry's own triangle
+// offset.
+struct InstArgs {
+    const kf_instance* src;
+    uint32_t n_geom;
+    const uint32_t* gflags;
+    const int* root;
+    const Node4* blas4;
+    uint32_t n_blas4;
+    const float4 *glo, *ghi;
+    const uint2* mesh;
+    const uint32_t* toff;
+    Inst* out;
+    float4 *ilo, *ihi;
+};
+
+// Record and padded world AABB (corners transformed in double) of instance i.
+KF_DEV_INLINE Box make_instance(const InstArgs& A, uint32_t i) {
+    const kf_instance in = A.src[i];
+    const uint32_t g = in.geometry_index, n_geom = A.n_geom;
     Inst rec;
-    for (int r = 0; r < 3; ++r) rec.w2o[r] = make_float4(w2o[12 * i + 4 * r], w2o[12 * i + 4 * r + 1],
-                                                         w2o[12 * i + 4 * r + 2], w2o[12 * i + 4 * r + 3]);
-    const int r4 = g < n_geom ? root[g] : kEmptyRef;
-    bool valid = g < n_geom && !(gflags[g] & KF_GEOM_HIDDEN) && r4 != kEmptyRef && (r4 < 0 || (uint32_t)r4 < n_blas4);
-    int flags = (valid ? kInstValid : 0) | ((g < n_geom && (gflags[g] & KF_GEOM_OPAQUE)) ? kInstOpaque : 0);
+    float w2o[12];
+    world_to_object(in.transform, w2o);
+    for (int r = 0; r < 3; ++r) rec.w2o[r] = make_float4(w2o[4 * r], w2o[4 * r + 1], w2o[4 * r + 2], w2o[4 * r + 3]);
+    const int r4 = g < n_geom ? A.root[g] : kEmptyRef;
+    bool valid = g < n_geom && !(A.gflags[g] & KF_GEOM_HIDDEN) && r4 != kEmptyRef && (r4 < 0 || (uint32_t)r4 < A.n_blas4);
+    int flags = (valid ? kInstValid : 0) | ((g < n_geom && (A.gflags[g] & KF_GEOM_OPAQUE)) ? kInstOpaque : 0);
     rec.info = make_int4(valid ? r4 : kEmptyRef, (int)g, flags, 0);
-    rec.shade = g < n_geom ? make_int4((int)mesh[g].x, (int)mesh[g].y, (int)toff[g], 0) : make_int4(0, 0, 0, 0);
+    rec.shade = g < n_geom ? make_int4((int)A.mesh[g].x, (int)A.mesh[g].y, (int)A.toff[g], 0) : make_int4(0, 0, 0, 0);
     // the BLAS root node, as the traversal's instance step tests it
     const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     rec.lox = rec.hix = rec.loy = rec.hiy = rec.loz = rec.hiz = z;
     rec.ref = make_int4((int)kEmptyItem, (int)kEmptyItem, (int)kEmptyItem, (int)kEmptyItem);
     if (valid && r4 >= 0) {
-        const Node4 nd = blas4[r4];
+        const Node4 nd = A.blas4[r4];
         rec.lox = nd.lox; rec.hix = nd.hix; rec.loy = nd.loy; rec.hiy = nd.hiy; rec.loz = nd.loz; rec.hiz = nd.hiz;
         rec.ref = nd.ref;
     } else if (valid) {  // one triangle: its box (the geometry's) as the only child
-        const float4 a = glo[g], b = ghi[g];
+        const float4 a = A.glo[g], b = A.ghi[g];
         rec.lox.x = a.x; rec.hix.x = b.x; rec.loy.x = a.y; rec.hiy.x = b.y; rec.loz.x = a.z; rec.hiz.x = b.z;
         rec.ref.x = (int)((3u << 30) | (uint32_t)~r4);  // triangle item
     }
-    out[i] = rec;
-    float4 lo = make_float4(INFINITY, INFINITY, INFINITY, 0), hi = make_float4(-INFINITY, -INFINITY, -INFINITY, 0);
+    A.out[i] = rec;
+    Box box = box_empty();
     if (valid) {
-        float4 a = glo[g], b = ghi[g];
+        const float4 a = A.glo[g], b = A.ghi[g];
         double l[3] = {INFINITY, INFINITY, INFINITY}, h[3] = {-INFINITY, -INFINITY, -INFINITY};
-        const float* t = in.transform;
         for (int c = 0; c < 8; ++c) {
             double p[3] = {(c & 1) ? b.x : a.x, (c & 2) ? b.y : a.y, (c & 4) ? b.z : a.z};
             for (int r = 0; r < 3; ++r) {
+                const float* t = in.transform;
                 double v = (double)t[r] * p[0] + (double)t[4 + r] * p[1] + (double)t[8 + r] * p[2] + (double)t[12 + r];
                 l[r] = fmin(l[r], v);
                 h[r] = fmax(h[r], v);
@@ -557,11 +582,18 @@ __global__ void k_instances(uint32_t n, const kf_instance* __restrict__ src, con
             fl[r] = nextafterf((float)(l[r] - pad), -INFINITY);
             fh[r] = nextafterf((float)(h[r] + pad), INFINITY);
         }
-        lo = make_float4(fl[0], fl[1], fl[2], 0);
-        hi = make_float4(fh[0], fh[1], fh[2], 0);
+        box.lo = make_float4(fl[0], fl[1], fl[2], 0);
+        box.hi = make_float4(fh[0], fh[1], fh[2], 0);
     }
-    ilo[i] = lo;
-    ihi[i] = hi;
+    A.ilo[i] = box.lo;
+    A.ihi[i] = box.hi;
+    return box;
+}
+
+__global__ void k_instances(uint32_t n, InstArgs A, const uint32_t* __restrict__ inst_env, uint32_t* __restrict__ iseg) {
+    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    make_instance(A, i);
     iseg[i] = inst_env ? inst_env[i] : 0u;  // the LBVH segment is the environment
 }
 
@@ -572,19 +604,20 @@ KF_DEV_INLINE float half_area(const float lo[3], const float hi[3]) {
 }
 
 // One item of the collapse: (BVH2 node b, BVH4 slot w) writes BVH4 node w
-// and queues its inner children for the next level.  err is set on any index
+// and queues its inner children for the next level.  b2 holds the n_b2 nodes
+// from node b2_base on.  err is set on any index
 // outside the arrays (malformed input), and nothing is written out of bounds.
-KF_DEV_INLINE void collapse_item(const Node* __restrict__ b2, uint32_t n_b2, int2 it, int2* __restrict__ out,
+KF_DEV_INLINE void collapse_item(const Node* __restrict__ b2, uint32_t b2_base, uint32_t n_b2, int2 it, int2* __restrict__ out,
                                  uint32_t* out_count, uint32_t out_cap, Node4* __restrict__ wide,
                                  uint32_t* wide_count, uint32_t wide_cap, uint32_t inner_kind, int* err) {
-    if ((uint32_t)it.x >= n_b2 || (uint32_t)it.y >= wide_cap) {
+    if ((uint32_t)it.x - b2_base >= n_b2 || (uint32_t)it.y >= wide_cap) {
         *err = 1;
         return;
     }
     float lo[4][3], hi[4][3];
     int ref[4];
     auto take = [&](int node, int s0, int s1) {
-        const Node n = b2[node];
+        const Node n = b2[(uint32_t)node - b2_base];
         lo[s0][0] = n.a.x; hi[s0][0] = n.a.y; lo[s0][1] = n.a.z; hi[s0][1] = n.a.w; lo[s0][2] = n.c.x; hi[s0][2] = n.c.y;
         lo[s1][0] = n.b.x; hi[s1][0] = n.b.y; lo[s1][1] = n.b.z; hi[s1][1] = n.b.w; lo[s1][2] = n.c.z; hi[s1][2] = n.c.w;
         ref[s0] = n.d.x;
@@ -604,7 +637,7 @@ KF_DEV_INLINE void collapse_item(const Node* __restrict__ b2, uint32_t n_b2, int
                 }
             }
         if (best < 0) break;
-        if ((uint32_t)ref[best] >= n_b2) {
+        if ((uint32_t)ref[best] - b2_base >= n_b2) {
             *err = 1;
             return;
         }
@@ -656,55 +689,189 @@ KF_DEV_INLINE void collapse_item(const Node* __restrict__ b2, uint32_t n_b2, int
     wide[it.y] = W;
 }
 
-// The whole collapse of a forest with no host round trip (TLAS updates,
-// every frame): block e collapses tree e, level after level.  Tree e has the
-// n_e = seg_off[e+1] - seg_off[e] leaves of its LBVH segment; for n_e >= 2
-// its n_e - 1 BVH2 nodes start at node_off[e], with the root first, and its
-// BVH4 takes slots [node_off[e], node_off[e] + n_e - 1) of `wide` (a BVH4
-// never has more nodes than its BVH2), root first; qa / qb hold its level
-// queues in the same index range.  cnt + 2e: [0] next free BVH4 slot,
-// [1] next-level queue length (scratch).
-constexpr int kTreeThreads = 1024;
-__global__ __launch_bounds__(kTreeThreads) void k_collapse_forest(const Node* __restrict__ b2, uint32_t n_b2,
-                                                                  const uint32_t* __restrict__ seg_off,
-                                                                  const uint32_t* __restrict__ node_off, int2* qa_all,
-                                                                  int2* qb_all, Node4* __restrict__ wide,
-                                                                  uint32_t inner_kind, uint32_t* cnt_all, int* err) {
-    const uint32_t e = blockIdx.x;
-    const uint32_t n_e = seg_off[e + 1] - seg_off[e];
-    if (n_e < 2u) return;  // a single instance or none: the root is a leaf or empty
-    const uint32_t base = node_off[e], cap_e = n_e - 1u;
-    if (base + cap_e > n_b2) {
-        if (threadIdx.x == 0) *err = 1;
-        return;
-    }
-    int2* qa = qa_all + base;
-    int2* qb = qb_all + base;
-    uint32_t* cnt = cnt_all + 2 * e;
-    __shared__ uint32_t n_in;
+// A block collapses one tree of n_e >= 2 leaves, level after level: BVH2
+// nodes [base, base + n_e - 1) (at b2), root first, into BVH4 slots [base,
+// base + n_e - 1) of `wide` (a BVH4 never has more nodes than its BVH2), root
+// first; qa / qb hold its level queues.  cnt[0]: next free BVH4 slot, cnt[1]:
+// next-level queue length.
+KF_DEV_INLINE void collapse_tree(const Node* b2, uint32_t base, uint32_t n_e, int2* qa, int2* qb,
+                                 Node4* __restrict__ wide, uint32_t inner_kind, uint32_t* cnt, uint32_t* n_in, int* err) {
+    const uint32_t cap_e = n_e - 1u;
     if (threadIdx.x == 0) {
-        n_in = 1u;
+        *n_in = 1u;
         cnt[0] = base + 1u;
         cnt[1] = 0u;
         qa[0] = make_int2((int)base, (int)base);
     }
     __syncthreads();
-    for (uint32_t level = 0; n_in > 0u; ++level) {
+    for (uint32_t level = 0; *n_in > 0u; ++level) {
         if (level > cap_e + 1u) {  // deeper than a well-formed tree can be
             if (threadIdx.x == 0) *err = 1;
             break;
         }
-        for (uint32_t i = threadIdx.x; i < n_in; i += blockDim.x)
-            collapse_item(b2, n_b2, qa[i], qb, &cnt[1], cap_e, wide, &cnt[0], base + cap_e, inner_kind, err);
+        for (uint32_t i = threadIdx.x; i < *n_in; i += blockDim.x)
+            collapse_item(b2, base, cap_e, qa[i], qb, &cnt[1], cap_e, wide, &cnt[0], base + cap_e, inner_kind, err);
         __syncthreads();
         if (threadIdx.x == 0) {
-            n_in = min(cnt[1], cap_e);
+            *n_in = min(cnt[1], cap_e);
             cnt[1] = 0u;
         }
         __syncthreads();
         int2* t = qa;
         qa = qb;
         qb = t;
+    }
+}
+
+// The whole collapse of a forest with no host round trip: block e collapses
+// tree e, the n_e = seg_off[e+1] - seg_off[e] leaves of its LBVH segment, whose
+// nodes start at node_off[e].  cnt_all + 2e: collapse_tree's counters.
+constexpr int kTreeThreads = 1024;
+__global__ __launch_bounds__(kTreeThreads) void k_collapse_forest(const Node* __restrict__ b2, uint32_t n_b2,
+                                                                  const uint32_t* __restrict__ seg_off,
+                                                                  const uint32_t* __restrict__ node_off, int2* qa_all,
+                                                                  int2* qb_all, Node4* __restrict__ wide,
+                                                                  uint32_t inner_kind, uint32_t* cnt_all, int* err) {
+    __shared__ uint32_t n_in;
+    const uint32_t e = blockIdx.x;
+    const uint32_t n_e = seg_off[e + 1] - seg_off[e];
+    if (n_e < 2u) return;  // a single instance or none: the root is a leaf or empty
+    const uint32_t base = node_off[e];
+    if (base + n_e - 1u > n_b2) {
+        if (threadIdx.x == 0) *err = 1;
+        return;
+    }
+    collapse_tree(b2 + base, base, n_e, qa_all + base, qb_all + base, wide, inner_kind, cnt_all + 2 * e, &n_in, err);
+}
+
+// ---------------------------------------------------------------- small TLAS
+// The TLAS of environment blockIdx.x in one block, for at most M instances:
+// instance records and boxes, centroid bounds, Morton codes, a bitonic sort on
+// (code, instance), the box pyramid, the Karras nodes and the BVH4 collapse,
+// all in LDS but for the results; the same trees as the general path, whose
+// 27 launches and 30 allocations took 281 us per update of 65 instances.  Now
+// 41 us, 32 of them this kernel: a chain of short steps (the double-precision
+// record, 28 compare-exchange rounds, four collapse levels) on one CU.
+// env_off, node_off: null for one environment of n instances.
+template <int M>
+__global__ __launch_bounds__(M) void k_tlas_small(uint32_t n, InstArgs A, const uint32_t* __restrict__ env_off,
+                                                  const uint32_t* __restrict__ node_off, Node* __restrict__ nodes,
+                                                  Node4* __restrict__ wide, uint32_t* __restrict__ cnt_all, int* err) {
+    struct Box6 {
+        float v[6];  // lo, hi
+    };
+    __shared__ unsigned long long key[M];
+    __shared__ Box6 pyr[2 * M];  // level k from entry 2M - (2M >> k)
+    __shared__ Node tree[M];
+    __shared__ int2 qa[M], qb[M];
+    __shared__ float bounds[6][M / 64];
+    __shared__ uint32_t cnt[2], n_in;
+    const uint32_t e = blockIdx.x, t = threadIdx.x;
+    const uint32_t so = env_off ? env_off[e] : 0u, n_e = (env_off ? env_off[e + 1] : n) - so;
+    const uint32_t nb = node_off ? node_off[e] : 0u;
+    if (n_e > (uint32_t)M) {  // the host sizes M for the largest environment
+        if (t == 0) *err = 1;
+        return;
+    }
+    const bool on = t < n_e;
+    Box box = box_empty();
+    if (on) box = make_instance(A, so + t);
+    if (n_e < 2u) return;  // uniform: a single instance or none has no node
+    // centroid bounds of the non-empty boxes
+    const bool full = on && box.lo.x <= box.hi.x;
+    const float c[3] = {0.5f * (box.lo.x + box.hi.x), 0.5f * (box.lo.y + box.hi.y), 0.5f * (box.lo.z + box.hi.z)};
+    float bl[3], bh[3];
+    for (int k = 0; k < 3; ++k) {
+        float l = full ? c[k] : INFINITY, h = full ? c[k] : -INFINITY;
+        for (int off = 32; off > 0; off >>= 1) {
+            l = fminf(l, __shfl_xor(l, off));
+            h = fmaxf(h, __shfl_xor(h, off));
+        }
+        if ((t & 63u) == 0u) {
+            bounds[k][t >> 6] = l;
+            bounds[3 + k][t >> 6] = h;
+        }
+    }
+    __syncthreads();
+    for (int k = 0; k < 3; ++k) {
+        bl[k] = INFINITY;
+        bh[k] = -INFINITY;
+        for (int w = 0; w < M / 64; ++w) {
+            bl[k] = fminf(bl[k], bounds[k][w]);
+            bh[k] = fmaxf(bh[k], bounds[3 + k][w]);
+        }
+    }
+    key[t] = on ? ((unsigned long long)morton30(full, c, bl, bh) << 32) | t : ~0ull;
+    // boxes by instance, where the pyramid's upper levels go later
+    for (int k = 0; k < 3; ++k) {
+        pyr[M + t].v[k] = k == 0 ? box.lo.x : k == 1 ? box.lo.y : box.lo.z;
+        pyr[M + t].v[3 + k] = k == 0 ? box.hi.x : k == 1 ? box.hi.y : box.hi.z;
+    }
+    for (uint32_t size = 2; size < 2u * n_e; size <<= 1)
+        for (uint32_t j = size >> 1; j > 0; j >>= 1) {
+            __syncthreads();
+            const uint32_t q = t ^ j;
+            if (q > t) {
+                const unsigned long long a = key[t], b = key[q];
+                if ((a > b) == ((t & size) == 0u)) {
+                    key[t] = b;
+                    key[q] = a;
+                }
+            }
+        }
+    __syncthreads();
+    Box6 mine = pyr[M + (on ? (uint32_t)key[t] : 0u)];
+    if (!on)
+        for (int k = 0; k < 6; ++k) mine.v[k] = k < 3 ? INFINITY : -INFINITY;
+    pyr[t] = mine;
+    __syncthreads();
+    for (uint32_t k = 1, w = M / 2; w > 0; ++k, w >>= 1) {
+        const uint32_t from = 2u * M - (2u * M >> (k - 1)), to = 2u * M - (2u * M >> k);
+        if (t < w)
+            for (int j = 0; j < 6; ++j) {
+                const float x = pyr[from + 2 * t].v[j], y = pyr[from + 2 * t + 1].v[j];
+                pyr[to + t].v[j] = j < 3 ? fminf(x, y) : fmaxf(x, y);
+            }
+        __syncthreads();
+    }
+    auto range = [&](uint32_t l, uint32_t r, Box6& b) {
+        b = pyr[l];
+        if (l == r) return;
+        for (int j = 0; j < 6; ++j) b.v[j] = j < 3 ? INFINITY : -INFINITY;
+        auto add = [&](uint32_t i) {
+            for (int j = 0; j < 6; ++j) b.v[j] = j < 3 ? fminf(b.v[j], pyr[i].v[j]) : fmaxf(b.v[j], pyr[i].v[j]);
+        };
+        for (uint32_t at = 0, w = M; l <= r; at += w, w >>= 1) {
+            if (l & 1u) add(at + l++);
+            if (!(r & 1u)) {
+                add(at + r);
+                if (r == 0u) break;
+                --r;
+            }
+            l >>= 1;
+            r >>= 1;
+        }
+    };
+    if (t + 1u < n_e) {
+        const KarrasNode kn = karras_node([&](int a) { return key[a] >> 32; }, (int)n_e, (int)t);
+        auto leaf = [&](int q) { return ~(int)(so + (uint32_t)key[q]); };
+        const int lref = kn.first == kn.split ? leaf(kn.split) : (int)nb + kn.split;
+        const int rref = kn.last == kn.split + 1 ? leaf(kn.split + 1) : (int)nb + kn.split + 1;
+        Box6 L, R;
+        range((uint32_t)kn.first, (uint32_t)kn.split, L);
+        range((uint32_t)kn.split + 1u, (uint32_t)kn.last, R);
+        Node m;
+        m.a = make_float4(L.v[0], L.v[3], L.v[1], L.v[4]);
+        m.b = make_float4(R.v[0], R.v[3], R.v[1], R.v[4]);
+        m.c = make_float4(L.v[2], L.v[5], R.v[2], R.v[5]);
+        m.d = make_int4(lref, rref, (int)so + kn.first, (int)so + kn.last);
+        tree[t] = m;
+        nodes[nb + t] = m;
+    }
+    collapse_tree(tree, nb, n_e, qa, qb, wide, 0u, cnt, &n_in, err);
+    if (t == 0) {
+        cnt_all[2 * e] = cnt[0];
+        cnt_all[2 * e + 1] = 0u;
     }
 }
 
@@ -743,12 +910,13 @@ void lbvh_build(uint32_t n, const float4* d_lo, const float4* d_hi, const uint32
         std::swap(k0, k1);
         if (!last) std::swap(v0, v1);
     }
-    const Pyramid P = build_pyramid(n, d_order, d_lo, d_hi, st);
+    Box* pyr = dalloc<Box>(pyramid_size(n));
+    const Pyramid P = build_pyramid(n, d_order, d_lo, d_hi, pyr, st);
     k_karras<<<blocks(n, TB), TB, 0, st>>>(n, k0, d_order, d_seg_off, d_node_off, P, d_nodes, leaf_is_slot);
     k_seg_root<<<blocks(n_seg, TB), TB, 0, st>>>(n_seg, d_seg_off, d_node_off, d_order, d_root, leaf_is_slot);
     KF_CHECK(hipGetLastError());
     dfree(sb); dfree(k0); dfree(k1); dfree(v0); dfree(v1);
-    dfree(hist); dfree(P.at);
+    dfree(hist); dfree(pyr);
 }
 
 // The geometry of every triangle.
@@ -757,6 +925,13 @@ void map_triangles(Scene& s) {
     if (s.n_tri)
         k_tri_geom<<<blocks(s.n_tri, 256), 256, 0, stream()>>>(s.n_tri, s.n_geom, s.d_toff, s.d_tri_geom);
     KF_CHECK(hipGetLastError());
+}
+
+// d_glo / d_ghi, after a build or refit.
+void blas_boxes(Scene& s) {
+    if (s.n_geom)
+        k_blas_box<<<blocks(s.n_geom, 256), 256, 0, stream()>>>(s.n_geom, s.d_blas_root, s.d_blas, s.d_tri, s.d_glo,
+                                                                s.d_ghi);
 }
 
 void build_blas(Scene& s) {
@@ -835,6 +1010,9 @@ void build_blas(Scene& s) {
     KF_CHECK(hipStreamSynchronize(st));
     dfree(err);
     if (h_err) throw Error("BLAS build: malformed BVH2");
+    s.d_glo = dalloc<float4>(std::max<uint32_t>(s.n_geom, 1));
+    s.d_ghi = dalloc<float4>(std::max<uint32_t>(s.n_geom, 1));
+    blas_boxes(s);
     upload_trav_roots(s);
     upload_mesh_sources(s);
 }
@@ -973,8 +1151,10 @@ __global__ void k_equal_vertices(uint32_t n_vert, uint32_t n_geom, const uint4* 
     }
 }
 
-// g leaves its group: the next member leads the rest.
-void leave_group(std::vector<uint32_t>& lead, uint32_t g) {
+// g leaves its group: the next member leads the rest.  False when it was
+// alone already.
+bool leave_group(std::vector<uint32_t>& lead, uint32_t g) {
+    bool moved = lead[g] != g;
     if (lead[g] == g) {
         uint32_t m = UINT32_MAX;
         for (uint32_t d = 0; d < lead.size(); ++d)
@@ -982,8 +1162,10 @@ void leave_group(std::vector<uint32_t>& lead, uint32_t g) {
                 if (m == UINT32_MAX) m = d;
                 lead[d] = m;
             }
+        moved = m != UINT32_MAX;
     }
     lead[g] = g;
+    return moved;
 }
 }  // namespace
 
@@ -1075,10 +1257,8 @@ void share_geometry(Scene& s, const kf_vertex* verts, const uint32_t* idx, bool 
 
 void unshare_geometry(Scene& s, uint32_t g) {
     if (g >= s.n_geom) return;
-    if (s.h_canon.size() == s.n_geom) leave_group(s.h_canon, g);
-    if (s.h_mesh.size() == s.n_geom) leave_group(s.h_mesh, g);
-    upload_trav_roots(s);
-    upload_mesh_sources(s);
+    if (s.h_canon.size() == s.n_geom && leave_group(s.h_canon, g)) upload_trav_roots(s);
+    if (s.h_mesh.size() == s.n_geom && leave_group(s.h_mesh, g)) upload_mesh_sources(s);
 }
 
 // ---------------------------------------------------------------- refit
@@ -1184,11 +1364,15 @@ void env_roots(const std::vector<uint32_t>& env_off, const std::vector<uint32_t>
 
 // TLAS (re)build, once per instance update: instance records + world boxes,
 // an LBVH over the instances of each environment (one segment each), the
-// BVH4 collapse of every environment's tree in one launch.  Nothing here
+// BVH4 collapse of every environment's tree, in one launch when no environment
+// has more than kTlasSmall instances (what a block's LDS holds).  Up to
+// kTlasDirect instances the kernel reads them from the pinned staging (80
+// bytes each over the bus, less than a copy's launch), beyond after a copy.  Nothing here
 // waits for the GPU: roots are known by construction (env_roots) and the
 // host inputs go through pinned staging.  One environment: its segment and
 // node offsets are written on the device (the instance count may change);
 // several: they are fixed at scene creation (the count may not).
+constexpr uint32_t kTlasSmall = 1024, kTlasDirect = 2048;
 void build_tlas(Scene& s, const kf_instance* h_inst, uint32_t n) {
     hipStream_t st = stream();
     const uint32_t TB = 256;
@@ -1214,43 +1398,43 @@ void build_tlas(Scene& s, const kf_instance* h_inst, uint32_t n) {
         KF_CHECK(hipMemsetAsync(s.d_tlas_err, 0, sizeof(int), st));
         KF_CHECK(hipEventCreateWithFlags(&s.stage_ev, hipEventDisableTiming));
     }
-    // host inputs -> pinned staging -> device
-    const size_t w2o_bytes = 12 * sizeof(float) * (size_t)n, inst_bytes = sizeof(kf_instance) * (size_t)n;
-    if (s.stage_pending) KF_CHECK(hipEventSynchronize(s.stage_ev));  // the previous update's copies are done
+    // host instances -> pinned staging, read by the kernel there (few) or
+    // copied to the device (many)
+    const size_t inst_bytes = sizeof(kf_instance) * (size_t)n;
+    if (s.stage_pending) KF_CHECK(hipEventSynchronize(s.stage_ev));  // the previous update has read it
     s.stage_pending = false;
-    if (w2o_bytes + inst_bytes > s.stage_cap) {
+    if (inst_bytes > s.stage_cap) {
         if (s.h_stage) KF_CHECK(hipHostFree(s.h_stage));
-        s.stage_cap = std::max<size_t>(w2o_bytes + inst_bytes, 4096);
-        KF_CHECK(hipHostMalloc((void**)&s.h_stage, s.stage_cap, hipHostMallocDefault));
+        s.h_stage = nullptr;
+        s.stage_cap = 0;
+        const size_t cap = std::max<size_t>(inst_bytes, 4096);
+        KF_CHECK(hipHostMalloc((void**)&s.h_stage, cap, hipHostMallocDefault));
+        s.stage_cap = cap;
     }
-    float* w2o = (float*)s.h_stage;
-    for (uint32_t i = 0; i < n; ++i) kf_world_to_object(h_inst[i].transform, &w2o[12 * i]);
-    if (n) std::memcpy(s.h_stage + w2o_bytes, h_inst, inst_bytes);
-    float* d_w2o = dalloc<float>(std::max<size_t>(12 * (size_t)n, 1));
-    if (n) {
-        KF_CHECK(hipMemcpyAsync(d_w2o, s.h_stage, w2o_bytes, hipMemcpyHostToDevice, st));
-        KF_CHECK(hipMemcpyAsync(s.d_inst_src, s.h_stage + w2o_bytes, inst_bytes, hipMemcpyHostToDevice, st));
-        KF_CHECK(hipEventRecord(s.stage_ev, st));
-        s.stage_pending = true;
+    if (n) std::memcpy(s.h_stage, h_inst, inst_bytes);
+    uint32_t most = n;  // instances of the largest environment
+    if (multi) {
+        most = 0;
+        for (uint32_t e = 0; e < s.n_env; ++e) most = std::max(most, s.h_env_off[e + 1] - s.h_env_off[e]);
     }
-    float4* glo = dalloc<float4>(std::max<uint32_t>(s.n_geom, 1));
-    float4* ghi = dalloc<float4>(std::max<uint32_t>(s.n_geom, 1));
-    if (s.n_geom) k_blas_box<<<blocks(s.n_geom, TB), TB, 0, st>>>(s.n_geom, s.d_blas_root, s.d_blas, s.d_tri, glo, ghi);
-    float4* ilo = s.d_ilo;  // kept: the renderer culls instances per pixel tile with them
-    float4* ihi = s.d_ihi;
-    uint32_t* iseg = dalloc<uint32_t>(std::max<uint32_t>(n, 1));
-    if (n)
-        k_instances<<<blocks(n, TB), TB, 0, st>>>(n, s.d_inst_src, d_w2o, s.n_geom, s.d_gflags, s.d_trav_root4,
-                                                  s.d_blas4, s.n_blas4, glo, ghi, s.d_mesh, s.d_toff,
-                                                  multi ? s.d_inst_env : nullptr, s.d_inst, ilo, ihi, iseg);
+    const bool small = most <= kTlasSmall;
+    const bool direct = small && n <= kTlasDirect;
+    if (n && !direct) KF_CHECK(hipMemcpyAsync(s.d_inst_src, s.h_stage, inst_bytes, hipMemcpyHostToDevice, st));
+    InstArgs A{};
+    A.src = direct ? (const kf_instance*)s.h_stage : s.d_inst_src;
+    A.n_geom = s.n_geom;
+    A.gflags = s.d_gflags;
+    A.root = s.d_trav_root4;
+    A.blas4 = s.d_blas4;
+    A.n_blas4 = s.n_blas4;
+    A.glo = s.d_glo;
+    A.ghi = s.d_ghi;
+    A.mesh = s.d_mesh;
+    A.toff = s.d_toff;
+    A.out = s.d_inst;
+    A.ilo = s.d_ilo;  // kept: the renderer culls instances per pixel tile with them
+    A.ihi = s.d_ihi;
     const uint32_t n_seg = multi ? s.n_env : 1u;
-    const uint32_t* seg_off = multi ? s.d_env_off : s.d_tlas_aux;
-    const uint32_t* node_off = multi ? s.d_env_node_off : s.d_tlas_aux + 2;
-    uint32_t* cnt = multi ? s.d_env_cnt : s.d_tlas_aux + 3;
-    if (!multi) k_tlas_aux<<<1, 1, 0, st>>>(n, s.d_tlas_aux);
-    uint32_t* order = dalloc<uint32_t>(std::max<uint32_t>(n, 1));
-    int* d_root = dalloc<int>(n_seg);
-    lbvh_build(n, ilo, ihi, iseg, n_seg, seg_off, node_off, s.d_tlas, order, d_root, false, st);
     // BVH2 nodes: n_e - 1 per environment of n_e >= 2 instances
     uint32_t n_tlas2 = 0;
     if (multi)
@@ -1268,17 +1452,40 @@ void build_tlas(Scene& s, const kf_instance* h_inst, uint32_t n) {
         s.tlas4_cap = std::max<uint32_t>(n_tlas2, 1);
         s.d_tlas4 = dalloc<Node4>(s.tlas4_cap);
     }
-    const uint32_t qcap = std::max<uint32_t>(n_tlas2, 1);
-    int2* qa = dalloc<int2>(qcap);
-    int2* qb = dalloc<int2>(qcap);
-    if (n_tlas2)
+    uint32_t* cnt = multi ? s.d_env_cnt : s.d_tlas_aux + 3;
+    if (small) {
+        const uint32_t* eo = multi ? s.d_env_off : nullptr;
+        const uint32_t* no = multi ? s.d_env_node_off : nullptr;
+        if (!n) {
+        } else if (most <= 64u) {
+            k_tlas_small<64><<<n_seg, 64, 0, st>>>(n, A, eo, no, s.d_tlas, s.d_tlas4, cnt, s.d_tlas_err);
+        } else if (most <= 256u) {
+            k_tlas_small<256><<<n_seg, 256, 0, st>>>(n, A, eo, no, s.d_tlas, s.d_tlas4, cnt, s.d_tlas_err);
+        } else {
+            k_tlas_small<kTlasSmall><<<n_seg, kTlasSmall, 0, st>>>(n, A, eo, no, s.d_tlas, s.d_tlas4, cnt, s.d_tlas_err);
+        }
+    } else {
+        const uint32_t* seg_off = multi ? s.d_env_off : s.d_tlas_aux;
+        const uint32_t* node_off = multi ? s.d_env_node_off : s.d_tlas_aux + 2;
+        uint32_t* iseg = dalloc<uint32_t>(n);
+        uint32_t* order = dalloc<uint32_t>(n);
+        int* d_root = dalloc<int>(n_seg);
+        int2* qa = dalloc<int2>(n_tlas2);
+        int2* qb = dalloc<int2>(n_tlas2);
+        k_instances<<<blocks(n, TB), TB, 0, st>>>(n, A, multi ? s.d_inst_env : nullptr, iseg);
+        if (!multi) k_tlas_aux<<<1, 1, 0, st>>>(n, s.d_tlas_aux);
+        lbvh_build(n, A.ilo, A.ihi, iseg, n_seg, seg_off, node_off, s.d_tlas, order, d_root, false, st);
         k_collapse_forest<<<n_seg, kTreeThreads, 0, st>>>(s.d_tlas, n_tlas2, seg_off, node_off, qa, qb, s.d_tlas4, 0u,
                                                           cnt, s.d_tlas_err);
+        dfree(iseg); dfree(order); dfree(d_root); dfree(qa); dfree(qb);
+    }
     KF_CHECK(hipGetLastError());
+    if (n) {
+        KF_CHECK(hipEventRecord(s.stage_ev, st));
+        s.stage_pending = true;
+    }
     s.tlas_root4 = roots[0];  // BVH4 and BVH2 roots coincide by construction
     s.n_tlas4 = n_tlas2 ? s.tlas4_cap : 0;  // index bound; the node count stays on the device
-    dfree(d_w2o); dfree(glo); dfree(ghi); dfree(iseg);
-    dfree(order); dfree(d_root); dfree(qa); dfree(qb);
 }
 
 // Geometry g's vertices were replaced on the device (same count, same
@@ -1288,19 +1495,26 @@ void refit_blas(Scene& s, uint32_t g) {
     const uint32_t TB = 256;
     const uint32_t n = s.h_toff[g + 1] - s.h_toff[g];
     if (n == 0) return;
-    float4* lo = dalloc<float4>(n);
-    float4* hi = dalloc<float4>(n);
+    // the slots' boxes and their pyramid, in a workspace that the scene keeps
+    const size_t need = 2 * (size_t)n * sizeof(float4) + pyramid_size(n) * sizeof(Box);
+    if (need > s.refit_cap) {
+        dfree(s.d_refit);
+        s.d_refit = nullptr;
+        s.refit_cap = 0;
+        s.d_refit = dalloc<uint8_t>(need);
+        s.refit_cap = need;
+    }
+    float4* lo = (float4*)s.d_refit;
+    float4* hi = lo + n;
     k_geom_slots<<<blocks(n, TB), TB, 0, st>>>(g, s.d_verts, s.d_idx, s.d_voff, s.d_toff, s.d_tri, lo, hi);
     if (n >= 2) {
-        const Pyramid P = build_pyramid(n, nullptr, lo, hi, st);
+        const Pyramid P = build_pyramid(n, nullptr, lo, hi, (Box*)(hi + n), st);
         k_geom_refit2<<<blocks(n - 1, TB), TB, 0, st>>>(g, s.d_toff, s.d_node_off, s.n_blas_nodes, P, s.d_blas);
         k_geom_refit4<<<blocks(n - 1, TB), TB, 0, st>>>(g, s.d_toff, s.d_node_off, s.d_blas_cnt, s.d_blas,
                                                        s.n_blas_nodes, s.d_tri, s.d_blas4);
-        dfree(P.at);
     }
+    blas_boxes(s);
     KF_CHECK(hipGetLastError());
-    dfree(lo);
-    dfree(hi);
 }
 
 }  // namespace kf

@@ -118,7 +118,7 @@ Scene::~Scene() {
     if (h_stage) (void)hipHostFree(h_stage);
     if (stage_ev) (void)hipEventDestroy(stage_ev);
     d_env_info = nullptr;  // points into d_tex_info, not an allocation of its own
-    release(d_inst_src); release(d_ilo); release(d_ihi); release(d_tex); release(d_tex_info); release(d_srgb);
+    release(d_inst_src); release(d_ilo); release(d_ihi); release(d_glo); release(d_ghi); release(d_refit); release(d_tex); release(d_tex_info); release(d_srgb);
 }
 
 // Environments of a batched scene: instance ranges, BVH2 / BVH4 node ranges
@@ -272,31 +272,7 @@ int kf_world_to_object(const float t[16], float out[12]) {
         set_error("kf_world_to_object: null argument");
         return -1;
     }
-    // m[r][c] = t[c*4 + r]; 3x3 inverse by cofactors in double; translation
-    // -M^-1 t; rounded to float (gl_WorldToObjectEXT).
-    double m[3][3], tr[3];
-    for (int r = 0; r < 3; ++r) {
-        for (int c = 0; c < 3; ++c) m[r][c] = t[c * 4 + r];
-        tr[r] = t[3 * 4 + r];
-    }
-    double c00 = m[1][1] * m[2][2] - m[1][2] * m[2][1];
-    double c01 = m[1][2] * m[2][0] - m[1][0] * m[2][2];
-    double c02 = m[1][0] * m[2][1] - m[1][1] * m[2][0];
-    double det = m[0][0] * c00 + m[0][1] * c01 + m[0][2] * c02;
-    double inv[3][3];
-    inv[0][0] = c00 / det;
-    inv[0][1] = (m[0][2] * m[2][1] - m[0][1] * m[2][2]) / det;
-    inv[0][2] = (m[0][1] * m[1][2] - m[0][2] * m[1][1]) / det;
-    inv[1][0] = c01 / det;
-    inv[1][1] = (m[0][0] * m[2][2] - m[0][2] * m[2][0]) / det;
-    inv[1][2] = (m[0][2] * m[1][0] - m[0][0] * m[1][2]) / det;
-    inv[2][0] = c02 / det;
-    inv[2][1] = (m[0][1] * m[2][0] - m[0][0] * m[2][1]) / det;
-    inv[2][2] = (m[0][0] * m[1][1] - m[0][1] * m[1][0]) / det;
-    for (int r = 0; r < 3; ++r) {
-        for (int c = 0; c < 3; ++c) out[r * 4 + c] = (float)inv[r][c];
-        out[r * 4 + 3] = (float)(-(inv[r][0] * tr[0] + inv[r][1] * tr[1] + inv[r][2] * tr[2]));
-    }
+    world_to_object(t, out);
     return 0;
 }
 

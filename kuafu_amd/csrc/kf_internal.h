@@ -37,6 +37,37 @@ inline uint32_t tea_host(uint32_t v0, uint32_t v1) {
     return v0;
 }
 
+// World -> object 3x4 (row-major) of a column-major transform, in double:
+// kf_world_to_object on the host, the instance records on the device (IEEE
+// operations in one order, so the same bits).
+__host__ __device__ inline void world_to_object(const float* t, float out[12]) {
+    // m[r][c] = t[c*4 + r]; 3x3 inverse by cofactors; translation -M^-1 t;
+    // rounded to float (gl_WorldToObjectEXT).
+    double m[3][3], tr[3];
+    for (int r = 0; r < 3; ++r) {
+        for (int c = 0; c < 3; ++c) m[r][c] = t[c * 4 + r];
+        tr[r] = t[3 * 4 + r];
+    }
+    double c00 = m[1][1] * m[2][2] - m[1][2] * m[2][1];
+    double c01 = m[1][2] * m[2][0] - m[1][0] * m[2][2];
+    double c02 = m[1][0] * m[2][1] - m[1][1] * m[2][0];
+    double det = m[0][0] * c00 + m[0][1] * c01 + m[0][2] * c02;
+    double inv[3][3];
+    inv[0][0] = c00 / det;
+    inv[0][1] = (m[0][2] * m[2][1] - m[0][1] * m[2][2]) / det;
+    inv[0][2] = (m[0][1] * m[1][2] - m[0][2] * m[1][1]) / det;
+    inv[1][0] = c01 / det;
+    inv[1][1] = (m[0][0] * m[2][2] - m[0][2] * m[2][0]) / det;
+    inv[1][2] = (m[0][2] * m[1][0] - m[0][0] * m[1][2]) / det;
+    inv[2][0] = c02 / det;
+    inv[2][1] = (m[0][1] * m[2][0] - m[0][0] * m[2][1]) / det;
+    inv[2][2] = (m[0][0] * m[1][1] - m[0][1] * m[1][0]) / det;
+    for (int r = 0; r < 3; ++r) {
+        for (int c = 0; c < 3; ++c) out[r * 4 + c] = (float)inv[r][c];
+        out[r * 4 + 3] = (float)(-(inv[r][0] * tr[0] + inv[r][1] * tr[1] + inv[r][2] * tr[2]));
+    }
+}
+
 // ------------------------------------------------------------------ BVH layout
 // BVH2 node, 64 B, both child boxes stored in the parent so one 64-B fetch
 // tests two children:
@@ -138,6 +169,8 @@ struct Scene {
     uint32_t* d_node_off = nullptr;          // h_node_off on the device
     uint32_t* d_blas_cnt = nullptr;          // 2 collapse counters per geometry: [2g] = next free BVH4 slot
     std::vector<kf_instance> h_inst;         // instances of the last TLAS build (for rebuilds after a refit)
+    uint8_t* d_refit = nullptr;              // workspace of refits (the largest geometry refitted so far)
+    size_t refit_cap = 0;
     uint8_t* h_vstage = nullptr;             // pinned staging of geometry vertex updates
     size_t vstage_cap = 0;
     hipEvent_t vstage_ev = nullptr;
@@ -170,6 +203,7 @@ struct Scene {
     Inst* d_inst = nullptr;
     kf_instance* d_inst_src = nullptr;
     float4 *d_ilo = nullptr, *d_ihi = nullptr;  // instance world boxes (the TLAS leaf boxes)
+    float4 *d_glo = nullptr, *d_ghi = nullptr;  // object-space box of each geometry's BLAS
     int tlas_root = kEmptyRef;
     // Batched environments: instances [h_env_off[e], h_env_off[e+1]) form
     // environment e, with its BVH2 nodes (and its BVH4 nodes, root first)

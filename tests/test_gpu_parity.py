@@ -85,6 +85,52 @@ def test_batch_sizes_give_the_same_hits(gpu, n):
         assert np.array_equal(hits["inst"], ref["inst"]) and np.array_equal(hits["prim"], ref["prim"])
 
 
+# Instances per TLAS around the block sizes of the one-launch build (64, 256,
+# 1024) and beyond it, created directly and by an update from another count.
+@pytest.mark.parametrize("n", [1, 2, 3, 63, 64, 65, 256, 257, 1024, 1025, 3000])
+def test_tlas_sizes(gpu, n):
+    rng = np.random.default_rng(n)
+    s = scenes.SceneData()
+    sv, si = scenes.uv_sphere(6, 4, 0.5)
+    one_v, one_t = scenes.quad(1.0)
+    s.add_geometry(sv, si, scenes.material())
+    s.add_geometry(one_v, one_t[:1], scenes.material())  # its BLAS root is a triangle
+    s.add_geometry(sv, si, scenes.material(), hidden=True)
+    for k in range(n):
+        pos = rng.uniform(-8, 8, 3) if k % 5 else (1.0, 2.0, 3.0)  # equal Morton codes too
+        s.add_instance(int(rng.choice(3, p=[0.8, 0.15, 0.05])),
+                       scenes.mat_from_rows(scenes.random_rotation(rng) * rng.uniform(0.3, 1.2), pos))
+    rays = np.zeros(600, abi.RAY_DTYPE)
+    rays["org"] = rng.uniform(-12, 12, (600, 3))
+    d = rng.uniform(-6, 6, (600, 3)) - rays["org"]
+    rays["dir"] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays["tmin"], rays["tmax"] = 0.001, 1e4
+    ref = oracle.Scene(s).trace_closest(rays)
+    gs = GpuScene(s)
+    few = scenes.SceneData()
+    few.__dict__.update(s.__dict__)
+    few.instances = s.instances[:max(1, n // 2)]
+    updated = GpuScene(few)
+    updated.update_instances(s.arrays()["inst"])
+    for g in (gs, updated):
+        hits = g.trace_closest(rays)
+        for f in ("inst", "prim", "t", "b1", "b2"):
+            hit = ref["inst"] != 0xFFFFFFFF if f in ("t", "b1", "b2") else slice(None)
+            assert np.array_equal(hits[f][hit], ref[f][hit]), f
+        nodes, roots = g.read_bvh4(1)
+        leaves, todo = [], [int(roots[0])] if n > 1 else []
+        while todo:
+            for c in nodes[todo.pop(), 24:28].copy().view(np.uint32):
+                if c == 0xFFFFFFFF:
+                    continue
+                if c >> 30 == 0:
+                    todo.append(int(c))
+                else:
+                    assert c >> 30 == 2
+                    leaves.append(int(c & 0x3FFFFFFF))
+        assert sorted(leaves) == (list(range(n)) if n > 1 else [])
+
+
 def test_blas_invariants(gpu):
     w = scenes.config1()
     gs = GpuScene(w.data)
