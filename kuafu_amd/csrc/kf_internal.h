@@ -267,7 +267,7 @@ struct Renderer {
     // wavefront state, sized for `cap` paths and `slots` NEE slots per path
     size_t cap = 0;
     uint32_t slots = 0;
-    float4 *ray_o = nullptr, *ray_d = nullptr, *thr = nullptr, *col = nullptr, *rw = nullptr, *em = nullptr;
+    float4 *ray_o = nullptr, *ray_d = nullptr, *thr = nullptr, *col = nullptr, *rw = nullptr;
     float4* hit = nullptr;
     uint32_t* hit_prim = nullptr;
     uint32_t* seed = nullptr;

@@ -32,18 +32,21 @@ namespace {
 constexpr int TB = 256;
 static_assert(TB == (int)kRingThreads, "traversal kernels index their LDS stack ring by a 256-thread block");
 
-// Device counters of one batch: per bounce b: [0] active paths, [1] shadow
-// rays, [2] next queue, [3] rays k_extend traces at bounce b.  Global, after
-// them: primary / extension / shadow rays, BVH4 node records / triangle tests
-// (closest-hit traversal), stack overflow, instance records, speculative
-// rays, TLAS node records (part of the node records), closest-hit rays
-// traced by k_tail (part of the extension rays).  Then, per bounce, the work
-// chunks of k_extend and of k_shadow (8 each, kChunkStride apart).
+// Device counters of one batch.  Per bounce b: active paths, shadow rays, rays
+// k_extend traces at bounce b, each on a line of its own (kChunkStride apart:
+// the appends of one launch go to different ones, and those to one line queue
+// up behind each other).  Global, after them: primary / extension / shadow
+// rays, BVH4 node records / triangle tests (closest-hit traversal), stack
+// overflow, instance records, speculative rays, TLAS node records (part of
+// the node records), closest-hit rays traced by k_tail (part of the extension
+// rays).  Then, per bounce, the work chunks of k_extend and of k_shadow (8
+// each, kChunkStride apart).
 constexpr int kMaxBounces = 64;
-constexpr int kCntPerBounce = 4;
+constexpr int kCntFields = 3;
+constexpr int kCntPerBounce = kCntFields * (int)kChunkStride;
+constexpr int kCntPaths = 0, kCntShadow = (int)kChunkStride, kCntExtQueue = 2 * (int)kChunkStride;
 // throughput and depth of a path before its first bounce
 __device__ constexpr float4 kPathStart = {1.0f, 1.0f, 1.0f, 0.0f};  // .w: depth 0 as uint bits
-constexpr int kCntExtQueue = 3;
 constexpr int kCntGlobal = kMaxBounces * kCntPerBounce;
 constexpr int kCntChunks = (kCntGlobal + 10 + (int)kChunkStride - 1) / (int)kChunkStride * (int)kChunkStride;
 constexpr int kChunksPerBounce = 2 * 8 * (int)kChunkStride;
@@ -81,48 +84,36 @@ KF_DEV void wave_add(unsigned long long* p, uint32_t v) {
     if ((threadIdx.x & 63) == 0 && v) atomicAdd(p, (unsigned long long)v);
 }
 
-// Wave-aggregated queue append; returns the slot index for lanes with pred.
-KF_DEV uint32_t wave_append(unsigned long long* counter, bool pred) {
-    unsigned long long m = __ballot(pred);
-    uint32_t lane = threadIdx.x & 63;
-    uint32_t leader = m ? (uint32_t)__ffsll((long long)m) - 1 : 0;
-    uint32_t base = 0;
-    if (m && lane == leader) base = (uint32_t)atomicAdd(counter, (unsigned long long)__popcll(m));
-    base = __shfl(base, leader);
-    unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    return base + (uint32_t)__popcll(m & lt);
-}
-
 // Block-aggregated queue append: one atomic per TB-thread block instead of
 // one per wave (appends to a single counter serialise in the memory system).
-// Every thread of the block must call it at the same point.
-KF_DEV uint32_t block_append(unsigned long long* counter, bool pred) {
-    __shared__ uint32_t s_wave[TB / 64];
-    __shared__ uint32_t s_base;
+// Every thread of the block must call it at the same point; turn alternates
+// 0, 1 between calls (the other turn's LDS may still be read).
+KF_DEV uint32_t block_append(unsigned long long* counter, bool pred, uint32_t turn) {
+    __shared__ uint32_t s_wave[2][TB / 64];
+    __shared__ uint32_t s_base[2];
     const unsigned long long m = __ballot(pred);
     const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    if (lane == 0) s_wave[w] = (uint32_t)__popcll(m);
+    if (lane == 0) s_wave[turn][w] = (uint32_t)__popcll(m);
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t tot = 0;
-        for (int i = 0; i < TB / 64; ++i) tot += s_wave[i];
-        s_base = tot ? (uint32_t)atomicAdd(counter, (unsigned long long)tot) : 0u;
+        for (int i = 0; i < TB / 64; ++i) tot += s_wave[turn][i];
+        s_base[turn] = tot ? (uint32_t)atomicAdd(counter, (unsigned long long)tot) : 0u;
     }
     __syncthreads();
-    uint32_t off = s_base;
-    for (uint32_t i = 0; i < w; ++i) off += s_wave[i];
-    const uint32_t r = off + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-    __syncthreads();  // s_wave and s_base are reused by the next call
-    return r;
+    uint32_t off = s_base[turn];
+    for (uint32_t i = 0; i < w; ++i) off += s_wave[turn][i];
+    return off + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
 }
 
 // Clears the counters of bounces 0 .. nb (their work chunks: of 0 .. nb - 1),
 // and the global ones on the frame's first batch.
 __global__ void k_zero(unsigned long long* c, int nb, int globals) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int small = globals ? kCntGlobal + 10 : (nb + 1) * kCntPerBounce;
-    if (i < small) c[i] = 0;
-    else if (i - small < nb * 16) c[kCntChunks + (i - small) * (int)kChunkStride] = 0;
+    const int paths = (nb + 1) * kCntFields, chunks = nb * 16;
+    if (i < paths) c[i * (int)kChunkStride] = 0;
+    else if (i < paths + chunks) c[kCntChunks + (i - paths) * (int)kChunkStride] = 0;
+    else if (globals && i < paths + chunks + 10) c[kCntGlobal + i - paths - chunks] = 0;
 }
 
 // ------------------------------------------------------------ camera-ray TLAS
@@ -441,8 +432,8 @@ __global__ __launch_bounds__(TB) void k_raygen(SceneView S, Frame F, const uint2
         }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        cnt[0 * kCntPerBounce + 0] = n;  // active paths at bounce 0
-        cnt[0 * kCntPerBounce + kCntExtQueue] = n;
+        cnt[kCntPaths] = n;  // active paths at bounce 0
+        cnt[kCntExtQueue] = n;
         atomicAdd(&cnt[kCntGlobal + 0], (unsigned long long)n);
     }
 }
@@ -569,47 +560,150 @@ KF_DEV bool light_eval(const SceneView& S, const DevLights* __restrict__ LT, int
 struct NeeCtx {
     ShadeCtx sh;
     uint32_t root;  // the path's TLAS root item
+    uint32_t rs;    // random state after the BSDF sample
     bool on;
 };
 
-// The deferred light loop for the paths of a block (rchit:457-460 order):
-// per light, the (ca, theta, cb, mode) record of the contribution and a
-// shadow ray, appended with one atomic per block.  Every thread of the
-// block calls it; threads without a shading point (nc.on false) append
-// nothing.
-KF_DEV void nee_deferred(const SceneView& S, const DevLights* __restrict__ LT, const NeeCtx& nc, uint32_t p,
-                         uint32_t K, float4* __restrict__ nee_a, float4* __restrict__ nee_b,
-                         float4* __restrict__ sh_o, float4* __restrict__ sh_d, uint32_t* __restrict__ sh_root,
-                         unsigned long long* __restrict__ shadow_ctr, uint32_t& n_shadow) {
-    const int nl = LT->n_slots;
-    uint32_t unused_rs = 0u;
-    for (int j = 0; j < nl; ++j) {
-        bool emit = false;
-        v3 Ld = splat(0.0f);
-        float maxd = 0.0f;
-        if (nc.on) {
-            const int kind = LT->kind[j], li = LT->index[j];
-            v3 lem;
-            const bool ok = light_eval<false>(S, LT, kind, li, nc.sh.worldPos, unused_rs, Ld, lem, maxd);
-            if (ok && dot(nc.sh.N, Ld) > 0.0f) {
-                v3 ca, cb;
-                float th;
-                int mode;
-                direct_split(nc.sh, Ld, lem, ca, cb, th, mode);
-                const size_t slot = (size_t)p * K + j;
-                nee_a[slot] = f4(ca, th);
-                nee_b[slot] = f4(cb, __int_as_float(mode | (kind << 4)));
-                emit = true;
-            }
-        }
-        const uint32_t at = block_append(shadow_ctr, emit);
-        if (emit) {
-            sh_o[at] = f4(nc.sh.worldPos, __uint_as_float((uint32_t)((size_t)p * K + j)));
-            sh_d[at] = f4(Ld, maxd);
-            if (S.n_env > 1) sh_root[at] = nc.root;
-            n_shadow++;
-        }
+// One light's contribution (rchit:103-171) is a choice between two colours
+// by a random number that is drawn only when the light is visible, so at the
+// path's v-th draw: v is known to be at most the number of lights before.
+// For the first kMaxPreLights lights the choice of every possible draw is
+// made here, from the path's random state, and k_connect only counts draws;
+// the record is then one colour unless the choice depends on the count.
+//   nee_a = (colour, bits): 1:0 the light's kind, 2 it draws, 3 two colours
+//           (nee_b holds the second), 8 + v the first one at draw v
+// More lights: nee_a = (ca, theta), nee_b = (cb, mode | kind << 4).
+constexpr uint32_t kMaxPreLights = 16;
+KF_DEV void nee_record(const ShadeCtx& sh, v3 Ld, v3 lem, int kind, uint32_t j, uint32_t K, uint32_t rs, size_t slot,
+                       float4* __restrict__ nee_a, float4* __restrict__ nee_b) {
+    v3 ca, cb;
+    float th;
+    int mode;
+    direct_split(sh, Ld, lem, ca, cb, th, mode);
+    if (K > kMaxPreLights) {
+        nee_a[slot] = f4(ca, th);
+        nee_b[slot] = f4(cb, __int_as_float(mode | (kind << 4)));
+        return;
     }
+    uint32_t pick = 0u;
+    if (mode != 0)
+#pragma unroll 1
+        for (uint32_t v = 0; v <= j; ++v) {
+            const float u = rnd(rs);
+            pick |= (mode == 1 ? (u <= th) : (u < th)) ? 1u << v : 0u;
+        }
+    const bool two = pick != 0u && pick != (2u << j) - 1u;
+    const uint32_t bits = (uint32_t)kind | (mode != 0 ? 4u : 0u) | (two ? 8u : 0u) | (pick << 8);
+    nee_a[slot] = f4(pick ? ca : cb, __uint_as_float(bits));
+    if (two) nee_b[slot] = f4(cb, 0.0f);
+}
+// The contribution of the visible light of a slot; draws counts the path's
+// draws of this bounce.
+KF_DEV v3 nee_resolve(const float4* __restrict__ nee_a, const float4* __restrict__ nee_b, size_t slot, uint32_t K,
+                      uint32_t& rs, uint32_t& draws, int& kind) {
+    const float4 a = nee_a[slot];
+    if (K > kMaxPreLights) {
+        const float4 b = nee_b[slot];
+        const int mb = __float_as_int(b.w);
+        kind = mb >> 4;
+        return direct_resolve(xyz(a), xyz(b), a.w, mb & 15, rs);
+    }
+    const uint32_t bits = __float_as_uint(a.w);
+    kind = (int)(bits & 3u);
+    v3 c = xyz(a);
+    if ((bits & 8u) && !((bits >> (8u + draws)) & 1u)) c = xyz(nee_b[slot]);
+    if (bits & 4u) {
+        (void)rnd(rs);
+        ++draws;
+    }
+    return c;
+}
+
+// The deferred light loop for the paths of a block (rchit:457-460 order): per
+// light the record of its contribution and a shadow ray, and the block's
+// appends to the shadow-ray queue and to the queue of the paths traced at the
+// next bounce (ext).  Every thread of the block calls it; threads without a
+// shading point (nc.on false) have no shadow rays.
+// The rays of the last kNeeGroup lights wait in LDS for their places, so that
+// they and the paths take one pair of barriers and one trip to the counters,
+// the two queues' atomics side by side: with an append per light and one for
+// the paths a block waited for two or three trips one after another
+// (128 environments of 512x512, 2 lights: k_shade 2.60 -> 1.81 ms per launch with the
+// shorter records).  Lights before those take an append each; a loop over
+// groups around the light loop spills 80 registers.
+constexpr int kNeeGroup = 4;
+KF_DEV uint32_t nee_deferred(const SceneView& S, const DevLights* __restrict__ LT, const NeeCtx& nc, uint32_t p,
+                             uint32_t K, bool ext, float4* __restrict__ nee_a, float4* __restrict__ nee_b,
+                             float4* __restrict__ sh_o, float4* __restrict__ sh_d, uint32_t* __restrict__ sh_root,
+                             unsigned long long* __restrict__ shadow_ctr, unsigned long long* __restrict__ ext_ctr,
+                             uint32_t& n_shadow, uint32_t& turn) {
+    __shared__ float4 ray[kNeeGroup][TB];  // (Ld, maxd) of the group's lights
+    __shared__ uint32_t s_wave[2][2][TB / 64];
+    __shared__ uint32_t s_base[2][2];
+    const int nl = LT->n_slots;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    uint32_t unused_rs = 0u;
+    auto light = [&](int j, float4& r) __attribute__((always_inline)) {
+        if (!nc.on) return false;
+        const int kind = LT->kind[j], li = LT->index[j];
+        v3 lem, Ld;
+        float maxd;
+        if (!light_eval<false>(S, LT, kind, li, nc.sh.worldPos, unused_rs, Ld, lem, maxd)) return false;
+        if (!(dot(nc.sh.N, Ld) > 0.0f)) return false;
+        nee_record(nc.sh, Ld, lem, kind, (uint32_t)j, K, nc.rs, (size_t)p * K + j, nee_a, nee_b);
+        r = f4(Ld, maxd);
+        return true;
+    };
+    auto put = [&](uint32_t at, int j, float4 r) __attribute__((always_inline)) {
+        sh_o[at] = f4(nc.sh.worldPos, __uint_as_float((uint32_t)((size_t)p * K + j)));
+        sh_d[at] = r;
+        if (S.n_env > 1) sh_root[at] = nc.root;
+        n_shadow++;
+    };
+    const int j0 = max(nl - kNeeGroup, 0);
+#pragma unroll 1
+    for (int j = 0; j < j0; ++j) {
+        float4 r = make_float4(0.f, 0.f, 0.f, 0.f);
+        const bool emit = light(j, r);
+        const uint32_t at = block_append(shadow_ctr, emit, turn);
+        turn ^= 1u;
+        if (emit) put(at, j, r);
+    }
+    uint32_t emits = 0u, before = 0u, total = 0u;  // this lane's rays; its wave's before and in all
+    const unsigned long long lt = (1ull << lane) - 1ull;
+#pragma unroll 1
+    for (int j = j0; j < nl; ++j) {
+        float4 r;
+        const bool emit = light(j, r);
+        if (emit) ray[j - j0][threadIdx.x] = r;
+        const unsigned long long m = __ballot(emit);
+        before += (uint32_t)__popcll(m & lt);
+        total += (uint32_t)__popcll(m);
+        emits |= emit ? 1u << (j - j0) : 0u;
+    }
+    const unsigned long long me = __ballot(ext);
+    if (lane == 0u) {
+        s_wave[turn][0][w] = total;
+        s_wave[turn][1][w] = (uint32_t)__popcll(me);
+    }
+    __syncthreads();
+    if (lane == 0u && w < 2u) {  // wave 0: the shadow rays, wave 1: the paths
+        uint32_t sum = 0;
+        for (int i = 0; i < TB / 64; ++i) sum += s_wave[turn][w][i];
+        s_base[turn][w] = sum ? (uint32_t)atomicAdd(w ? ext_ctr : shadow_ctr, (unsigned long long)sum) : 0u;
+    }
+    __syncthreads();
+    uint32_t at = s_base[turn][0] + before;
+    uint32_t ext_at = s_base[turn][1] + (uint32_t)__popcll(me & lt);
+    for (uint32_t i = 0; i < w; ++i) {
+        at += s_wave[turn][0][i];
+        ext_at += s_wave[turn][1][i];
+    }
+    turn ^= 1u;
+#pragma unroll 1
+    for (int j = j0; j < nl; ++j)
+        if (emits >> (j - j0) & 1u) put(at++, j, ray[j - j0][threadIdx.x]);
+    return ext_at;
 }
 
 // The per-path inputs of shading (throughput, hit, ray, random state),
@@ -639,7 +733,7 @@ KF_DEV ShadeIn shade_in(uint32_t p, float4 t4, const float4* __restrict__ hit, c
 template <bool NEE_INLINE>
 KF_DEV bool shade_path(const SceneView& S, const Frame& F, const DevLights* __restrict__ LT, int bounce, uint32_t p,
                        const ShadeIn& in, bool aov, float4* __restrict__ ray_o, float4* __restrict__ ray_d,
-                       float4* __restrict__ rw, float4* __restrict__ em, uint32_t* __restrict__ seed, float4* __restrict__ nee_a,
+                       float4* __restrict__ rw, uint32_t* __restrict__ seed, float4* __restrict__ nee_a,
                        float4* __restrict__ nee_b, uint8_t* __restrict__ vis, float4* __restrict__ sh_o,
                        float4* __restrict__ sh_d, uint32_t* __restrict__ sh_root, float4* __restrict__ albedo_out,
                        float4* __restrict__ normal_out, unsigned long long* __restrict__ cnt, uint32_t& n_shadow,
@@ -656,16 +750,14 @@ KF_DEV bool shade_path(const SceneView& S, const Frame& F, const DevLights* __re
     const uint32_t root = bounce == 0 ? env_root_item(S, (p % F.WH) / F.WHe) : __float_as_uint(rd.w);
     uint32_t rs = in.rs;
     uint32_t inst = __float_as_uint(h.w);
-    for (uint32_t j = 0; j < K; ++j) vis[(size_t)p * K + j] = 0;
     if (inst == ~0u) {
         // miss (rmiss:12-31)
         v3 e = miss_emission(S, F.pc, rdir);
-        em[p] = f4(e, __uint_as_float(1u));
+        rw[p] = f4(e, __uint_as_float(1u));
         if (aov) {
             albedo_out[p] = make_float4(0.f, 0.f, 0.f, 1.f);
             normal_out[p] = make_float4(0.f, 0.f, 0.f, 1.f);
         }
-        if (NEE_INLINE) nee_a[(size_t)p * K] = make_float4(0.f, 0.f, 0.f, 0.f);
     } else {
         uint32_t hp = in.hp;
         uint32_t prim = hp & 0x7fffffffu;
@@ -709,12 +801,11 @@ KF_DEV bool shade_path(const SceneView& S, const Frame& F, const DevLights* __re
         }
         v3 emission = mk(m.emission[0], m.emission[1], m.emission[2]) * m.emission[3];
         if (!all_zero(emission)) {
-            em[p] = f4(emission, __uint_as_float(1u));
+            rw[p] = f4(emission, __uint_as_float(1u));
             if (aov) {
                 albedo_out[p] = make_float4(0.f, 0.f, 0.f, 1.f);
                 normal_out[p] = make_float4(0.f, 0.f, 0.f, 1.f);
             }
-            if (NEE_INLINE) nee_a[(size_t)p * K] = make_float4(0.f, 0.f, 0.f, 0.f);
         } else {
             auto tex = [&](int id) -> float4 {
                 return tex_sample(S, S.tex_data, S.tex_info[id], uvx, uvy, true);
@@ -797,8 +888,10 @@ KF_DEV bool shade_path(const SceneView& S, const Frame& F, const DevLights* __re
             // with the whole block (nee_deferred).
             v3 sum_d = splat(0.0f), sum_p = splat(0.0f), sum_a = splat(0.0f);
             if (!NEE_INLINE) {
+                for (uint32_t j = 0; j < K; ++j) vis[(size_t)p * K + j] = 0;
                 nc.sh = sh;
                 nc.root = root;
+                nc.rs = rs;
                 nc.on = true;
             }
             const int nl = NEE_INLINE ? LT->n_slots : 0;
@@ -829,8 +922,7 @@ KF_DEV bool shade_path(const SceneView& S, const Frame& F, const DevLights* __re
             if (NEE_INLINE) nee_a[(size_t)p * K] = f4((sum_d + sum_p) + sum_a, 0.0f);
             ray_o[p] = f4(worldPos, 0.0f);
             ray_d[p] = f4(L, __uint_as_float(root));
-            em[p] = make_float4(0.f, 0.f, 0.f, __uint_as_float(0u));
-            rw[p] = f4(weight, 0.0f);
+            rw[p] = f4(weight, __uint_as_float(0u));
             ext = !all_zero(xyz(t4) * weight) && depth + 1u <= F.pc.path_depth;  // as in k_connect
             if (aov) {
                 albedo_out[p] = f4(base, 1.0f);
@@ -852,17 +944,18 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(NEE_INLINE ?
                                               const uint32_t* __restrict__ queue, float4* __restrict__ ray_o,
                                               float4* __restrict__ ray_d, const float4* __restrict__ thr,
                                               const float4* __restrict__ hit, const uint32_t* __restrict__ hit_prim,
-                                              float4* __restrict__ rw, float4* __restrict__ em,
+                                              float4* __restrict__ rw,
                                               uint32_t* __restrict__ seed, float4* __restrict__ nee_a,
                                               float4* __restrict__ nee_b, uint8_t* __restrict__ vis,
                                               float4* __restrict__ sh_o, float4* __restrict__ sh_d,
                                               uint32_t* __restrict__ sh_root, float4* __restrict__ albedo_out,
                                               float4* __restrict__ normal_out,
                                               uint32_t* __restrict__ ext_queue, unsigned long long* __restrict__ cnt) {
-    const uint32_t n = (uint32_t)min(cnt[bounce * kCntPerBounce + 0], (unsigned long long)(F.WH * F.nsamp));
+    const uint32_t n = (uint32_t)min(cnt[bounce * kCntPerBounce + kCntPaths], (unsigned long long)(F.WH * F.nsamp));
     const uint32_t stride = gridDim.x * blockDim.x, tid = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t iters = (n + stride - 1) / stride;
     uint32_t n_shadow = 0, ovf = 0;  // shadow rays of this thread
+    uint32_t turn = 0;
     // A software pipeline over the thread's paths: the queue entry two paths
     // ahead and the inputs of the next path are fetched before this path is
     // shaded, so that their memory round trips overlap its shading.
@@ -888,12 +981,17 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(NEE_INLINE ?
         NeeCtx nc;
         nc.on = false;
         if (active)
-            ext = shade_path<NEE_INLINE>(S, F, LT, bounce, p, in, aov, ray_o, ray_d, rw, em, seed, nee_a, nee_b, vis,
+            ext = shade_path<NEE_INLINE>(S, F, LT, bounce, p, in, aov, ray_o, ray_d, rw, seed, nee_a, nee_b, vis,
                                          sh_o, sh_d, sh_root, albedo_out, normal_out, cnt, n_shadow, ovf, nc);
-        if (!NEE_INLINE)
-            nee_deferred(S, LT, nc, p, F.slots, nee_a, nee_b, sh_o, sh_d, sh_root, &cnt[bounce * kCntPerBounce + 1],
-                         n_shadow);
-        const uint32_t at = block_append(&cnt[(bounce + 1) * kCntPerBounce + kCntExtQueue], ext);
+        unsigned long long* ext_ctr = &cnt[(bounce + 1) * kCntPerBounce + kCntExtQueue];
+        uint32_t at;
+        if (NEE_INLINE) {
+            at = block_append(ext_ctr, ext, turn);
+            turn ^= 1u;
+        } else {
+            at = nee_deferred(S, LT, nc, p, F.slots, ext, nee_a, nee_b, sh_o, sh_d, sh_root,
+                              &cnt[bounce * kCntPerBounce + kCntShadow], ext_ctr, n_shadow, turn);
+        }
         if (ext) ext_queue[at] = p;
         active = active1;
         p = p1;
@@ -909,7 +1007,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_num_vgpr(48))) void k_sha
                                                const float4* __restrict__ sh_d, const uint32_t* __restrict__ sh_root,
                                                uint8_t* __restrict__ vis,
                                                unsigned long long* __restrict__ cnt, uint32_t refill, uint32_t grab) {
-    const uint32_t n = (uint32_t)min(cnt[bounce * kCntPerBounce + 1], (unsigned long long)cap);
+    const uint32_t n = (uint32_t)min(cnt[bounce * kCntPerBounce + kCntShadow], (unsigned long long)cap);
     const uint32_t root0 = env_root_item(S, 0u);
     uint32_t ovf = 0;
     TCount tot{0, 0, 0, 0};
@@ -936,19 +1034,19 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_num_vgpr(48))) void k_sha
 // whether the path continues; a finished path writes its radiance to out.
 template <bool NEE_INLINE>
 KF_DEV bool connect_path(const Frame& F, int bounce, uint32_t p, float4* __restrict__ thr, float4* __restrict__ col,
-                         const float4* __restrict__ rw, const float4* __restrict__ em, uint32_t* __restrict__ seed,
+                         const float4* __restrict__ rw, uint32_t* __restrict__ seed,
                          const float4* __restrict__ nee_a, const float4* __restrict__ nee_b,
                          const uint8_t* __restrict__ vis, float4* __restrict__ out) {
     const uint32_t K = F.slots;
     const uint32_t maxDepth = F.pc.path_depth;
     bool cont = false;
-    const bool first = bounce == 0;  // the path's state is kPathStart, colour 0, weight 0
+    const bool first = bounce == 0;  // the path's state is kPathStart, colour 0
     float4 t4 = first ? kPathStart : thr[p];
     v3 weight = xyz(t4);
     uint32_t depth = __float_as_uint(t4.w);
     v3 color = first ? splat(0.0f) : xyz(col[p]);
-    float4 e4 = em[p];
-    bool term = __float_as_uint(e4.w) != 0u;
+    const float4 r4 = rw[p];  // BSDF weight, or the emission that ends the path
+    const bool term = __float_as_uint(r4.w) != 0u;
     uint32_t rs = seed[p];
     v3 shadow = splat(0.0f);
     if (!term) {
@@ -956,13 +1054,12 @@ KF_DEV bool connect_path(const Frame& F, int bounce, uint32_t p, float4* __restr
             shadow = xyz(nee_a[(size_t)p * K]);
         } else {
             v3 sd = splat(0.0f), sp = splat(0.0f), sa = splat(0.0f);
+            uint32_t draws = 0;
             for (uint32_t j = 0; j < K; ++j) {
                 size_t slot = (size_t)p * K + j;
                 if (!vis[slot]) continue;
-                float4 a = nee_a[slot], b = nee_b[slot];
-                int mb = __float_as_int(b.w);
-                v3 cj = direct_resolve(xyz(a), xyz(b), a.w, mb & 15, rs);
-                int kind = mb >> 4;
+                int kind;
+                const v3 cj = nee_resolve(nee_a, nee_b, slot, K, rs, draws, kind);
                 if (kind == 0) sd = sd + cj;
                 else if (kind == 1) sp = sp + cj;
                 else sa = sa + cj;
@@ -970,11 +1067,9 @@ KF_DEV bool connect_path(const Frame& F, int bounce, uint32_t p, float4* __restr
             shadow = (sd + sp) + sa;
         }
     }
-    // rgen:109-138
-    color = color + xyz(e4) * weight;
-    // k_shade wrote rw for every path it continues; a path it ended at
-    // bounce 0 still has the initial weight 0
-    weight = weight * ((first && term) ? splat(0.0f) : xyz(rw[p]));
+    // rgen:109-138; without emission the product still adds 0 x weight
+    color = color + (term ? xyz(r4) : splat(0.0f)) * weight;
+    weight = weight * (term ? splat(first ? 0.0f : 1.0f) : xyz(r4));
     color = color + shadow * weight;
     uint32_t d2 = term ? maxDepth + 1 : depth;
     cont = true;
@@ -1001,12 +1096,11 @@ KF_DEV bool connect_path(const Frame& F, int bounce, uint32_t p, float4* __restr
 template <bool NEE_INLINE>
 __global__ __launch_bounds__(TB) void k_connect(Frame F, int bounce, const uint32_t* __restrict__ queue,
                                                 uint32_t* __restrict__ next, float4* __restrict__ thr,
-                                                float4* __restrict__ col, const float4* __restrict__ rw,
-                                                const float4* __restrict__ em, uint32_t* __restrict__ seed,
+                                                float4* __restrict__ col, const float4* __restrict__ rw, uint32_t* __restrict__ seed,
                                                 const float4* __restrict__ nee_a, const float4* __restrict__ nee_b,
                                                 const uint8_t* __restrict__ vis, float4* __restrict__ out,
                                                 unsigned long long* __restrict__ cnt) {
-    uint32_t n = (uint32_t)min(cnt[bounce * kCntPerBounce + 0], (unsigned long long)(F.WH * F.nsamp));
+    uint32_t n = (uint32_t)min(cnt[bounce * kCntPerBounce + kCntPaths], (unsigned long long)(F.WH * F.nsamp));
     uint32_t stride = gridDim.x * blockDim.x;
     uint32_t iters = (n + stride - 1) / stride;
     for (uint32_t it = 0; it < iters; ++it) {
@@ -1015,9 +1109,9 @@ __global__ __launch_bounds__(TB) void k_connect(Frame F, int bounce, const uint3
         uint32_t p = 0;
         if (q < n) {
             p = queue[q];
-            cont = connect_path<NEE_INLINE>(F, bounce, p, thr, col, rw, em, seed, nee_a, nee_b, vis, out);
+            cont = connect_path<NEE_INLINE>(F, bounce, p, thr, col, rw, seed, nee_a, nee_b, vis, out);
         }
-        uint32_t at = block_append(&cnt[bounce * kCntPerBounce + 2], cont);
+        uint32_t at = block_append(&cnt[(bounce + 1) * kCntPerBounce + kCntPaths], cont, it & 1u);
         if (cont) next[at] = p;
     }
 }
@@ -1033,12 +1127,11 @@ __global__ __launch_bounds__(TB) void k_tail(SceneView S, Frame F, const DevLigh
                                              const uint32_t* __restrict__ queue, float4* __restrict__ ray_o,
                                              float4* __restrict__ ray_d, float4* __restrict__ thr,
                                              float4* __restrict__ col, float4* __restrict__ hit,
-                                             uint32_t* __restrict__ hit_prim, float4* __restrict__ rw,
-                                             float4* __restrict__ em, uint32_t* __restrict__ seed,
+                                             uint32_t* __restrict__ hit_prim, float4* __restrict__ rw, uint32_t* __restrict__ seed,
                                              float4* __restrict__ nee_a, float4* __restrict__ nee_b,
                                              uint8_t* __restrict__ vis, float4* __restrict__ out,
                                              unsigned long long* __restrict__ cnt, uint32_t min_n) {
-    const uint32_t n = (uint32_t)min(cnt[b0 * kCntPerBounce + 0], (unsigned long long)(F.WH * F.nsamp));
+    const uint32_t n = (uint32_t)min(cnt[b0 * kCntPerBounce + kCntPaths], (unsigned long long)(F.WH * F.nsamp));
     if (n <= min_n) return;  // k_tail2 takes these paths
     const uint32_t S0 = F.fv->S0;
     uint32_t n_shadow = 0, n_ext = 0, n_traced = 0, ovf = 0;
@@ -1058,9 +1151,9 @@ __global__ __launch_bounds__(TB) void k_tail(SceneView S, Frame F, const DevLigh
             hit_prim[p] = h.prim | (h.back << 31);
             NeeCtx nc;
             shade_path<true>(S, F, LT, b, p, shade_in(p, thr[p], hit, hit_prim, ray_o, ray_d, seed), false, ray_o,
-                             ray_d, rw, em, seed, nee_a, nee_b, vis, nullptr, nullptr, nullptr, nullptr, nullptr, cnt,
+                             ray_d, rw, seed, nee_a, nee_b, vis, nullptr, nullptr, nullptr, nullptr, nullptr, cnt,
                              n_shadow, ovf, nc);
-            if (!connect_path<true>(F, b, p, thr, col, rw, em, seed, nee_a, nee_b, vis, out)) break;
+            if (!connect_path<true>(F, b, p, thr, col, rw, seed, nee_a, nee_b, vis, out)) break;
             ++n_ext;  // traced at the next bounce
         }
     }
@@ -1089,12 +1182,7 @@ KF_DEV bool nee_slots(const SceneView& S, const DevLights* __restrict__ LT, cons
             v3 lem;
             const bool ok = light_eval<false>(S, LT, kind, li, nc.sh.worldPos, unused_rs, Ld, lem, maxd);
             if (ok && dot(nc.sh.N, Ld) > 0.0f) {
-                v3 ca, cb;
-                float th;
-                int mode;
-                direct_split(nc.sh, Ld, lem, ca, cb, th, mode);
-                nee_a[slot] = f4(ca, th);
-                nee_b[slot] = f4(cb, __int_as_float(mode | (kind << 4)));
+                nee_record(nc.sh, Ld, lem, kind, j, K, nc.rs, slot, nee_a, nee_b);
                 emit = true;
             }
         }
@@ -1122,13 +1210,12 @@ __global__ __launch_bounds__(TB) void k_tail2(SceneView S, Frame F, const DevLig
                                               const uint32_t* __restrict__ queue, float4* __restrict__ ray_o,
                                               float4* __restrict__ ray_d, float4* __restrict__ thr,
                                               float4* __restrict__ col, float4* __restrict__ hit,
-                                              uint32_t* __restrict__ hit_prim, float4* __restrict__ rw,
-                                              float4* __restrict__ em, uint32_t* __restrict__ seed,
+                                              uint32_t* __restrict__ hit_prim, float4* __restrict__ rw, uint32_t* __restrict__ seed,
                                               float4* __restrict__ nee_a, float4* __restrict__ nee_b,
                                               uint8_t* __restrict__ vis, float4* __restrict__ sh_o,
                                               float4* __restrict__ sh_d, float4* __restrict__ out,
                                               unsigned long long* __restrict__ cnt, uint32_t max_n) {
-    const uint32_t n = (uint32_t)min(cnt[b0 * kCntPerBounce + 0], (unsigned long long)(F.WH * F.nsamp));
+    const uint32_t n = (uint32_t)min(cnt[b0 * kCntPerBounce + kCntPaths], (unsigned long long)(F.WH * F.nsamp));
     if (n > max_n) return;  // k_tail takes these paths
     const uint32_t S0 = F.fv->S0;
     const uint32_t K = F.slots;
@@ -1220,7 +1307,7 @@ __global__ __launch_bounds__(TB) void k_tail2(SceneView S, Frame F, const DevLig
             if (!second) {
                 bool done = false;
                 if (b > b0) {  // bounce b - 1: lights in order, path update, Russian roulette
-                    if (connect_path<false>(F, b - 1, p, thr, col, rw, em, seed, nee_a, nee_b, vis, out)) {
+                    if (connect_path<false>(F, b - 1, p, thr, col, rw, seed, nee_a, nee_b, vis, out)) {
                         ++n_ext;
                     } else {
                         done = true;
@@ -1232,7 +1319,7 @@ __global__ __launch_bounds__(TB) void k_tail2(SceneView S, Frame F, const DevLig
                     nc.on = false;
                     const bool ext = shade_path<false>(S, F, LT, b, p,
                                                        shade_in(p, thr[p], hit, hit_prim, ray_o, ray_d, seed), false,
-                                                       ray_o, ray_d, rw, em, seed, nee_a, nee_b, vis, nullptr,
+                                                       ray_o, ray_d, rw, seed, nee_a, nee_b, vis, nullptr,
                                                        nullptr, nullptr, nullptr, nullptr, cnt, unused, ovf, nc);
                     const bool sh = nee_slots(S, LT, nc, p, K, nee_a, nee_b, sh_o, sh_d);
                     flags = 1 | (ext ? 2 : 0) | (sh ? 4 : 0);
@@ -1253,19 +1340,19 @@ __global__ __launch_bounds__(TB) void k_tail2(SceneView S, Frame F, const DevLig
     if (ovf) atomicAdd(&cnt[kCntGlobal + 5], 1ull);
 }
 
-__global__ void k_next_count(int bounce, unsigned long long* cnt) {
-    unsigned long long nx = cnt[bounce * kCntPerBounce + 2];
-    cnt[(bounce + 1) * kCntPerBounce + 0] = nx;
-    cnt[kCntGlobal + 1] += nx;
-    // next-bounce rays traced for paths Russian roulette then ended
-    cnt[kCntGlobal + 7] += cnt[(bounce + 1) * kCntPerBounce + kCntExtQueue] - nx;
-}
-
 // Sum the batch's samples into acc in sample order (rgen:140), then on the
 // last batch: average, running mean over frames (rgen:153-163).
 __global__ __launch_bounds__(TB) void k_resolve(Frame F, const float4* __restrict__ out, float4* __restrict__ acc,
-                                                float4* __restrict__ rgba, float* __restrict__ keep, int last) {
+                                                float4* __restrict__ rgba, float* __restrict__ keep, int last,
+                                                int b_tail, unsigned long long* __restrict__ cnt) {
     uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
+    if (px == 0) {  // the batch's extension rays, and those of paths Russian roulette then ended
+        for (int b = 1; b <= b_tail; ++b) {
+            const unsigned long long n = cnt[b * kCntPerBounce + kCntPaths];
+            cnt[kCntGlobal + 1] += n;
+            cnt[kCntGlobal + 7] += cnt[b * kCntPerBounce + kCntExtQueue] - n;
+        }
+    }
     if (px >= F.WH) return;
     v3 c = F.s0 == 0 ? splat(0.0f) : xyz(acc[px]);
     for (uint32_t i = 0; i < F.nsamp; ++i) {
@@ -1332,7 +1419,7 @@ Renderer::~Renderer() {
     for (auto e : ev) (void)hipEventDestroy(e);
     for (auto e : sync_ev) (void)hipEventDestroy(e);
     if (h_totals) (void)hipHostFree(h_totals);
-    void* ptrs[] = {d_rgba, d_albedo, d_normal, d_bgra, ray_o, ray_d, thr, col, rw, em, hit, hit_prim, seed,
+    void* ptrs[] = {d_rgba, d_albedo, d_normal, d_bgra, ray_o, ray_d, thr, col, rw, hit, hit_prim, seed,
                     queue_a, queue_b, queue_e, sh_o, sh_d, sh_root, nee_a, nee_b, vis, samples, counters, d_lights,
                     d_jump, d_acc, d_out, d_cams, d_fv, d_ftlas, d_tile_root};
     for (void* p : ptrs)
@@ -1351,7 +1438,7 @@ bool Renderer::ensure(size_t paths, uint32_t nslots, uint32_t spp) {
         };
         const size_t f4 = want * sizeof(float4), u4 = want * sizeof(uint32_t), s4 = wslots * f4;
         const Buf bufs[] = {{(void**)&ray_o, f4},   {(void**)&ray_d, f4},   {(void**)&thr, f4},
-                            {(void**)&col, f4},     {(void**)&rw, f4},      {(void**)&em, f4},
+                            {(void**)&col, f4},     {(void**)&rw, f4},
                             {(void**)&hit, f4},     {(void**)&hit_prim, u4}, {(void**)&seed, u4},
                             {(void**)&queue_a, u4}, {(void**)&queue_b, u4}, {(void**)&queue_e, u4},
                             {(void**)&sh_o, s4},    {(void**)&sh_d, s4},    {(void**)&sh_root, wslots * u4},
@@ -1638,7 +1725,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
         F.s0 = s0;
         F.nsamp = std::min(spb, pc->spp - s0);
         const uint32_t B = WH * F.nsamp;
-        const int nz = (s0 == 0 ? kCntGlobal + 10 : (int)(nb + 1) * kCntPerBounce) + (int)nb * 16;
+        const int nz = (int)(nb + 1) * kCntFields + (int)nb * 16 + 10;
         k_zero<<<(nz + TB - 1) / TB, TB, 0, st>>>(r->counters, (int)nb, s0 == 0 ? 1 : 0);
         if (timed) KF_CHECK(hipEventRecord(r->ev[0], st));
         if (tiles && s0 == 0)
@@ -1680,21 +1767,21 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
                 const uint32_t pair_max = (inline_nee || !r->tune_pairs) ? 0u : grid * TB / 8u;
                 if (!inline_nee)
                     k_tail2<<<grid, TB, 0, st>>>(S, F, d_lights, (int)b, qa, r->ray_o, r->ray_d, r->thr, r->col,
-                                                 r->hit, r->hit_prim, r->rw, r->em, r->seed, r->nee_a, r->nee_b,
+                                                 r->hit, r->hit_prim, r->rw, r->seed, r->nee_a, r->nee_b,
                                                  r->vis, r->sh_o, r->sh_d, d_out, r->counters, pair_max);
                 k_tail<<<grid, TB, 0, st>>>(S, F, d_lights, (int)b, qa, r->ray_o, r->ray_d, r->thr, r->col, r->hit,
-                                            r->hit_prim, r->rw, r->em, r->seed, r->nee_a, r->nee_b, r->vis, d_out,
+                                            r->hit_prim, r->rw, r->seed, r->nee_a, r->nee_b, r->vis, d_out,
                                             r->counters, pair_max);
                 break;
             }
             if (inline_nee)
                 k_shade<true><<<grid, TB, 0, st>>>(S, F, d_lights, (int)b, qa, r->ray_o, r->ray_d, r->thr, r->hit,
-                                                   r->hit_prim, r->rw, r->em, r->seed, r->nee_a, r->nee_b, r->vis,
+                                                   r->hit_prim, r->rw, r->seed, r->nee_a, r->nee_b, r->vis,
                                                    r->sh_o, r->sh_d, r->sh_root, r->d_albedo, r->d_normal,
                                                    r->queue_e, r->counters);
             else
                 k_shade<false><<<grid, TB, 0, st>>>(S, F, d_lights, (int)b, qa, r->ray_o, r->ray_d, r->thr, r->hit,
-                                                    r->hit_prim, r->rw, r->em, r->seed, r->nee_a, r->nee_b, r->vis,
+                                                    r->hit_prim, r->rw, r->seed, r->nee_a, r->nee_b, r->vis,
                                                     r->sh_o, r->sh_d, r->sh_root, r->d_albedo, r->d_normal,
                                                     r->queue_e, r->counters);
             KF_CHECK(hipEventRecord(r->sync_ev[2 * b], st));
@@ -1711,12 +1798,11 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
                 ++n_sh;
             }
             if (inline_nee)
-                k_connect<true><<<grid_conn, TB, 0, r->st2>>>(F, (int)b, qa, qb, r->thr, r->col, r->rw, r->em,
+                k_connect<true><<<grid_conn, TB, 0, r->st2>>>(F, (int)b, qa, qb, r->thr, r->col, r->rw,
                                                               r->seed, r->nee_a, r->nee_b, r->vis, d_out, r->counters);
             else
-                k_connect<false><<<grid_conn, TB, 0, r->st2>>>(F, (int)b, qa, qb, r->thr, r->col, r->rw, r->em,
+                k_connect<false><<<grid_conn, TB, 0, r->st2>>>(F, (int)b, qa, qb, r->thr, r->col, r->rw,
                                                                r->seed, r->nee_a, r->nee_b, r->vis, d_out, r->counters);
-            k_next_count<<<1, 1, 0, r->st2>>>((int)b, r->counters);
             KF_CHECK(hipEventRecord(r->sync_ev[2 * b + 1], r->st2));
             if (b + 1 < b_tail) launch_extend(b + 1, r->queue_e);
             KF_CHECK(hipStreamWaitEvent(st, r->sync_ev[2 * b + 1], 0));
@@ -1724,7 +1810,8 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
         }
         const bool last = s0 + F.nsamp >= pc->spp;
         k_resolve<<<(WH + TB - 1) / TB, TB, 0, st>>>(F, d_out, d_acc, r->d_rgba,
-                                                     o.keep_samples ? r->samples : nullptr, last ? 1 : 0);
+                                                     o.keep_samples ? r->samples : nullptr, last ? 1 : 0, (int)b_tail,
+                                                     r->counters);
         if (timed) KF_CHECK(hipEventRecord(r->ev[1], st));
         KF_CHECK(hipGetLastError());
     };
@@ -1747,7 +1834,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
         };
         const uint32_t sched[12] = {spb, K, nb, refill, grab, grid, (uint32_t)o.count_traversal,
                                     (uint32_t)o.keep_samples, b_tail, grab0, grabs, r->tune_pairs};
-        const void* bufs[] = {r->ray_o, r->ray_d, r->thr, r->col, r->rw, r->em, r->hit, r->hit_prim, r->seed,
+        const void* bufs[] = {r->ray_o, r->ray_d, r->thr, r->col, r->rw, r->hit, r->hit_prim, r->seed,
                               r->queue_a, r->queue_b, r->queue_e, r->sh_o, r->sh_d, r->sh_root, r->nee_a,
                               r->nee_b, r->vis, r->samples, r->counters, d_lights, d_jump, d_acc, d_out,
                               r->d_rgba, r->d_albedo, r->d_normal, (const void*)r->st2,

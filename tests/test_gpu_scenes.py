@@ -241,3 +241,25 @@ def test_config3_full_frame(gpu):
             gray = rd.download_gray32f()
             assert gray.shape == (w.height, w.width)
             assert (gray == (rgba[..., 0] + rgba[..., 1] + rgba[..., 2]) / np.float32(3.0)).all()
+
+
+# Lights per scene around the group whose shadow rays are appended together (4)
+# and the most whose choices are resolved ahead of the shadow rays (16), up to
+# every slot; transmissive spheres take the other form of the choice.
+@pytest.mark.parametrize("points,active", [(0, 0), (1, 0), (2, 1), (3, 1), (10, 4), (11, 4), (32, 8)])
+def test_render_parity_light_counts(gpu, points, active):
+    w = scenes.config1(48, 32, spp=3, path_depth=5)
+    w.data.point_lights = abi.PointLights()
+    w.data._n_point = 0
+    for k in range(points):
+        w.data.add_point_light((4.0 * np.cos(k), 2.0 + 0.05 * k, 4.0 * np.sin(k)), (1, 0.9, 0.8), 3.0, radius=0.0)
+    for k in range(active):
+        view = scenes.look_at((3.0 * np.cos(2 * k), 4.0, 3.0 * np.sin(2 * k)), (0.0, 0.3, 0.0), (0, 1, 0))
+        w.data.add_active_light(view, (0.8, 0.9, 1.0), fov=0.9, strength=20.0)
+    (res,) = render_both(w)
+    assert_frame_parity(*res)
+    assert res[0].shadow_rays > 0
+    full = Renderer(w.width, w.height)  # every bounce in the wavefront
+    full.set_schedule(tail_bounce=w.pc.path_depth + 1)
+    full.render(GpuScene(w.data), w.cam, w.pc, seed=0, keep_samples=True)
+    assert full.read_samples(w.pc.spp).tobytes() == res[1].tobytes()
