@@ -89,10 +89,11 @@ struct alignas(16) Node {
 // child as a traversal item: bits 31:30 the kind (0 TLAS node, 1 BLAS node,
 // 2 instance, 3 triangle slot), bits 29:0 its index; kEmptyItem marks an
 // unused slot (its box is all zero).  The traversal reads these; the BVH2
-// stays for the builder and its tests.
+// stays for the builder and its tests.  The low planes come first, where a
+// triangle record has its coordinates: the same three loads serve both.
 constexpr uint32_t kEmptyItem = 0xffffffffu;
 struct alignas(16) Node4 {
-    float4 lox, hix, loy, hiy, loz, hiz;
+    float4 lox, loy, loz, hix, hiy, hiz;
     int4 ref;
     int4 pad;
 };
@@ -108,7 +109,7 @@ struct alignas(16) Node4 {
 // the arrays the geometry's shading reads and the geometry's own triangle
 // offset (its material indices), 0.
 struct alignas(16) Inst {
-    float4 lox, hix, loy, hiy, loz, hiz;
+    float4 lox, loy, loz, hix, hiy, hiz;
     int4 ref;
     float4 w2o[3];
     int4 info;

@@ -181,10 +181,10 @@ KF_DEV DV dir_at(const DirMap& m, double px, double py) {
 KF_DEV void tile_child(Node4* __restrict__ nd, uint32_t c, float4 lo, float4 hi, uint32_t item) {
     float* f = reinterpret_cast<float*>(nd);
     f[c] = lo.x;
-    f[4 + c] = hi.x;
-    f[8 + c] = lo.y;
-    f[12 + c] = hi.y;
-    f[16 + c] = lo.z;
+    f[4 + c] = lo.y;
+    f[8 + c] = lo.z;
+    f[12 + c] = hi.x;
+    f[16 + c] = hi.y;
     f[20 + c] = hi.z;
     uint32_t* u = reinterpret_cast<uint32_t*>(nd);
     u[24 + c] = item;
@@ -438,12 +438,18 @@ __global__ __launch_bounds__(TB) void k_raygen(SceneView S, Frame F, const uint2
     }
 }
 
-// Register budgets of the two traversal kernels that run side by side
-// (k_extend of bounce b+1 beside k_shadow of bounce b): 4 waves of k_extend
-// at 104 VGPRs and one wave of k_shadow at 96 fill a SIMD's 512, so the
-// shadow rays are traced while the closest-hit launch is still resident.
-// amdgpu_num_vgpr counts in units of two registers on gfx950 (the unified
-// VGPR/AGPR file), hence 52 and 48.
+// Registers of the two traversal kernels that run side by side (k_extend of
+// bounce b+1 beside k_shadow of bounce b): 4 waves of k_extend (95 VGPRs) and
+// one of k_shadow (84) share a SIMD's 512, so the shadow rays are traced
+// while the closest-hit launch is still resident.  A fifth wave of k_extend
+// fits when it is alone and keeps them out: 1080p frame 18.0 ms against 17.0
+// (kExtendBlocks; within 1 % for the camera rays, which have none beside
+// them).  At 80 VGPRs (40 spilled) the frame took 37 ms.
+// Bound by the vector ALUs (2 M rays: busy 76 % before and 69 % now, 19 % less
+// instructions) and by the vector L1, one lane's line per cycle (91 % before,
+// 68 % now).  amdgpu_num_vgpr counts in units of two registers on gfx950 (the
+// unified VGPR/AGPR file).
+constexpr uint32_t kExtendBlocks = 4;  // per CU
 template <bool COUNT>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_num_vgpr(52))) void k_extend(SceneView S, int bounce, uint32_t cap, const uint32_t* __restrict__ queue,
                                                const float4* __restrict__ ray_o, const float4* __restrict__ ray_d,
@@ -1288,7 +1294,7 @@ __global__ __launch_bounds__(TB) void k_tail2(SceneView S, Frame F, const DevLig
             }
             if (second && pending) alive = start_shadow();
             while (__ballot(alive) != 0ull) {
-                const bool more = T.step(TS, stk, ovf, alive);
+                const bool more = lane_in(T.step(TS, stk, ovf, lanes_of(alive)));
                 if (alive && !more) {
                     alive = false;
                     if (!second) {
@@ -1705,8 +1711,8 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     const uint32_t grab0 = r->tune_grab0 ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grab0)) : grab;
     // shadow rays: short any-hit queries, which favour smaller reservations
     const uint32_t grabs = r->tune_grabs ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grabs)) : grab;
-    // Persistent traversal kernels: exactly the blocks that fit at once.
-    static const uint32_t grid_ext0 = resident_grid(k_extend<false>, n_cu);
+    // Persistent traversal kernels: the blocks that fit at once.
+    static const uint32_t grid_ext0 = std::min(resident_grid(k_extend<false>, n_cu), kExtendBlocks * (uint32_t)n_cu);
     static const uint32_t grid_ext1 = resident_grid(k_extend<true>, n_cu);
     static const uint32_t grid_sh = resident_grid(k_shadow, n_cu);
     const uint32_t nb = pc->path_depth + 1;

@@ -18,7 +18,7 @@
 
 namespace kf {
 
-constexpr int kStack = 64;
+constexpr int kStack = 65;
 constexpr uint32_t kMaxSteps = 1u << 22;  // bound on loop iterations (malformed-tree guard)
 // Slab margin: each computed slab distance (b - o) * rcp(d) carries three
 // roundings, one of them the 1-ulp hardware reciprocal (2 units of 2^-24),
@@ -28,48 +28,45 @@ constexpr float kUnit = 5.96046448e-8f;  // 2^-24
 constexpr float kGamma5 = 5.0f * kUnit / (1.0f - 5.0f * kUnit);
 constexpr float kSlabScale = 1.0f + 2.0f * kGamma5;
 
-// The shear axes kx, ky, kz are kept as lane masks (k0: axis 0, k1: axis
-// 1, neither: axis 2), which the compiler holds in scalar registers.
+// The shear of the watertight test for a wave's object-space rays: axes kx,
+// ky, kz as wave-wide lane masks (bit l: lane l; k0: axis 0, k1: axis 1,
+// neither: axis 2), which the compiler holds in scalar registers, and the
+// scales Sz = 1 / d[kz] correctly rounded, Sx = d[kx] * Sz, Sy = d[ky] * Sz.
+struct Axes {
+    uint64_t x0, x1, y0, y1, z0, z1;
+};
 struct Pre {
-    v3 o, invd;  // invd: culling only (hardware reciprocal)
-    bool x0, x1, y0, y1, z0, z1;
+    bool x0, x1, y0, y1, z0, z1;  // one lane's axes
     float Sx, Sy, Sz;
 };
 
-KF_DEV float comp(v3 a, int i) { return i == 0 ? a.x : (i == 1 ? a.y : a.z); }
 KF_DEV float comp2(v3 a, bool k0, bool k1) { return k0 ? a.x : (k1 ? a.y : a.z); }
 // Component-wise choice.  (c ? a : b on structure lvalues compiles to a copy
 // from a chosen address, which forces the traversal state into memory.)
 KF_DEV v3 sel3(bool c, v3 a, v3 b) { return mk(c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z); }
 KF_DEV v3 rcp3(v3 d) { return mk(__builtin_amdgcn_rcpf(d.x), __builtin_amdgcn_rcpf(d.y), __builtin_amdgcn_rcpf(d.z)); }
+KF_DEV uint64_t lanes_of(bool c) { return __builtin_amdgcn_ballot_w64(c); }
+KF_DEV bool lane_in(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 
-// Shear constants of the watertight test: kz = dominant axis, (kx, ky)
-// swapped when d[kz] < 0 to keep the winding; Sz = 1 / d[kz] correctly
-// rounded, Sx = d[kx] * Sz, Sy = d[ky] * Sz.  In two parts so that a caller
-// can share the division: precompute_axes returns d[kz], precompute_scale
-// takes its correctly rounded reciprocal.  The caller sets invd.
-// kz = (ax >= ay) ? ((ax >= az) ? 0 : 2) : ((ay >= az) ? 1 : 2), kx = kz + 1
-// and ky = kz + 2 (mod 3), swapped when d[kz] < 0; the flags are written as
-// logic on the three comparisons (lane masks, no integer axes).
-KF_DEV float precompute_axes(v3 o, v3 d, Pre& p) {
-    p.o = o;
+// Shear axes of rays with direction d for the lanes in E; the others keep
+// theirs.  kz = the dominant axis, (kx, ky) swapped when d[kz] < 0 to keep
+// the winding: kz = (ax >= ay) ? ((ax >= az) ? 0 : 2) : ((ay >= az) ? 1 : 2),
+// kx = kz + 1 and ky = kz + 2 (mod 3).  Scalar logic on the ballots of the
+// four comparisons: as per-lane flags the compiler made 0/1 registers of them
+// and compared those again (25 vector instructions per step).  Returns d[kz].
+KF_DEV float shear_axes(v3 d, uint64_t E, Axes& A) {
     const float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
-    const bool xy = ax >= ay, xz = ax >= az, yz = ay >= az;
-    const bool z0 = xy && xz, z1 = !xy && yz, z2 = !z0 && !z1;
-    const float dz = z0 ? d.x : (z1 ? d.y : d.z);
-    const bool sw = dz < 0.0f;
-    p.z0 = z0;
-    p.z1 = z1;
-    p.x0 = sw ? z1 : z2;  // the (swapped) x axis is 0
-    p.x1 = sw ? z2 : z0;  // ... is 1
-    p.y0 = sw ? z2 : z1;  // the (swapped) y axis is 0
-    p.y1 = sw ? z0 : z2;  // ... is 1
+    const uint64_t xy = lanes_of(ax >= ay), xz = lanes_of(ax >= az), yz = lanes_of(ay >= az);
+    const uint64_t z0 = xy & xz, z1 = ~xy & yz, z2 = ~(z0 | z1);
+    const float dz = comp2(d, lane_in(z0), lane_in(z1));
+    const uint64_t sw = lanes_of(dz < 0.0f);
+    A.z0 = (z0 & E) | (A.z0 & ~E);
+    A.z1 = (z1 & E) | (A.z1 & ~E);
+    A.x0 = (((sw & z1) | (~sw & z2)) & E) | (A.x0 & ~E);  // the (swapped) x axis is 0
+    A.x1 = (((sw & z2) | (~sw & z0)) & E) | (A.x1 & ~E);  // ... is 1
+    A.y0 = (((sw & z2) | (~sw & z1)) & E) | (A.y0 & ~E);  // the (swapped) y axis is 0
+    A.y1 = (((sw & z0) | (~sw & z2)) & E) | (A.y1 & ~E);  // ... is 1
     return dz;
-}
-KF_DEV void precompute_scale(v3 d, float rcp_dz, Pre& p) {
-    p.Sz = rcp_dz;
-    p.Sx = comp2(d, p.x0, p.x1) * p.Sz;
-    p.Sy = comp2(d, p.y0, p.y1) * p.Sz;
 }
 
 struct TriHit {
@@ -88,7 +85,7 @@ struct TriEdge {
     float U, V, W, det, Tn;
     bool outside;
 };
-KF_DEV TriEdge intersect_begin(const Pre& p, v3 A, v3 B, v3 C, bool en) {  // A, B, C: vertices - p.o
+KF_DEV TriEdge intersect_begin(const Pre& p, v3 A, v3 B, v3 C, bool en) {  // A, B, C: vertices - ray origin
     float Akz = comp2(A, p.z0, p.z1), Bkz = comp2(B, p.z0, p.z1), Ckz = comp2(C, p.z0, p.z1);
     float Ax = comp2(A, p.x0, p.x1) - p.Sx * Akz;
     float Ay = comp2(A, p.y0, p.y1) - p.Sy * Akz;
@@ -121,7 +118,7 @@ KF_DEV bool intersect_end(const TriEdge& e, float rcp_det, float tmin, float tma
     h.t = t;
     h.b1 = e.V * rcp_det;
     h.b2 = e.W * rcp_det;
-    h.back = e.det < 0.0f ? 1u : 0u;
+    h.back = __float_as_uint(e.det) & 0x80000000u;  // det < 0 (a hit's det is neither 0 nor NaN)
     return !e.outside && e.det != 0.0f && t >= tmin && t <= tmax;
 }
 
@@ -158,9 +155,8 @@ KF_DEV v3 xform_dir(const Inst& I, v3 v) {
 // lanes of a wave wait on one memory round trip per step whatever kind of
 // record each lane is on.  An instance record carries its BLAS root node:
 // its step transforms the ray and tests the root's children at once, so
-// entering an instance costs no step of its own.  The stack keeps its top
-// in a register; the entry below it is read with every record fetch, so a
-// pop costs no extra round trip.
+// entering an instance costs no step of its own.  The newest stack entry is
+// read with every record fetch, so a pop costs no extra round trip.
 enum : uint32_t { kTlasNode = 0u, kBlasNode = 1u, kInstance = 2u, kTriangle = 3u };
 constexpr uint32_t kIdxMask = 0x3fffffffu;  // scenes are limited to 2^30 records of each kind
 constexpr uint32_t kNoPrim = 0x7fffffffu;   // best.prim before the first hit
@@ -180,36 +176,39 @@ KF_DEV T opaque_sgpr(T v) {
     return v;
 }
 
-__device__ const float4 kZeroRecord[8] = {};  // at least the lines a step reads of any record
-
 struct TravScene {
     const float4 *tlas, *blas, *inst, *tri;
     uint32_t n_tlas, n_blas, n_inst, n_tri;
-    const float4* zero;  // 128 zero bytes, read in place of an out-of-range record
     const kf_material* mats;
     const uint32_t *matidx, *toff;
     KF_DEV explicit TravScene(const SceneView& S)
         : tlas((const float4*)S.tlas), blas((const float4*)S.blas), inst((const float4*)S.inst), tri(S.tri),
           n_tlas(S.n_tlas_nodes), n_blas(S.n_blas_nodes), n_inst(S.n_inst), n_tri(S.n_tri),
-          zero(kZeroRecord), mats(S.mats), matidx(S.matidx), toff(S.toff) {}
+          mats(S.mats), matidx(S.matidx), toff(S.toff) {}
 };
 
 // ------------------------------------------------------------- stacks
-// A lane's traversal stack below its register-cached top.  Entry i is the
-// i-th oldest; sp counts the entries.
+// A lane's traversal stack.  Entry i is the i-th oldest; sp counts the
+// entries.
 //   peek(sp): entry sp - 1 (read speculatively every step; any in-range
-//             address when sp == 0);  push(sp, v): store v as entry sp;
-//   popped(sp): entry sp has just become the register top (sp is the new
-//             count).
+//             address when sp == 0);
+//   push(sp, k, e0, e1, e2): store the first k of e0, e1, e2 as entries sp,
+//             sp + 1, sp + 2; returns the lanes that had room for them (a
+//             malformed tree: not all);
+//   popped(sp): entry sp has just been taken (sp is the new count).
 struct PrivStack {  // everything in private memory
-    static constexpr int kCap = kStack;
+    static constexpr uint32_t kCap = kStack;
     uint32_t a[kStack];
-    KF_DEV uint32_t peek(int sp) const { return a[sp > 0 ? sp - 1 : 0]; }
-    KF_DEV void push(int sp, uint32_t v, uint32_t& overflow) {
-        if (sp < kStack) a[sp] = v;
-        else overflow = 1;
+    KF_DEV uint32_t peek(uint32_t sp) const { return a[sp > 0u ? sp - 1u : 0u]; }
+    KF_DEV uint64_t push(uint32_t sp, uint32_t k, uint32_t e0, uint32_t e1, uint32_t e2) {
+        const uint64_t room = lanes_of(sp + k <= kCap);
+        k = sp + k <= kCap ? k : 0u;
+        if (k > 0u) a[sp] = e0;
+        if (k > 1u) a[sp + 1u] = e1;
+        if (k > 2u) a[sp + 2u] = e2;
+        return room;
     }
-    KF_DEV void popped(int) {}
+    KF_DEV void popped(uint32_t) {}
 };
 
 // The newest kRing entries in an LDS ring, one column per thread of the
@@ -222,24 +221,35 @@ struct PrivStack {  // everything in private memory
 // stayed in scratch, so every step reloaded the ring pointer from scratch and
 // reached the ring through flat loads and stores (which wait on every
 // outstanding global load as well).
-constexpr int kRing = 16;                 // power of two
+constexpr uint32_t kRing = 16;            // power of two
 constexpr uint32_t kRingThreads = 256;    // block size of kernels using RingStack
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 struct RingStack {
-    static constexpr int kCap = kRing + kStack;
+    static constexpr uint32_t kCap = kRing + kStack;
     lds_u32* ring;    // this thread's column: slot k at ring[k * kRingThreads]
     uint32_t* spill;  // kStack entries in private memory
-    KF_DEV lds_u32& slot(int i) const { return ring[(uint32_t)(i & (kRing - 1)) * kRingThreads]; }
-    KF_DEV uint32_t peek(int sp) const { return slot(sp - 1); }
-    KF_DEV void push(int sp, uint32_t v, uint32_t& overflow) {
-        if (sp >= kCap) {
-            overflow = 1;
-            return;
+    KF_DEV lds_u32& slot(uint32_t i) const { return ring[(i & (kRing - 1u)) * kRingThreads]; }
+    KF_DEV uint32_t peek(uint32_t sp) const { return slot(sp - 1u); }
+    KF_DEV uint64_t push(uint32_t sp, uint32_t k, uint32_t e0, uint32_t e1, uint32_t e2) {
+        // While no lane of the wave is near the ring's end all three are
+        // stored unasked: what lies above the new count is free.
+        if (lanes_of(sp + 3u > kRing) == 0u) {
+            lds_u32* w = ring + sp * kRingThreads;
+            w[0] = e0;
+            w[kRingThreads] = e1;
+            w[2u * kRingThreads] = e2;
+            return ~0ull;
         }
-        if (sp >= kRing) spill[sp - kRing] = slot(sp);  // evict the entry that shares the slot
-        slot(sp) = v;
+        const uint64_t room = lanes_of(sp + k <= kCap);
+        k = sp + k <= kCap ? k : 0u;
+        for (uint32_t i = 0; i < k; ++i) {
+            const uint32_t s = sp + i;
+            if (s >= kRing) spill[s - kRing] = slot(s);  // evict the entry that shares the slot
+            slot(s) = i == 0u ? e0 : (i == 1u ? e1 : e2);
+        }
+        return room;
     }
-    KF_DEV void popped(int sp) {
+    KF_DEV void popped(uint32_t sp) {
         if (sp >= kRing) slot(sp) = spill[sp - kRing];  // bring the next older entry back into the ring
     }
 };
@@ -272,47 +282,48 @@ KF_DEV uint32_t env_root_item(const SceneView& S, uint32_t e) {
 // coin (alpha_coin).  MIXED (with ANY false): each lane's query is a shadow
 // query or a closest-hit one (any_q), so that lanes of one wave trace both
 // kinds with the same steps.
+// What bounds it: the vector ALUs (about 340 instructions per step) and the
+// vector L1 about equally.  Each lane loading its own record's lines only, the
+// shear axes as scalar logic, the sort on 64-bit keys and a stack without a
+// cached top took 19 % of the vector instructions and 26 % of the L1 accesses:
+// 2 M rays 1.05 -> 0.97 ms, 1080p frame at 16 spp 18.7 -> 17.2 ms, 128
+// environments of 512x512 at 8 spp 137.7 -> 129 ms.
 template <bool ANY, bool COUNT, bool MIXED = false>
 struct Trav {
     v3 o, d;         // world-space ray
-    Pre obj;         // object-space ray of the current instance (its axis
-                     // flags are kept in the masks below instead)
-    // Shear axes of the object-space ray as wave-wide lane masks (bit l:
-    // lane l's flag), updated with scalar instructions when lanes enter an
-    // instance and read back as per-lane conditions at no cost; as per-lane
-    // flags their update took about 30 vector instructions per step.
-    uint64_t mx0, mx1, my0, my1, mz0, mz1;
+    // The ray of the level the lane is at: the world-space one in a TLAS, the
+    // current instance's object-space one in its BLAS (a BLAS's items lie on
+    // the stack above all TLAS items, so the world-space one is back before
+    // the next instance); ri: 1 / direction, culling only (hardware reciprocal).
+    v3 ro, ri;
+    Axes ax;         // shear of the current instance's object-space ray
+    float Sx, Sy, Sz;
     float tmin;
     THit best;
     uint32_t cur_inst;  // instance whose BLAS the object-space ray belongs to
     uint32_t cur;    // item processed by the next step
-    uint32_t top;    // stack top, cached in a register (valid when has_top)
-    uint32_t spx;    // bits 7:0 the entries in the stack below the cached
-                     // top, bits 31:8 the steps taken (malformed-tree guard)
-    bool has_top, found, use_alpha;
+    uint32_t spx;    // bits 7:0 the stack's entries, bits 31:8 the steps taken
+                     // (malformed-tree guard); 0 without a query
+    bool found, use_alpha;
     bool any_q;      // MIXED: this lane's query is a shadow query
     uint32_t alpha_seed;
     TCount cnt;
 
-    // Benign state for a lane without a query (it then reads only the zero
-    // record until start() gives it one).
+    // Benign state for a lane without a query.
     KF_DEV void reset() {
-        o = d = mk(0.0f, 0.0f, 0.0f);
-        obj.o = obj.invd = o;
-        obj.x0 = obj.y1 = true;  // kx = 0, ky = 1, kz = 2
-        obj.x1 = obj.y0 = obj.z0 = obj.z1 = false;
-        mx0 = my1 = ~0ull;
-        mx1 = my0 = mz0 = mz1 = 0ull;
-        obj.Sx = obj.Sy = obj.Sz = 0.0f;
+        o = d = ro = ri = mk(0.0f, 0.0f, 0.0f);
+        ax.x0 = ax.y1 = ~0ull;  // kx = 0, ky = 1, kz = 2
+        ax.x1 = ax.y0 = ax.z0 = ax.z1 = 0ull;
+        Sx = Sy = Sz = 0.0f;
         tmin = 0.001f;  // the path tracer's constant, so that its kernels can fold it
         best.t = best.b1 = best.b2 = 0.0f;
         best.inst = ~0u;
         best.prim = kNoPrim;  // closest hit: bit 31 holds the hit kind while tracing
         best.back = 0u;
         cur_inst = 0u;
-        cur = top = 0u;
+        cur = 0u;
         spx = 0u;
-        has_top = found = false;
+        found = false;
         use_alpha = false;
         any_q = false;
         alpha_seed = 0u;
@@ -334,7 +345,6 @@ struct Trav {
         best.back = f ? 0u : best.back;
         cur = f ? root : cur;
         spx = f ? 0u : spx;
-        has_top = f ? false : has_top;
         found = f ? false : found;
         use_alpha = f ? use_alpha_ : use_alpha;
         alpha_seed = f ? r.alpha_seed : alpha_seed;
@@ -354,58 +364,71 @@ struct Trav {
         return r;
     }
 
-    // One record; returns false when the query has finished.  stk: kStack
-    // private entries owned by this query (a separate array so that the
-    // scalar state above stays in registers).
+    // One record for each lane in `live`, the lanes that hold a query; returns
+    // those whose query has not finished.  stk: the
+    // query's stack (a separate object so that the scalar state above stays in
+    // registers).
     //
-    // The entry below the cached top is loaded speculatively together with
-    // the record, so a pop needs no memory access of its own: every step
-    // costs the wave one memory round trip.  Each branch only decides an
-    // action; the stack is updated once at the end.
-    // live: the lane holds a query.  Lanes without one read the zero record
-    // and have no side effects beyond their own (discarded) state.
+    // The newest stack entry is loaded speculatively together with the
+    // record, so a pop needs no memory access of its own: every step costs
+    // the wave one memory round trip.
+    // Lanes without a query fetch nothing and have no side effects beyond
+    // their own (discarded) state.  Sets of lanes are masks in scalar
+    // registers; as per-lane flags they cost a select and a comparison each.
     template <class Stack>
-    KF_DEV bool step(const TravScene& S, Stack& stk, uint32_t& overflow, bool live) {
-        enum { kNext, kPush, kPop, kDone };
+    KF_DEV uint64_t step(const TravScene& S, Stack& stk, uint32_t& overflow, uint64_t live) {
         const uint32_t kind = cur >> 30, idx = cur & kIdxMask;
         // All operands of the per-lane choices are evaluated unconditionally,
         // so the choices stay selects (an asm cannot be speculated).
         const uint32_t n_tlas = opaque_sgpr(S.n_tlas), n_blas = opaque_sgpr(S.n_blas);
         const uint32_t n_inst = opaque_sgpr(S.n_inst), n_tri = opaque_sgpr(S.n_tri);
         const float4 *p_tlas = opaque_sgpr(S.tlas), *p_blas = opaque_sgpr(S.blas);
-        const float4 *p_inst = opaque_sgpr(S.inst), *p_tri = opaque_sgpr(S.tri), *p_zero = opaque_sgpr(S.zero);
+        const float4 *p_inst = opaque_sgpr(S.inst), *p_tri = opaque_sgpr(S.tri);
         const uint32_t lim = kind == kTlasNode ? n_tlas : kind == kBlasNode ? n_blas : kind == kInstance ? n_inst : n_tri;
-        // Out-of-range record or step budget spent (malformed tree): read the
-        // zero record instead and finish the query with the overflow flag.
-        // Kept free of branches: an early exit here makes the compiler copy
-        // the whole traversal state on every step.
-        int sp = (int)(spx & 0xffu);
-        const uint32_t steps = (spx & ~0xffu) + 0x100u;  // this step counted, in bits 31:8
-        const bool bad = live && (idx >= lim || steps > (kMaxSteps << 8));
-        const bool on = live && !bad;
+        // Out-of-range record or step budget spent (malformed tree): fetch
+        // nothing and finish the query with the overflow flag.  Kept free of
+        // early exits: one here makes the compiler copy the whole traversal
+        // state on every step.
+        const uint32_t sp = spx & 0xffu;
+        spx += 0x100u;  // this step counted
+        const uint64_t ON = live & lanes_of(idx < lim) & lanes_of(spx <= ((kMaxSteps << 8) | 0xffu));
+        const bool on = lane_in(ON);
         const float4* base = kind == kTlasNode ? p_tlas : kind == kBlasNode ? p_blas : kind == kInstance ? p_inst : p_tri;
-        const bool node_kind = kind <= kBlasNode;
-        const float4* P = on ? base + (node_kind ? 8u : (kind == kTriangle ? 3u : 12u)) * (size_t)idx : p_zero;
-        // Ten 16-byte global loads issued together: lines 0-6 of a BVH4 node
-        // (128 B) or of an instance record's root node, lines 7-9 of an
-        // instance record (its transform; other lanes read the zero record
-        // there).  A triangle's x, y and z lines (48 B) go where a node's
-        // low x, y and z planes go (r0, r2, r4), and its other loads repeat
-        // its own lines instead of reading past the record.  The empty asm needs all
-        // results, which keeps the compiler from sinking parts of the fetch
-        // into the kind-specific code below (each sunk load would cost the
-        // wave another memory round trip).
-        const gf4* G = (const gf4*)P;
-        const bool wide = kind != kTriangle && on;
-        const bool irec = kind == kInstance && on;
-        const gf4* GI = irec ? G + 7 : (const gf4*)p_zero;
-        const bool trec = kind == kTriangle && on;
-        const vf4 r0 = G[0], r1 = G[1], r2 = G[trec ? 1 : 2], r3 = G[trec ? 2 : 3];
-        const vf4 r4 = G[wide ? 4 : 2], r5 = G[wide ? 5 : 1], r6 = G[wide ? 6 : 0];  // line 7 of a node is padding
-        const vf4 r7 = GI[0], r8 = GI[1], r9 = GI[2];
-        const uint32_t below = stk.peek(sp);
-        asm volatile("" ::"v"(r0), "v"(r1), "v"(r2), "v"(r3), "v"(r4), "v"(r5), "v"(r6), "v"(r7), "v"(r8), "v"(r9),
-                     "v"(below));
+        const uint32_t lines = kind <= kBlasNode ? 8u : (kind == kTriangle ? 3u : 12u);
+        const gf4* G = (const gf4*)(base + (size_t)lines * idx);
+        const uint64_t tri_kind = lanes_of(kind == kTriangle);
+        const uint64_t E = ON & lanes_of(kind == kInstance);
+        const bool is_node = lane_in(ON & ~tri_kind), is_tri = lane_in(ON & tri_kind), is_inst = lane_in(E);
+        // 16-byte global loads issued together: lines 0-2 of any record, a
+        // node's low planes or a triangle's x, y and z; lines 3-6 of a node or
+        // of an instance record's root node; lines 7-9 of an instance record,
+        // its transform.  Each lane loads only its record's lines: the vector
+        // L1 serves one lane's line per cycle, so that ten loads by all 64
+        // lanes kept it busy 81 % of the time beside vector ALUs at 76 % (2 M
+        // rays, 256 icospheres).  The empty asm needs all results, which keeps the
+        // compiler from sinking parts of the fetch into the kind-specific
+        // code below (each sunk load would cost the wave another memory round
+        // trip); what a lane did not load is any value.
+        vf4 r0, r1, r2, r3, r4, r5, r6, r7, r8, r9;
+        if (on) {
+            r0 = G[0];
+            r1 = G[1];
+            r2 = G[2];
+            if (is_node) {
+                r3 = G[3];
+                r4 = G[4];
+                r5 = G[5];
+                r6 = G[6];  // line 7 of a node is for its refits
+                if (is_inst) {
+                    r7 = G[7];
+                    r8 = G[8];
+                    r9 = G[9];
+                }
+            }
+        }
+        uint32_t below = stk.peek(sp);
+        asm volatile("" : "+v"(r0), "+v"(r1), "+v"(r2), "+v"(r3), "+v"(r4), "+v"(r5), "+v"(r6), "+v"(r7), "+v"(r8),
+                     "+v"(r9), "+v"(below));
 
         // Every lane evaluates the record as a node, an instance and a
         // triangle and keeps the result of its kind: per-lane branches would
@@ -417,11 +440,8 @@ struct Trav {
         // instead of 1.13, 4096 rays 0.15 instead of 0.16 (whole calls), and
         // the long launches of full waves are no slower.  An instance record
         // is a node as well (its BLAS root's children).
-        const bool is_node = kind != kTriangle && on;
-        const bool is_inst = irec;
-        const bool is_tri = kind == kTriangle && on;
-        const bool any_inst = __builtin_amdgcn_ballot_w64(is_inst) != 0;
-        const bool any_tri = __builtin_amdgcn_ballot_w64(is_tri) != 0;
+        const bool any_inst = E != 0u;
+        const bool any_tri = (ON & tri_kind) != 0u;
 
         // instance: its BLAS is entered with the object-space ray, which this
         // step's node test already uses for the BLAS root's children (an
@@ -430,8 +450,8 @@ struct Trav {
         // A lane enters an instance or tests a triangle, never both: the two
         // correctly rounded reciprocals (1 / d[kz] of the new shear, 1 / det
         // of the triangle) share one division.
-        const bool enter = is_inst;
-        Pre nobj;
+        const bool world = kind == kTlasNode;
+        ro = sel3(world, o, ro);
         v3 nd = d;
         float dz = 1.0f;
         if (any_inst) {
@@ -439,60 +459,48 @@ struct Trav {
             I.w2o[0] = make_float4(r7.x, r7.y, r7.z, r7.w);
             I.w2o[1] = make_float4(r8.x, r8.y, r8.z, r8.w);
             I.w2o[2] = make_float4(r9.x, r9.y, r9.z, r9.w);
-            nd = xform_dir(I, d);
-            dz = precompute_axes(xform_point(I, o), nd, nobj);
-            obj.o = sel3(enter, nobj.o, obj.o);
-            // lanes outside the exec mask are not in E and keep their bits
-            const uint64_t E = __builtin_amdgcn_ballot_w64(enter);
-            mx0 = (__builtin_amdgcn_ballot_w64(nobj.x0) & E) | (mx0 & ~E);
-            mx1 = (__builtin_amdgcn_ballot_w64(nobj.x1) & E) | (mx1 & ~E);
-            my0 = (__builtin_amdgcn_ballot_w64(nobj.y0) & E) | (my0 & ~E);
-            my1 = (__builtin_amdgcn_ballot_w64(nobj.y1) & E) | (my1 & ~E);
-            mz0 = (__builtin_amdgcn_ballot_w64(nobj.z0) & E) | (mz0 & ~E);
-            mz1 = (__builtin_amdgcn_ballot_w64(nobj.z1) & E) | (mz1 & ~E);
-            cur_inst = enter ? idx : cur_inst;
+            ro = sel3(is_inst, xform_point(I, o), ro);
+            nd = sel3(is_inst, xform_dir(I, d), d);
+            dz = shear_axes(nd, E, ax);
+            cur_inst = is_inst ? idx : cur_inst;
         }
-        // one set of hardware reciprocals (culling only) for the ray this
-        // step's node test uses fresh: the world ray of a TLAS node, the new
-        // object-space ray of an instance (BLAS nodes reuse obj.invd)
-        const bool world = kind == kTlasNode;
-        const v3 rinv = rcp3(sel3(world, d, nd));
-        obj.invd = sel3(enter, rinv, obj.invd);
+        // one set of hardware reciprocals (culling only) where the ray
+        // changes: the world ray of a TLAS node, the new object-space ray of
+        // an instance
+        ri = sel3(world || is_inst, rcp3(nd), ri);
 
-        // The ray this step's node test uses: the world ray for a TLAS node,
-        // the object-space ray (new for an instance) otherwise.  Its low-plane
-        // differences are, on a triangle's lines, the triangle's vertices
-        // minus the object-space origin.
-        const v3 ro = sel3(world, o, obj.o), ri = sel3(world, rinv, obj.invd);
+        // The low planes against that ray's origin; on a triangle's lines the
+        // triangle's vertices relative to the object-space origin.
         const float dlx[4] = {r0.x - ro.x, r0.y - ro.x, r0.z - ro.x, r0.w - ro.x};
-        const float dly[4] = {r2.x - ro.y, r2.y - ro.y, r2.z - ro.y, r2.w - ro.y};
-        const float dlz[4] = {r4.x - ro.z, r4.y - ro.z, r4.z - ro.z, r4.w - ro.z};
+        const float dly[4] = {r1.x - ro.y, r1.y - ro.y, r1.z - ro.y, r1.w - ro.y};
+        const float dlz[4] = {r2.x - ro.z, r2.y - ro.z, r2.z - ro.z, r2.w - ro.z};
 
         // triangle, against the current instance's object-space ray (lanes
         // entering an instance discard it)
+        Pre pre;
+        pre.x0 = lane_in(ax.x0);
+        pre.x1 = lane_in(ax.x1);
+        pre.y0 = lane_in(ax.y0);
+        pre.y1 = lane_in(ax.y1);
+        pre.z0 = lane_in(ax.z0);
+        pre.z1 = lane_in(ax.z1);
+        pre.Sx = Sx;
+        pre.Sy = Sy;
+        pre.Sz = Sz;
         TriEdge te;
         te.det = 1.0f;
-        if (any_tri) {
-            Pre pt = obj;
-            pt.x0 = __builtin_amdgcn_inverse_ballot_w64(mx0);
-            pt.x1 = __builtin_amdgcn_inverse_ballot_w64(mx1);
-            pt.y0 = __builtin_amdgcn_inverse_ballot_w64(my0);
-            pt.y1 = __builtin_amdgcn_inverse_ballot_w64(my1);
-            pt.z0 = __builtin_amdgcn_inverse_ballot_w64(mz0);
-            pt.z1 = __builtin_amdgcn_inverse_ballot_w64(mz1);
-            te = intersect_begin(pt, mk(dlx[0], dly[0], dlz[0]), mk(dlx[1], dly[1], dlz[1]),
+        if (any_tri)
+            te = intersect_begin(pre, mk(dlx[0], dly[0], dlz[0]), mk(dlx[1], dly[1], dlz[1]),
                                  mk(dlx[2], dly[2], dlz[2]), is_tri);
-        }
         TriHit h;
         bool tri_hit = false;
         if (any_tri || any_inst) {
-            const float q = 1.0f / (enter ? dz : te.det);
+            const float q = 1.0f / (is_inst ? dz : te.det);
             if (any_tri) tri_hit = intersect_end(te, q, tmin, best.t, h) && is_tri;
             if (any_inst) {
-                precompute_scale(nd, q, nobj);
-                obj.Sx = enter ? nobj.Sx : obj.Sx;
-                obj.Sy = enter ? nobj.Sy : obj.Sy;
-                obj.Sz = enter ? nobj.Sz : obj.Sz;
+                Sx = is_inst ? comp2(nd, pre.x0, pre.x1) * q : Sx;
+                Sy = is_inst ? comp2(nd, pre.y0, pre.y1) * q : Sy;
+                Sz = is_inst ? q : Sz;
             }
         }
         const uint32_t prim = __float_as_uint(r0.w);
@@ -516,19 +524,22 @@ struct Trav {
             best.b1 = take ? h.b1 : best.b1;
             best.b2 = take ? h.b2 : best.b2;
             best.inst = take ? cur_inst : best.inst;
-            best.prim = take ? (prim | (h.back << 31)) : best.prim;
+            best.prim = take ? (prim | h.back) : best.prim;
         }
         found = found || take;
 
-        // node: four child boxes (Node4 layout: lox, hix, loy, hiy, loz, hiz,
-        // ref), against the world ray (TLAS) or the object-space ray (BLAS
-        // nodes, and instance records, whose ray was set above)
-        const float hix[4] = {r1.x, r1.y, r1.z, r1.w};
-        const float hiy[4] = {r3.x, r3.y, r3.z, r3.w};
+        // node: four child boxes (lines lox, loy, loz, hix, hiy, hiz, ref)
+        // against the level's ray.  A child's sort key is its entry distance
+        // with its item below it, as one 64-bit float whose order is that of
+        // the distances (equal ones by item): an exchange of the sorting
+        // network is then a 64-bit min and max instead of a comparison and
+        // four selects.  No key is a NaN (the high word is a float).
+        const float hix[4] = {r3.x, r3.y, r3.z, r3.w};
+        const float hiy[4] = {r4.x, r4.y, r4.z, r4.w};
         const float hiz[4] = {r5.x, r5.y, r5.z, r5.w};
-        uint32_t citem[4] = {__float_as_uint(r6.x), __float_as_uint(r6.y), __float_as_uint(r6.z), __float_as_uint(r6.w)};
-        float key[4];
-        int nhit = 0;
+        const uint32_t item[4] = {__float_as_uint(r6.x), __float_as_uint(r6.y), __float_as_uint(r6.z), __float_as_uint(r6.w)};
+        double key[4];
+        uint32_t n = 0;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             const float l0x = dlx[c] * ri.x, l1x = (hix[c] - ro.x) * ri.x;
@@ -536,65 +547,45 @@ struct Trav {
             const float l0z = dlz[c] * ri.z, l1z = (hiz[c] - ro.z) * ri.z;
             const float tn = fmaxf(fmaxf(fminf(l0x, l1x), fminf(l0y, l1y)), fmaxf(fminf(l0z, l1z), tmin));
             const float tf = fminf(fminf(fmaxf(l0x, l1x), fmaxf(l0y, l1y)), fminf(fmaxf(l0z, l1z), best.t));
-            const bool h = tn <= tf * kSlabScale && citem[c] != kEmptyItem;
+            const bool h = tn <= tf * kSlabScale && item[c] != kEmptyItem;
             // Nearer child first; any-hit queries take leaf children
             // (triangles, instances: kinds 2 and 3) before inner ones, which
             // finds occluders sooner.
-            key[c] = h ? (((ANY || (MIXED && any_q)) && (citem[c] >> 31)) ? -INFINITY : tn) : INFINITY;
-            nhit += h ? 1 : 0;
+            const float k = h ? (((ANY || (MIXED && any_q)) && (item[c] >> 31)) ? -INFINITY : tn) : INFINITY;
+            key[c] = __hiloint2double((int)__float_as_uint(k), (int)item[c]);
+            n += h ? 1u : 0u;
         }
-        // sorting network on (key, item), ascending
-        auto cx = [&](int i, int j) {
-            const bool sw = key[j] < key[i];
-            const float ki = key[i], kj = key[j];
-            const uint32_t ii = citem[i], ij = citem[j];
-            key[i] = sw ? kj : ki;
-            key[j] = sw ? ki : kj;
-            citem[i] = sw ? ij : ii;
-            citem[j] = sw ? ii : ij;
+        auto cx = [&](int i, int j) __attribute__((always_inline)) {
+            const double a = key[i], b = key[j];
+            asm("v_min_f64 %0, %1, %2" : "=v"(key[i]) : "v"(a), "v"(b));
+            asm("v_max_f64 %0, %1, %2" : "=v"(key[j]) : "v"(a), "v"(b));
         };
         cx(0, 1);
         cx(2, 3);
         cx(0, 2);
         cx(1, 3);
         cx(1, 2);
+        const uint32_t c0 = (uint32_t)__double2loint(key[0]), c1 = (uint32_t)__double2loint(key[1]);
+        const uint32_t c2 = (uint32_t)__double2loint(key[2]), c3 = (uint32_t)__double2loint(key[3]);
 
         if (COUNT) {
-            cnt.nodes += (node_kind && on) ? 1u : 0u;
+            cnt.nodes += (kind <= kBlasNode && on) ? 1u : 0u;
             cnt.tlas += (on && kind == kTlasNode) ? 1u : 0u;
             cnt.tris += is_tri ? 1u : 0u;
             cnt.insts += is_inst ? 1u : 0u;
         }
-        const int node_act = nhit >= 2 ? kPush : (nhit == 1 ? kNext : kPop);
-        int act = is_node ? node_act : (((ANY || (MIXED && any_q)) && take) ? kDone : kPop);
-        const uint32_t next = citem[0];
-        if (bad) {
-            overflow = 1;
-            act = kDone;
-        }
-
-        // Stack update, resolved with selects.  A node with k >= 2 hit
-        // children pushes the k - 1 farther ones, farthest first, so the
-        // nearest of them ends up as the cached top.
-        const bool push = act == kPush, popping = act == kPop;
-        if (!live) act = kDone;
-        const bool alive = act != kDone && (!popping || has_top);
-        const uint32_t popped_item = top;
-#pragma unroll
-        for (int j = 3; j >= 1; --j) {
-            const bool pj = push && j < nhit;
-            if (pj && has_top) stk.push(sp, top, overflow);
-            sp = (pj && has_top && sp < Stack::kCap) ? sp + 1 : sp;
-            top = pj ? citem[j] : top;
-            has_top = has_top || pj;
-        }
-        cur = popping ? popped_item : next;
-        const int sp_in = sp;
-        sp = (popping && sp_in > 0) ? sp_in - 1 : sp_in;
-        top = popping ? below : top;
-        has_top = popping ? sp_in > 0 : has_top;
-        if (popping && sp_in > 0) stk.popped(sp_in - 1);
-        spx = steps | (uint32_t)sp;
+        // The nearest of n hit children is next and the n - 1 others are
+        // pushed, farthest first; without one the newest entry is popped.
+        n = is_node ? n : 0u;
+        const bool pop = n == 0u;
+        uint64_t alive = ON & lanes_of(n + sp != 0u);
+        if (ANY || MIXED) alive &= ~lanes_of((ANY || any_q) && take);
+        const uint64_t room = stk.push(sp, pop ? 0u : n - 1u, n == 2u ? c1 : (n == 3u ? c2 : c3), n == 3u ? c1 : c2, c1);
+        overflow |= lane_in(live & ~(ON & room)) ? 1u : 0u;
+        alive &= room;
+        cur = pop ? below : c0;
+        if (pop && sp > 0u) stk.popped(sp - 1u);
+        spx = lane_in(alive) ? spx + n - 1u : 0u;
         return alive;
     }
 };
@@ -617,7 +608,7 @@ KF_DEV bool traverse(const SceneView& S, uint32_t root, v3 o, v3 d, float tmin, 
     r.payload = 0u;
     T.start(true, r, root, use_alpha);
     if (root != kEmptyItem)
-        while (T.step(TS, stk, overflow, true)) {
+        while (lane_in(T.step(TS, stk, overflow, lanes_of(true)))) {
         }
     best = T.result();
     cnt.nodes += T.cnt.nodes;
@@ -671,7 +662,7 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
     RingStack stk;
     stk.ring = (lds_u32*)(ring + threadIdx.x);
     stk.spill = spill;
-    bool live = false;
+    uint64_t live = 0;  // lanes that hold a query
     uint32_t payload = 0;
     const uint32_t waves = gridDim.x * (kRingThreads / 64u);
     const uint32_t most = n < 64u * waves ? 64u : ~0u;  // queries of one reservation
@@ -679,9 +670,10 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
     bool more = n > 0u;                // some chunk may have queries left
     uint32_t seen = ~0u;               // queries of this chunk known to be taken (~0: not looked at yet)
     uint32_t res_q = 0, res_n = 0;     // reserved queries [res_q, res_q + res_n)
-    auto finish = [&](bool alive) __attribute__((always_inline)) {
-        if (live && !alive) {
-            live = false;
+    auto finish = [&](uint64_t alive) __attribute__((always_inline)) {
+        const bool done = lane_in(live & ~alive);
+        live &= alive;
+        if (done) {
             store(payload, T.result(), T.found);
             if (COUNT) {
                 total.nodes += T.cnt.nodes;
@@ -694,7 +686,7 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
     while (true) {
         // lane numbers by mbcnt: no per-lane mask to keep
         const uint32_t lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-        const unsigned long long idle = __ballot(!live);
+        const uint64_t idle = ~live;
         const uint32_t nidle = (uint32_t)__popcll(idle);
         if ((res_n > 0u || more) && (nidle >= refill || nidle == 64u)) {
             bool fresh = false;
@@ -706,7 +698,7 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
             r.alpha_seed = r.payload = 0u;
             const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
                                                             __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
-            const bool wants = !live;
+            const bool wants = lane_in(idle);
             uint32_t got = 0;
             while (got < nidle && (res_n > 0u || more)) {
                 if (res_n == 0u) {
@@ -758,12 +750,12 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
                 // as a miss.
                 const bool empty = fresh && (!(r.tmin <= r.tmax) || r.root == kEmptyItem);
                 if (empty) store(r.payload, T.result(), false);
-                live = live || (fresh && !empty);
+                live |= lanes_of(fresh) & ~lanes_of(empty);
             }
         }
-        if (!more && res_n == 0u && __ballot(live) == 0ull) break;
-        // The step runs even when no lane holds a query (idle lanes read the
-        // zero record): a path that skipped it would make every step pay for
+        if (!more && res_n == 0u && live == 0u) break;
+        // The step runs even when no lane holds a query (idle lanes fetch
+        // nothing): a path that skipped it would make every step pay for
         // merging the two paths' registers, and the refill state lives only
         // in its branch.
         finish(T.step(TS, stk, overflow, live));

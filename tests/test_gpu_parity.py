@@ -85,6 +85,39 @@ def test_batch_sizes_give_the_same_hits(gpu, n):
         assert np.array_equal(hits["inst"], ref["inst"]) and np.array_equal(hits["prim"], ref["prim"])
 
 
+# Triangles one behind the other whose boxes every ray meets: three children
+# stay on the stack per BVH4 level (log4 n levels), below, at and beyond what
+# the LDS ring holds.  Half the rays pass all triangles but the last one.
+@pytest.mark.parametrize("n", [4, 64, 300, 1024, 4096, 40000])
+def test_stack_depths(gpu, n):
+    v = np.zeros(3 * n, abi.VERTEX_DTYPE)
+    z = np.repeat(np.arange(n) / n, 3)
+    v["pos"] = np.stack([np.tile([0.0, 1.0, 0.0], n), np.tile([0.0, 0.0, 1.0], n), z], 1)
+    v["pos"][-3:, :2] = [[-4.0, -4.0], [8.0, -4.0], [-4.0, 8.0]]
+    v["normal"] = (0.0, 0.0, 1.0)
+    s = scenes.SceneData()
+    s.add_geometry(v, np.arange(3 * n, dtype=np.uint32).reshape(-1, 3), scenes.material())
+    s.add_instance(0, scenes.mat_from_rows(np.eye(3), (0.0, 0.0, 0.0)))
+    rng = np.random.default_rng(n)
+    rays = np.zeros(500, abi.RAY_DTYPE)
+    xy = rng.uniform(0.05, 0.95, (500, 2))
+    up = rng.random(500) < 0.5
+    rays["org"] = np.concatenate([xy, np.where(up, -1.0, 2.0)[:, None]], 1)
+    d = np.concatenate([rng.uniform(-1e-3, 1e-3, (500, 2)), np.where(up, 1.0, -1.0)[:, None]], 1)
+    rays["dir"] = d
+    rays["tmin"], rays["tmax"] = 0.001, 1e4
+    ref = oracle.Scene(s).trace_closest(rays)
+    gs = GpuScene(s)
+    hits = gs.trace_closest(rays)
+    for f in ("inst", "prim", "t", "b1", "b2"):
+        assert hits[f].tobytes() == ref[f].tobytes(), f
+    assert (hits["prim"] == n - 1).any() and (n < 64 or (hits["prim"] != n - 1).any())
+    assert gs.trace_any(rays).all()
+    rays["tmax"] = 2.0 - 1.5 / n  # upwards: past all but the last triangle
+    far = up & (ref["prim"] == n - 1)
+    assert not gs.trace_any(rays)[far].any()
+
+
 # Instances per TLAS around the block sizes of the one-launch build (64, 256,
 # 1024) and beyond it, created directly and by an update from another count.
 @pytest.mark.parametrize("n", [1, 2, 3, 63, 64, 65, 256, 257, 1024, 1025, 3000])
