@@ -9,13 +9,11 @@
 //   final 3x3 conv to RGB, residual on log1p(noisy RGB).
 // Tensors are NHWC BF16 with FP32 accumulation.  Convolutions are implicit
 // GEMMs on v_mfma_f32_16x16x32_bf16:
-//   k_conv2  the plain, pooled-output and upsampled-input convolutions
-//            (forward, and the unmasked data gradient): 8 waves, 32 x 16
-//            tiles, double-buffered LDS filled by loads straight into LDS
-//   k_conv   the first layer (packs the float4 render targets itself), the
-//            FP32 output layer and the masked data gradients (the same
+//   k_conv2  every layer but the first, and the data gradients (the same
 //            kernel on flipped, transposed weights, ReLU mask of the forward
-//            input fused); bias + ReLU fused in both
+//            input fused): 8 waves, 32 x 16 tiles, double-buffered LDS filled
+//            by loads straight into LDS; bias + ReLU fused
+//   k_conv2_pack  the first layer (packs the float4 render targets itself)
 //   k_wgrad  weight and bias gradients, pixels as the K dimension, split-K
 //            with partial sums added in order (k_wgrad_sum)
 // Concatenations cost no copies: producers write into channel slices of the
@@ -80,19 +78,14 @@ struct PackSrc {
 
 // ---------------------------------------------------------------- convolution
 // y[p, co] = sum_{tap, ci} x[p + off(tap), ci] * w[tap, co, ci]   (zero padding)
-// Work item: a tile of 32 x 8 pixels of one image x BN output channels (BN =
+// Work item: a tile of 32 x 16 pixels of one image x BN output channels (BN =
 // 16, 32 or 64, chosen from the channels actually stored); step: an item and
 // one 32-channel chunk of its input.  Per step the block holds in LDS the
-// 34 x 10 input halo of its tile and the weights of all 9 taps, so one
-// barrier pair covers 9 taps x 4 x BN/16 MFMAs per wave; wave w owns a
+// 34 x 18 input halo of its tile and the weights of all 9 taps, so one
+// barrier covers 9 taps x 4 x BN/16 MFMAs per wave; wave w owns a
 // 16 x 4 block of pixels (four 16-pixel MFMA tiles, one per row).
-// The grid is persistent: block b takes items b, b + gridDim.x, ... and,
-// while its waves run the MFMAs of one step, holds the global loads of the
-// next step in registers (written to LDS after the next barrier), so memory
-// latency hides behind matrix work instead of behind other blocks.  Weights
-// stay in LDS while consecutive steps need the same ones (one input chunk
-// and the same output channels).
-// Cin must be a multiple of 32; ldx, ldy multiples of 8.
+// The grid is persistent: block b takes items b, b + gridDim.x, ...  Cin must
+// be a multiple of 32; ldx, ldy multiples of 8.
 constexpr int CBK = 32;
 // LDS rows of the convolution tiles: 32 halves (64 bytes) per pixel or
 // weight row, 16-byte group q of row r stored at group q ^ ((r / 2) % 4), so
@@ -102,22 +95,29 @@ constexpr int CBK = 32;
 constexpr int CCLD = CBK;
 __device__ inline int cofs(int row, int q) { return row * CCLD + ((q ^ ((row >> 1) & 3)) << 3); }
 
+// Division of a uniform 0 <= n < 2^31 by a launch constant 0 < d < 2^31 with
+// scalar instructions (Granlund and Montgomery, "Division by invariant
+// integers using multiplication", 1994): m = ceil(2^(32+s) / d) with s =
+// ceil(log2 d) - 1, so that n (m d - 2^(32+s)) < 2^(32+s).  The compiler's
+// division is some 20 vector instructions by every wave.
+struct FastDiv {
+    uint32_t m = 0, s = 0;  // m 0: d = 1
+    FastDiv() = default;
+    explicit FastDiv(uint32_t d) {
+        if (d < 2u) return;
+        while ((2ull << s) < d) ++s;
+        m = (uint32_t)(((1ull << (32 + s)) + d - 1) / d);
+    }
+    __device__ int operator()(int n) const { return m ? (int)(__umulhi((uint32_t)n, m) >> s) : n; }
+};
+
 // Raw buffer resource over `bytes` bytes at p (stride 0, 32-bit data format):
 // loads at offsets >= bytes return zeros and touch no memory.
 constexpr uint32_t kOOB = 0x80000000u;  // an offset past every resource built here (< 2^31 bytes)
 __device__ inline __amdgpu_buffer_rsrc_t buffer_rsrc(const void* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
-constexpr int TX = 32, TY = 8, HXX = TX + 2, HYY = TY + 2, NHALO = HXX * HYY;
-
-template <int BN>
-struct ConvShape {
-    static constexpr int kHaloU4 = NHALO * 4;               // 16-byte groups of the halo
-    static constexpr int kWU4 = 9 * BN * 4;                 // ... of one chunk of weights
-    static constexpr int kHR = (kHaloU4 + TB - 1) / TB;     // per thread
-    static constexpr int kWR = (kWU4 + TB - 1) / TB;
-    static constexpr int kLds = NHALO * CCLD + 9 * BN * CCLD + 2 * BN;  // halves (+ BN FP32 biases)
-};
+constexpr int TX = 32, HXX = TX + 2;
 
 // FUSE bits: kFuseUp upsampled input channels, kFusePool pooled output,
 // kFusePack the 32-channel network input computed from the render targets
@@ -125,24 +125,137 @@ struct ConvShape {
 // masked by M > 0.
 constexpr int kFuseUp = 1, kFusePool = 2, kFusePack = 4, kOutF32 = 8, kMask = 16;
 
-// Waves per SIMD the register budget is set for: 3 (168 registers) where that
-// needs no spills, else 2 (64 output channels per item, masked data
-// gradient).
-constexpr int conv_waves(int bn, int fuse) { return (bn > 32 || (fuse & kMask)) ? 2 : 3; }
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+// v_cvt_pk_bf16_f32: round to nearest even, as f2bf
+__device__ inline uint32_t pk_bf16(float a, float b) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
 
-// Epilogue of a work item, straight from the accumulators (bias from Bsm,
-// ReLU, optional mask, BF16 or FP32 store, optional 2x2 average pool).
+// 8 bytes into LDS.  As an asm, because before a plain LDS write the compiler
+// waits for all loads into LDS, here those of the next step.
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+__device__ inline void lds_write8(uint16_t* p, uint32_t lo, uint32_t hi) {
+    const uint64_t v = (uint64_t)hi << 32 | lo;
+    asm volatile("ds_write_b64 %0, %1" ::"v"((uint32_t)(uintptr_t)(lds_u16*)p), "v"(v) : "memory");
+}
+
+typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) u32x4v lds_u32x4;
+
+// The mask of a wave's 4 rows and 32 channels from nbp * 32 on, in the layout
+// conv_store writes a whole tile in: lane l, 8 channels of pixel l / 4.
+__device__ inline u32x4v conv_mask(const uint16_t* M, int ldm, int n, int y, int x0, int ch0, int H, int W, int wv,
+                                  int lane) {
+    return *(const u32x4v*)(M + ((size_t)(n * H + y) * W + x0 + (wv & 1) * 16 + (lane >> 2)) * ldm + ch0 + (lane & 3) * 8);
+}
+
+// Whether conv_store takes a wave's 4 rows, the tile's columns and the item's
+// channels whole, 16 bytes per lane.
+template <int BN, int FUSE>
+__device__ inline bool conv_whole(int y0, int x0, int co0, int wv, int H, int W, const uint16_t* Y, int ldy, int cstore,
+                                  const uint16_t* M, int ldm) {
+    return BN >= 32 && (FUSE & kOutF32) == 0 && y0 + 4 * (wv >> 1) + 4 <= H && x0 + TX <= W && co0 + BN <= cstore &&
+           ((uintptr_t)Y & 15) == 0 && (ldy & 7) == 0 &&
+           ((FUSE & kMask) == 0 || (((uintptr_t)M & 15) == 0 && (ldm & 7) == 0));
+}
+
+// Epilogue of a work item, from the accumulators (bias from Bsm, ReLU,
+// optional mask, BF16 or FP32 store, optional 2x2 average pool).  mk: the
+// mask of conv_mask for a whole item, else unused.
+// An accumulator lane holds 4 channels of one pixel and the next lane the next
+// pixel, so that stored as they are (8 bytes per lane) every lane is a line
+// access of its own in the vector L1: 64 per store with 64 channels, which
+// kept it busy two thirds of the time in the layers with few input channels.
+// Whole items therefore go through LDS (tr: 1 KB per wave, 16 pixels x 32
+// channels), which gives each lane 8 channels and four lanes a pixel's 64
+// bytes: 16 accesses per store and half the stores.
 template <int BN, int FUSE>
 __device__ __attribute__((always_inline)) inline void conv_store(const f32x4 (&acc)[4][BN / 16], const float* Bsm,
-                                                                int n, int y0, int x0, int co0, int wv, int lane,
-                                                                int H, int W, uint16_t* __restrict__ Y, int ldy,
-                                                                float* __restrict__ Yf, int ldyf, int cstore,
-                                                                const uint16_t* __restrict__ M, int ldm, int relu,
-                                                                uint16_t* __restrict__ P) {
+                                                                uint16_t* tr, const u32x4v* mk, int n, int y0, int x0,
+                                                                int co0, int wv, int lane, int H, int W,
+                                                                uint16_t* __restrict__ Y, int ldy, float* __restrict__ Yf,
+                                                                int ldyf, int cstore, const uint16_t* __restrict__ M,
+                                                                int ldm, int relu, uint16_t* __restrict__ P) {
     const int fr = lane & 15;
     const struct {
         int n, y0, x0, co0;
     } cur = {n, y0, x0, co0};
+    if constexpr (BN >= 32 && (FUSE & kOutF32) == 0)
+        if (tr && conv_whole<BN, FUSE>(y0, x0, co0, wv, H, W, Y, ldy, cstore, M, ldm)) {
+            uint16_t* Yb = Y + ((size_t)(cur.n * H + cur.y0 + 4 * (wv >> 1)) * W + cur.x0 + (wv & 1) * 16) * ldy + cur.co0;
+            const uint32_t vo = 2u * (uint32_t)((lane >> 2) * ldy + (lane & 3) * 8);
+            // 16-byte group q of pixel p at group q ^ (p / 4): a wave's writes
+            // and reads spread over all banks
+            uint16_t* wr = tr + fr * 32 + (lane >> 4 & 1) * 4;
+            const int wq = (lane >> 5), wx = fr >> 2;
+            const uint16_t* rd = tr + (lane >> 2) * 32 + (((lane & 3) ^ (lane >> 4)) << 3);
+#pragma unroll
+            for (int nbp = 0; nbp < BN / 32; ++nbp) {
+                u32x4v out[4];
+                const f32x4 bias[2] = {*(const f32x4*)&Bsm[nbp * 32 + (lane >> 4) * 4],
+                                       *(const f32x4*)&Bsm[nbp * 32 + 16 + (lane >> 4) * 4]};
+#pragma unroll
+                for (int mt = 0; mt < 4; ++mt) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const int nb = 2 * nbp + h;
+                        float v[4];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            v[e] = acc[mt][nb][e] + bias[h][e];
+                            if (relu) v[e] = fmaxf(v[e], 0.0f);
+                        }
+                        lds_write8(wr + (((2 * h + wq) ^ wx) << 3), pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]));
+                    }
+                    out[mt] = *(const volatile lds_u32x4*)(const lds_u16*)rd;  // after the writes: LDS keeps a wave's order
+                    if constexpr ((FUSE & kMask) != 0) {
+                        const u32x4v m = mk[mt * (BN / 32) + nbp];
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const uint32_t lo = bf2f((uint16_t)m[k]) > 0.0f ? 0xffffu : 0u;
+                            const uint32_t hi = bf2f((uint16_t)(m[k] >> 16)) > 0.0f ? 0xffff0000u : 0u;
+                            out[mt][k] &= lo | hi;
+                        }
+                    }
+                    *(u32x4v*)((char*)(Yb + (size_t)mt * W * ldy + nbp * 32) + vo) = out[mt];
+                }
+                if constexpr ((FUSE & kFusePool) != 0) {
+                    // 2x2 average pool of the rounded outputs: rows 2 mp, 2 mp + 1
+                    // of this lane's pixel (an even one) and of the next, four
+                    // lanes on; summed in the order (2y, 2x), (2y, 2x + 1),
+                    // (2y + 1, 2x), (2y + 1, 2x + 1)
+                    uint16_t* Pb = P + ((size_t)(cur.n * (H >> 1) + (cur.y0 >> 1) + 2 * (wv >> 1)) * (W >> 1) +
+                                        ((cur.x0 + (wv & 1) * 16) >> 1)) * cstore + cur.co0;
+                    const uint32_t po = 2u * (uint32_t)((lane >> 3) * cstore + (lane & 3) * 8);
+#pragma unroll
+                    for (int mp = 0; mp < 2; ++mp) {
+                        u32x4v pv;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const uint32_t q0 = out[2 * mp][k], q2 = out[2 * mp + 1][k];
+                            // row_shl:4 (lane l takes lane l + 4's, within 16 lanes)
+                            const uint32_t q1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)q0, 0x104, 0xF, 0xF, false);
+                            const uint32_t q3 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)q2, 0x104, 0xF, 0xF, false);
+                            float m[2];
+#pragma unroll
+                            for (int e = 0; e < 2; ++e) {
+                                float sum = 0.0f;
+                                sum += bf2f((uint16_t)(q0 >> (16 * e)));
+                                sum += bf2f((uint16_t)(q1 >> (16 * e)));
+                                sum += bf2f((uint16_t)(q2 >> (16 * e)));
+                                sum += bf2f((uint16_t)(q3 >> (16 * e)));
+                                m[e] = 0.25f * sum;
+                            }
+                            pv[k] = pk_bf16(m[0], m[1]);
+                        }
+                        if (!(lane & 4))
+                            *(u32x4v*)((char*)(Pb + (size_t)mp * (W >> 1) * cstore + nbp * 32) + po) = pv;
+                    }
+                }
+            }
+            return;
+        }
     // Epilogue straight from the accumulators: lane holds channels
     // co0 + nb * 16 + 4 (lane / 16) .. + 3 of pixel (lane % 16) of row mt.
     const int xo = cur.x0 + (wv & 1) * 16 + fr;
@@ -170,15 +283,19 @@ __device__ __attribute__((always_inline)) inline void conv_store(const f32x4 (&a
                         v[e] = 0.0f;
             }
             if constexpr ((FUSE & kOutF32) != 0) {
+                float* yp = Yf + pbase * ldyf + (unsigned)(loc * ldyf + ch0);
+                if (cstore == 3) {  // RGB: one store
+                    struct __attribute__((packed, aligned(4))) F3 {
+                        float x, y, z;
+                    };
+                    *(F3*)yp = F3{v[0], v[1], v[2]};
+                    continue;
+                }
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (ch0 + e < cstore) Yf[pbase * ldyf + (unsigned)(loc * ldyf + ch0 + e)] = v[e];
+                    if (ch0 + e < cstore) yp[e] = v[e];
             } else {
-                // v_cvt_pk_bf16_f32: round to nearest even, as f2bf
-                typedef float f2 __attribute__((ext_vector_type(2)));
-                typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-                const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{v[0], v[1]}, b2));
-                const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{v[2], v[3]}, b2));
+                const uint32_t lo = pk_bf16(v[0], v[1]), hi = pk_bf16(v[2], v[3]);
                 uint16_t* yp = Y + pbase * ldy + (unsigned)(loc * ldy + ch0);
                 if (ch0 + 4 <= cstore) {
                     *(uint2*)yp = make_uint2(lo, hi);
@@ -221,10 +338,7 @@ __device__ __attribute__((always_inline)) inline void conv_store(const f32x4 (&a
                     for (int k = 0; k < 4; ++k) sum += bf2f((uint16_t)(q4[k][e >> 1] >> (16 * (e & 1))));
                     m[e] = 0.25f * sum;
                 }
-                typedef float f2 __attribute__((ext_vector_type(2)));
-                typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-                const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{m[0], m[1]}, b2));
-                const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{m[2], m[3]}, b2));
+                const uint32_t lo = pk_bf16(m[0], m[1]), hi = pk_bf16(m[2], m[3]);
                 const size_t qbase = (size_t)(cur.n * (H >> 1) + (cur.y0 >> 1)) * (W >> 1) + (cur.x0 >> 1);
                 const int qloc = (2 * (wv >> 1) + mp) * (W >> 1) + (xl >> 1);
                 *(uint2*)(P + qbase * cstore + (unsigned)(qloc * cstore + ch0)) = make_uint2(lo, hi);
@@ -233,171 +347,34 @@ __device__ __attribute__((always_inline)) inline void conv_store(const f32x4 (&a
     }
 }
 
-template <int BN, int FUSE>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(conv_waves(BN, FUSE), conv_waves(BN, FUSE)))) void k_conv(const uint16_t* __restrict__ X, int ldx, int Cin,
-                                             const uint16_t* __restrict__ Wt, const float* __restrict__ bias,
-                                             int Cout, int N, int H, int W, uint16_t* __restrict__ Y, int ldy,
-                                             float* __restrict__ Yf, int ldyf, int cstore,
-                                             const uint16_t* __restrict__ M, int ldm, int relu, int n_items,
-                                             const uint16_t* __restrict__ X2, int ldx2, int csplit,
-                                             uint16_t* __restrict__ P) {
-    using SH = ConvShape<BN>;
-    __shared__ __attribute__((aligned(16))) uint16_t smem[SH::kLds];
-    uint16_t* Hs = smem;
-    uint16_t* Ws = smem + NHALO * CCLD;
-    float* Bsm = (float*)(smem + NHALO * CCLD + 9 * BN * CCLD);  // biases of the LDS weights' channels
-    const int tiles_x = (W + TX - 1) / TX, tiles_y = (H + TY - 1) / TY;
-    const int n_tiles = N * tiles_x * tiles_y;
-    const int nchunk = Cin / CBK;
-    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    const int fr = lane & 15;
-    const uint4 zero = make_uint4(0, 0, 0, 0);
-    struct Item {
-        int n, y0, x0, co0;
-    };
-    auto decode = [&](int i) {  // i is uniform: the fields live in scalar registers
-        Item it;
-        const int tile = i % n_tiles;
-        it.co0 = __builtin_amdgcn_readfirstlane((i / n_tiles) * BN);
-        it.x0 = __builtin_amdgcn_readfirstlane((tile % tiles_x) * TX);
-        const int r = tile / tiles_x;
-        it.y0 = __builtin_amdgcn_readfirstlane((r % tiles_y) * TY);
-        it.n = __builtin_amdgcn_readfirstlane(r / tiles_y);
-        return it;
-    };
-    uint4 hreg[SH::kHR], wreg[SH::kWR];
-    auto load_halo = [&](const Item& it, int ci0, bool valid) {
-        // Halo slot r of this thread: pixel hp = (t + r TB) / 4 of the (TX + 2) x
-        // (TY + 2) halo, 16-byte channel group q, read through a buffer
-        // resource over the item's image: offsets past its end (pixels off the
-        // image, unused slots, or every slot when there is no next step) read
-        // zeros without a branch.
-        const int y0 = it.y0 - 1, x0 = it.x0 - 1;
-        const bool up = (FUSE & kFuseUp) != 0 && ci0 >= csplit;  // the upsampled half-resolution tensor
-        const int sh = up ? 1 : 0, Wl = W >> sh, ld = up ? ldx2 : ldx, c0 = up ? ci0 - csplit : ci0;
-        const uint32_t img = (uint32_t)(H >> sh) * (uint32_t)Wl * (uint32_t)ld;  // elements of one image
-        const uint16_t* base = (up ? X2 : X) + (size_t)it.n * img;
-        const __amdgpu_buffer_rsrc_t rs = buffer_rsrc(base, valid ? 2 * img : 0);
-#pragma unroll
-        for (int r = 0; r < SH::kHR; ++r) {
-            const int i = t + r * TB;
-            const int hp = i >> 2, q = i & 3;
-            const int hy = hp / HXX, hx = hp - hy * HXX;
-            const int yy = y0 + hy, xx = x0 + hx;
-            const bool ok = i < SH::kHaloU4 && (unsigned)yy < (unsigned)H && (unsigned)xx < (unsigned)W;
-            const uint32_t off = ok ? 2u * (uint32_t)(((yy >> sh) * Wl + (xx >> sh)) * ld + c0 + q * 8) : kOOB;
-            hreg[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
-        }
-    };
-    float breg = 0.0f;
-    auto load_w = [&](int co0, int ci0) {
-        const __amdgpu_buffer_rsrc_t rb = buffer_rsrc(bias, bias ? 4u * Cout : 0u);
-        const bool okb = t < BN && co0 + t < Cout;
-        breg = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, okb ? 4u * (co0 + t) : kOOB, 0, 0));
-        const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(Wt, 18u * Cout * Cin);
-#pragma unroll
-        for (int r = 0; r < SH::kWR; ++r) {
-            const int i = t + r * TB;
-            const int q = i & 3, rr = (i >> 2) % BN, tap = (i >> 2) / BN;
-            const int co = co0 + rr;
-            const bool ok = i < SH::kWU4 && co < Cout;
-            const uint32_t off = ok ? 2u * (uint32_t)((tap * Cout + co) * Cin + ci0 + q * 8) : kOOB;
-            wreg[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw, off, 0, 0));
-        }
-    };
-    int i = blockIdx.x, c = 0;
-    if (i >= n_items) return;
-    Item cur = decode(i);
-    load_halo(cur, 0, true);
-    load_w(cur.co0, 0);
-    bool need_w = true;
-    f32x4 acc[4][BN / 16];
-    while (true) {
-        __syncthreads();  // the previous step's LDS reads (and epilogue) are done
-        {
-#pragma unroll
-            for (int r = 0; r < SH::kHR; ++r) {
-                const int k = t + r * TB;
-                if (k < SH::kHaloU4) *(uint4*)&Hs[cofs(k >> 2, k & 3)] = hreg[r];
-            }
-        }
-        if (need_w) {
-            if (t < BN) Bsm[t] = breg;
-#pragma unroll
-            for (int r = 0; r < SH::kWR; ++r) {
-                const int k = t + r * TB;
-                if (k < SH::kWU4) *(uint4*)&Ws[cofs(k >> 2, k & 3)] = wreg[r];
-            }
-        }
-        __syncthreads();
-        // the next step; its loads go out between the MFMAs below
-        int ni = i, nc = c + 1;
-        if (nc == nchunk) {
-            nc = 0;
-            ni = i + gridDim.x;
-        }
-        const bool has_next = ni < n_items;
-        const Item nxt = has_next ? decode(ni) : cur;
-        const bool next_w = has_next && (nxt.co0 != cur.co0 || nc != c);
-        if (c == 0) {
-#pragma unroll
-            for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-                for (int nb = 0; nb < BN / 16; ++nb) acc[mt][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        // Wave w owns pixel rows 4 (w / 2) .. + 3 of the 16 columns (w % 2) * 16 ..;
-        // per horizontal offset dx it reads the 6 halo rows it spans once and
-        // uses each for up to 3 vertical taps.  The weights are the MFMA's A
-        // operand and the pixels its B operand, so each lane ends up holding 4
-        // consecutive output channels of one pixel.
-#pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-            bf16x8 a[6];
-#pragma unroll
-            for (int j = 0; j < 6; ++j)
-                a[j] = __builtin_bit_cast(
-                    bf16x8, *(const uint4*)&Hs[cofs((4 * (wv >> 1) + j) * HXX + (wv & 1) * 16 + fr + dx, lane >> 4)]);
-#pragma unroll
-            for (int dy = 0; dy < 3; ++dy) {
-                const int tap = dy * 3 + dx;
-#pragma unroll
-                for (int nb = 0; nb < BN / 16; ++nb) {
-                    const bf16x8 b =
-                        __builtin_bit_cast(bf16x8, *(const uint4*)&Ws[cofs(tap * BN + nb * 16 + fr, lane >> 4)]);
-#pragma unroll
-                    for (int mt = 0; mt < 4; ++mt)
-                        acc[mt][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, a[mt + dy], acc[mt][nb], 0, 0, 0);
-                }
-            }
-            if (dx == 0) load_halo(nxt, nc * CBK, has_next);
-            if (dx == 1 && next_w) load_w(nxt.co0, nc * CBK);
-        }
-        if (c == nchunk - 1)
-            conv_store<BN, FUSE>(acc, Bsm, cur.n, cur.y0, cur.x0, cur.co0, wv, lane, H, W, Y, ldy, Yf, ldyf, cstore, M, ldm,
-                                 relu, P);
-        if (!has_next) break;
-        i = ni;
-        c = nc;
-        cur = nxt;
-        need_w = next_w;
-    }
-}
-
 // ---------------------------------------------------------- convolution, 8 waves
-// The forward convolutions without packed input, mask or FP32 output (plain,
-// upsampled input, pooled output), for 32 or 64 output channels per item:
-// blocks of 8 waves on 32 x 16 pixel tiles (wave w owns the same 16 x 4
-// pixel block as in k_conv, rows 4 (w / 2) ..), with two LDS buffers, each
+// Blocks of 8 waves, wave w on rows 4 (w / 2) .. + 3 and columns (w % 2) * 16 ..
+// of the tile, with two LDS buffers, each
 // holding one step's 34 x 18 halo and weights.  Both go from memory straight
 // into LDS (buffer loads with the LDS bit: lane l's 16 bytes land at the
 // instruction's LDS base + 16 l, and an offset past the resource writes
 // zeros), so the loads of step s + 1 run into one buffer while the waves
-// run the MFMAs of step s on the other, without staging registers.  The
-// MFMAs, their order and the epilogue are those of k_conv, so the outputs are
-// the same bits.
+// run the MFMAs of step s on the other, without staging registers.  Per
+// horizontal offset a wave reads the 6 halo rows it spans once and uses each
+// for up to 3 vertical taps; the weights are the MFMA's A operand and the
+// pixels its B operand, so each lane ends up holding 4 consecutive output
+// channels of one pixel.
+//
+// What bounds it (32 x 512x512, all 19 layers 2.7 ms; the MFMAs alone 1.6):
+// loads, stores and MFMAs of a step overlap only in part, each about a fifth
+// of the time when taken out.  Against 2.98 ms before: addresses kept per lane
+// and scalar divisions (the vector ALUs spent 2-9 instructions per MFMA, now
+// 2-6; 1-3 %), stores of 16 bytes per lane (2.98 -> 2.78), resident weights of
+// three chunks and half-resolution halos (2.78 -> 2.71).  Measured and not
+// taken: LDS reads a tap ahead of their MFMAs (two fragment sets, 256
+// registers), +9 %; the stores of an item moved behind the next step's loads,
+// no gain; waves of one SIMD at different priorities, no gain.
+constexpr int kTrans = 512;  // halves of a wave's transposition buffer (conv_store)
 constexpr int TB2 = 512, TY2 = 16, HYY2 = TY2 + 2, NHALO2 = HXX * HYY2;
 constexpr int kHaloUnits2 = NHALO2 * 4;                      // 16-byte units of the halo
 constexpr int kHaloLoads2 = (kHaloUnits2 + 63) / 64;         // wave loads that cover it
+constexpr int HXU = HXX / 2 + 1, HYU = HYY2 / 2 + 1;         // the half-resolution pixels under a halo
+constexpr int kUpUnits2 = HXU * HYU * 4, kUpLoads2 = (kUpUnits2 + 63) / 64;
 typedef __attribute__((address_space(3))) void lds_void;
 
 template <int BN>
@@ -409,79 +386,172 @@ struct Conv2Shape {
     static_assert(kWUnits % 64 == 0, "whole wave loads of weights");
 };
 
-template <int BN, int FUSE>
+// Division of the item number into channel block and tile, of the tile into
+// image, row and column of tiles.
+struct ConvDiv {
+    FastDiv tiles, cols, rows;
+};
+
+// RES (32 output channels per item, at most kRes2 input chunks): the weights
+// of an item's output channels stay in LDS for all its chunks; else each step
+// brings its chunk's, unless its buffer holds them already (two chunks).
+constexpr int kRes2 = 3;
+
+template <int BN, int FUSE, bool RES>
 __global__ __launch_bounds__(TB2) void k_conv2(const uint16_t* __restrict__ X, int ldx, int Cin,
                                               const uint16_t* __restrict__ Wt, const float* __restrict__ bias,
-                                              int Cout, int N, int H, int W, uint16_t* __restrict__ Y, int ldy,
-                                              float* __restrict__ Yf, int ldyf, int cstore, int relu, int n_items,
+                                              int Cout, int H, int W, uint16_t* __restrict__ Y, int ldy,
+                                              float* __restrict__ Yf, int ldyf, int cstore,
+                                              const uint16_t* __restrict__ M, int ldm, int relu, int n_items,
                                               const uint16_t* __restrict__ X2, int ldx2, int csplit,
-                                              uint16_t* __restrict__ P) {
-    static_assert(((FUSE & ~(kFuseUp | kFusePool)) == 0 && (BN == 32 || BN == 64)) || (FUSE == kOutF32 && BN == 16),
+                                              uint16_t* __restrict__ P, int n_tiles, ConvDiv div) {
+    static_assert(((FUSE & ~(kFuseUp | kFusePool)) == 0 && (BN == 32 || (BN == 64 && !RES))) ||
+                      (FUSE == kMask && BN == 32) || (FUSE == kOutF32 && BN == 16 && !RES),
                   "k_conv2 variants");
     using SH = Conv2Shape<BN>;
     // two separate arrays, so that the compiler tells the buffers apart and
     // the MFMA reads of one need not wait for the loads into the other
-    __shared__ __attribute__((aligned(16))) uint16_t buf0[SH::kBuf];
-    __shared__ __attribute__((aligned(16))) uint16_t buf1[SH::kBuf];
+    __shared__ __attribute__((aligned(16))) uint16_t buf0[RES ? SH::kHalo : SH::kBuf];
+    __shared__ __attribute__((aligned(16))) uint16_t buf1[RES ? SH::kHalo : SH::kBuf];
+    __shared__ __attribute__((aligned(16))) uint16_t wres[RES ? kRes2 * SH::kWUnits * 8 + 2 * 64 : 8];
+    __shared__ __attribute__((aligned(16))) uint16_t tr[TB2 / 64 * kTrans];
     const int tiles_x = (W + TX - 1) / TX, tiles_y = (H + TY2 - 1) / TY2;
-    const int n_tiles = N * tiles_x * tiles_y;
     const int nchunk = Cin / CBK;
     const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
     const int fr = lane & 15;
     struct Item {
         int n, y0, x0, co0;
     };
-    auto decode = [&](int i) {  // i is uniform: the fields live in scalar registers
+    auto decode = [&](int i) __attribute__((always_inline)) {  // i is uniform: scalar arithmetic
         Item it;
-        const int tile = i % n_tiles;
-        it.co0 = __builtin_amdgcn_readfirstlane((i / n_tiles) * BN);
-        it.x0 = __builtin_amdgcn_readfirstlane((tile % tiles_x) * TX);
-        const int r = tile / tiles_x;
-        it.y0 = __builtin_amdgcn_readfirstlane((r % tiles_y) * TY2);
-        it.n = __builtin_amdgcn_readfirstlane(r / tiles_y);
+        const int cb = div.tiles(i), tile = i - cb * n_tiles;
+        const int r = div.cols(tile);
+        it.co0 = cb * BN;
+        it.x0 = (tile - r * tiles_x) * TX;
+        it.n = div.rows(r);
+        it.y0 = (r - it.n * tiles_y) * TY2;
         return it;
     };
     // The loads of one step into buffer B: halo unit u = load j, lane l is
     // LDS row u / 4 (a halo pixel), 16-byte slot u % 4, which holds channel
     // group (u % 4) ^ ((row / 2) % 4) of that pixel (the swizzle of cofs).
-    auto issue = [&](uint16_t* B, const Item& it, int ci0, bool with_w) __attribute__((always_inline)) {
+    // A lane's offsets from the halo's first pixel and from the step's first
+    // weight are the same in every step: kept in registers, with the step's
+    // part in the instruction's scalar offset, so that a step's loads cost no
+    // vector instructions.  Only tiles at the image's edge, whose pixels off
+    // the image read zeros, and blocks of fewer than BN output channels form
+    // their offsets anew.
+    constexpr int kHaloPer = (kHaloLoads2 + TB2 / 64 - 1) / (TB2 / 64), kWPer = (SH::kWLoads + TB2 / 64 - 1) / (TB2 / 64);
+    // HALF: a chunk of upsampled channels brings the half-resolution pixels its
+    // halo repeats, 18 x 10 instead of 34 x 18.  At 64 output channels per item
+    // the second set of LDS addresses spills (40 registers: 364 -> 520 us for
+    // the 64 + 96 channel layer of 32 x 512x512), at 32 it fits.
+    constexpr bool HALF = BN == 32;
+    constexpr int kUpUnits = HALF ? kUpUnits2 : kHaloUnits2, kUpLoads = HALF ? kUpLoads2 : kHaloLoads2;
+    constexpr int kUpPer = (kUpLoads + TB2 / 64 - 1) / (TB2 / 64);
+    uint32_t hoff[kHaloPer], uoff[kUpPer], woff[kWPer];
+#pragma unroll
+    for (int k = 0; k < kHaloPer; ++k) {
+        // the last load's lanes past the halo repeat its last unit
+        const int u = min((wv + k * (TB2 / 64)) * 64 + lane, kHaloUnits2 - 1), r = u >> 2;
+        const int q = (u & 3) ^ ((r >> 1) & 3);
+        const int hy = r / HXX, hx = r - hy * HXX;
+        hoff[k] = 2u * (uint32_t)((hy * W + hx) * ldx + q * 8);
+    }
+#pragma unroll
+    for (int k = 0; k < kUpPer; ++k) {
+        const int u = min((wv + k * (TB2 / 64)) * 64 + lane, kUpUnits - 1), r = u >> 2;
+        const int q = (u & 3) ^ ((r >> 1) & 3);
+        int hy = r / (HALF ? HXU : HXX), hx = r - hy * (HALF ? HXU : HXX);
+        if (!HALF) hy = (hy + 1) >> 1, hx = (hx + 1) >> 1;
+        uoff[k] = 2u * (uint32_t)((hy * (W >> 1) + hx) * ldx2 + q * 8);
+    }
+#pragma unroll
+    for (int k = 0; k < kWPer; ++k) {
+        const int u = (wv + k * (TB2 / 64)) * 64 + lane, r = u >> 2;
+        const int q = (u & 3) ^ ((r >> 1) & 3);
+        const int tap = r / BN;
+        woff[k] = 2u * (uint32_t)((tap * Cout + (r - tap * BN)) * Cin + q * 8);
+    }
+    // Pixel (y0 - 1 + hy) / 2 of the half-resolution tensor is y0 / 2 - 1 +
+    // (hy + 1) / 2 (y0, x0 are even), and is off it where the pixel is off the
+    // image.
+    auto issue_halo = [&](uint16_t* B, const Item& it, int ci0) __attribute__((always_inline)) {
         const bool up = (FUSE & kFuseUp) != 0 && ci0 >= csplit;  // the upsampled half-resolution tensor
-        const int sh = up ? 1 : 0, Wl = W >> sh, ld = up ? ldx2 : ldx, c0 = up ? ci0 - csplit : ci0;
-        const uint32_t img = (uint32_t)(H >> sh) * (uint32_t)Wl * (uint32_t)ld;
+        const int sh = up ? 1 : 0, Hl = H >> sh, Wl = W >> sh, ld = up ? ldx2 : ldx, c0 = up ? ci0 - csplit : ci0;
+        const int y0 = (it.y0 >> sh) - 1, x0 = (it.x0 >> sh) - 1;  // the halo's first pixel
+        const uint32_t img = (uint32_t)Hl * (uint32_t)Wl * (uint32_t)ld;
         const __amdgpu_buffer_rsrc_t rs = buffer_rsrc((up ? X2 : X) + (size_t)it.n * img, 2 * img);
-        for (int j = wv; j < kHaloLoads2; j += TB2 / 64) {
-            const int u = j * 64 + lane, r = u >> 2;
-            const int q = (u & 3) ^ ((r >> 1) & 3);
-            const int hy = r / HXX, hx = r - hy * HXX;
-            const int yy = it.y0 - 1 + hy, xx = it.x0 - 1 + hx;
-            const bool ok = u < kHaloUnits2 && (unsigned)yy < (unsigned)H && (unsigned)xx < (unsigned)W;
-            const uint32_t off = ok ? 2u * (uint32_t)(((yy >> sh) * Wl + (xx >> sh)) * ld + c0 + q * 8) : kOOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(B + j * 512), 16, off, 0, 0, 0);
-        }
-        if (with_w) {
-            const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(Wt, 18u * Cout * Cin);
-            uint16_t* Ws = B + SH::kHalo;
-            for (int j = wv; j < SH::kWLoads; j += TB2 / 64) {
+        const int hh = up ? HYU : HYY2, hw = up ? HXU : HXX;  // its size
+        const bool inside = y0 >= 0 && x0 >= 0 && y0 + hh <= Hl && x0 + hw <= Wl;
+        const uint32_t s0 = inside ? 2u * (uint32_t)((y0 * Wl + x0) * ld + c0) : 0u;
+        auto load = [&](int k, int units, int width, uint32_t off) __attribute__((always_inline)) {
+            const int j = wv + k * (TB2 / 64);
+            if (!inside) {
                 const int u = j * 64 + lane, r = u >> 2;
-                const int q = (u & 3) ^ ((r >> 1) & 3);
-                const int tap = r / BN, co = it.co0 + (r - tap * BN);
-                const uint32_t off = co < Cout ? 2u * (uint32_t)((tap * Cout + co) * Cin + ci0 + q * 8) : kOOB;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void*)(Ws + j * 512), 16, off, 0, 0, 0);
+                int hy = r / width, hx = r - hy * width;
+                if (!HALF && up) hy = (hy + 1) >> 1, hx = (hx + 1) >> 1;
+                const bool ok = u < units && (unsigned)(y0 + hy) < (unsigned)Hl && (unsigned)(x0 + hx) < (unsigned)Wl;
+                off = ok ? off + 2u * (uint32_t)((y0 * Wl + x0) * ld + c0) : kOOB;
             }
-            if (wv == TB2 / 64 - 1) {  // the biases of the item's channels, 4 bytes per lane
-                const __amdgpu_buffer_rsrc_t rb = buffer_rsrc(bias, bias ? 4u * Cout : 0u);
-                const uint32_t off = it.co0 + lane < Cout ? 4u * (uint32_t)(it.co0 + lane) : kOOB;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void*)(Ws + SH::kWUnits * 8), 4, off, 0, 0, 0);
-            }
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_void*)(B + j * 512), 16, off, s0, 0, 0);
+        };
+        if (up) {
+#pragma unroll
+            for (int k = 0; k < kUpPer; ++k)
+                if ((k + 1) * (TB2 / 64) <= kUpLoads || wv + k * (TB2 / 64) < kUpLoads)
+                    load(k, kUpUnits, HALF ? HXU : HXX, uoff[k]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < kHaloPer; ++k)
+                if ((k + 1) * (TB2 / 64) <= kHaloLoads2 || wv + k * (TB2 / 64) < kHaloLoads2)
+                    load(k, kHaloUnits2, HXX, hoff[k]);
         }
+    };
+    // the weights of chunk ci0 of the item's output channels to Ws
+    auto issue_w = [&](uint16_t* Ws, const Item& it, int ci0) __attribute__((always_inline)) {
+            const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(Wt, 18u * Cout * Cin);
+            const bool whole = it.co0 + BN <= Cout;
+            const uint32_t s0 = whole ? 2u * (uint32_t)(it.co0 * Cin + ci0) : 0u;
+#pragma unroll
+            for (int k = 0; k < kWPer; ++k) {
+                const int j = wv + k * (TB2 / 64);
+                if ((k + 1) * (TB2 / 64) > SH::kWLoads && j >= SH::kWLoads) continue;
+                uint32_t off = woff[k];
+                if (!whole) {
+                    const int r = (j * 64 + lane) >> 2, co = it.co0 + r % BN;
+                    off = co < Cout ? off + 2u * (uint32_t)(it.co0 * Cin + ci0) : kOOB;
+                }
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_void*)(Ws + j * 512), 16, off, s0, 0, 0);
+            }
+    };
+    // the biases of the item's channels, 4 bytes per lane
+    auto issue_b = [&](uint16_t* Bs, const Item& it) __attribute__((always_inline)) {
+        if (wv == TB2 / 64 - 1) {
+            const __amdgpu_buffer_rsrc_t rb = buffer_rsrc(bias, bias ? 4u * Cout : 0u);
+            const uint32_t off = it.co0 + lane < Cout ? 4u * (uint32_t)(it.co0 + lane) : kOOB;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_void*)Bs, 4, off, 0, 0, 0);
+        }
+    };
+    constexpr int kW1 = SH::kWUnits * 8;  // halves of one chunk's weights
+    auto issue_all = [&](const Item& it) __attribute__((always_inline)) {  // RES: all chunks' weights
+        for (int q = 0; q < nchunk; ++q) issue_w(wres + q * kW1, it, q * CBK);
+        issue_b(wres + kRes2 * kW1, it);
     };
     int i = blockIdx.x, c = 0;
     if (i >= n_items) return;
     Item cur = decode(i);
     // weights (output block, chunk) held by each buffer: a step whose weights
     // a buffer already holds loads only the halo
-    int wkey0 = cur.co0 * 1024, wkey1 = -1;
-    issue(buf0, cur, 0, true);
+    // (RES: wkey0 the output block held)
+    int wkey0 = RES ? cur.co0 : cur.co0 * 1024, wkey1 = -1;
+    issue_halo(buf0, cur, 0);
+    if constexpr (RES) {
+        issue_all(cur);
+    } else {
+        issue_w(buf0 + SH::kHalo, cur, 0);
+        issue_b(buf0 + SH::kHalo + kW1, cur);
+    }
     f32x4 acc[4][BN / 16];
     // One step: MFMAs of (cur, c) from buffer A while the next step's loads
     // go into buffer B.  Returns false after the block's last step.
@@ -495,13 +565,35 @@ __global__ __launch_bounds__(TB2) void k_conv2(const uint16_t* __restrict__ X, i
         const Item nxt = has_next ? decode(ni) : cur;
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's loads into A have landed
         __syncthreads();                     // every wave's; and B is no longer read
+        if constexpr (RES) {
+            if (c == 0 && cur.co0 != wkey0) {  // other output channels: once per BN of them
+                issue_all(cur);
+                wkey0 = cur.co0;
+                __builtin_amdgcn_s_waitcnt(0x0F70);
+                __syncthreads();
+            }
+        }
         if (has_next) {
+            issue_halo(B, nxt, nc * CBK);
             const int k = nxt.co0 * 1024 + nc;
-            issue(B, nxt, nc * CBK, k != wkeyB);
-            wkeyB = k;
+            if (!RES && k != wkeyB) {
+                issue_w(B + SH::kHalo, nxt, nc * CBK);
+                issue_b(B + SH::kHalo + kW1, nxt);
+                wkeyB = k;
+            }
         }
         const uint16_t* Hs = A;
-        const uint16_t* Ws = A + SH::kHalo;
+        const uint16_t* Ws = RES ? wres + c * kW1 : A + SH::kHalo;
+        const float* Bsm = (const float*)(RES ? wres + kRes2 * kW1 : A + SH::kHalo + kW1);
+        u32x4v mk[4 * (BN / 32 + (BN < 32))];
+        if constexpr ((FUSE & kMask) != 0)
+            if (c == nchunk - 1 && conv_whole<BN, FUSE>(cur.y0, cur.x0, cur.co0, wv, H, W, Y, ldy, cstore, M, ldm)) {
+                // the mask, under way beside the MFMAs
+#pragma unroll
+                for (int k = 0; k < 4 * (BN / 32); ++k)
+                    mk[k] = conv_mask(M, ldm, cur.n, cur.y0 + 4 * (wv >> 1) + k / (BN / 32), cur.x0,
+                                      cur.co0 + k % (BN / 32) * 32, H, W, wv, lane);
+            }
         if (c == 0) {
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt)
@@ -510,32 +602,45 @@ __global__ __launch_bounds__(TB2) void k_conv2(const uint16_t* __restrict__ X, i
         }
         // per horizontal offset dx: the 6 halo rows and the 3 x BN / 16 weight
         // fragments of its taps are read up front, so that the reads are in
-        // flight together and the MFMAs (in k_conv's order) wait on them once
+        // flight together and the MFMAs wait on them once
+        auto mma = [&](auto upc) __attribute__((always_inline)) {
+            constexpr bool UP = decltype(upc)::value;  // A holds half-resolution pixels
+            // halo rows j = 0 .. 5 of the wave's pixel rows; half-resolution
+            // rows (j + 1) / 2 of them, four in all
+            constexpr int kRows = UP ? 4 : 6;
+            int col = (wv & 1) * 16 + fr, grp = lane >> 4;
+            if (UP) asm volatile("" : "+v"(col), "+v"(grp));  // addresses formed here, not kept in registers
 #pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-            bf16x8 a[6], bw[3][BN / 16];
+            for (int dx = 0; dx < 3; ++dx) {
+                bf16x8 a[kRows], bw[3][BN / 16];
 #pragma unroll
-            for (int j = 0; j < 6; ++j)
-                a[j] = __builtin_bit_cast(
-                    bf16x8, *(const uint4*)&Hs[cofs((4 * (wv >> 1) + j) * HXX + (wv & 1) * 16 + fr + dx, lane >> 4)]);
+                for (int j = 0; j < kRows; ++j) {
+                    const int hx = col + dx;
+                    const int r = UP ? (2 * (wv >> 1) + j) * HXU + ((hx + 1) >> 1) : (4 * (wv >> 1) + j) * HXX + hx;
+                    a[j] = __builtin_bit_cast(bf16x8, *(const uint4*)&Hs[cofs(r, grp)]);
+                }
 #pragma unroll
-            for (int dy = 0; dy < 3; ++dy)
+                for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
-                for (int nb = 0; nb < BN / 16; ++nb)
-                    bw[dy][nb] = __builtin_bit_cast(
-                        bf16x8, *(const uint4*)&Ws[cofs((dy * 3 + dx) * BN + nb * 16 + fr, lane >> 4)]);
-            __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the MFMAs
+                    for (int nb = 0; nb < BN / 16; ++nb)
+                        bw[dy][nb] = __builtin_bit_cast(
+                            bf16x8, *(const uint4*)&Ws[cofs((dy * 3 + dx) * BN + nb * 16 + fr, lane >> 4)]);
+                __builtin_amdgcn_sched_barrier(0);  // keep the reads ahead of the MFMAs
 #pragma unroll
-            for (int dy = 0; dy < 3; ++dy)
+                for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
-                for (int nb = 0; nb < BN / 16; ++nb)
+                    for (int nb = 0; nb < BN / 16; ++nb)
 #pragma unroll
-                    for (int mt = 0; mt < 4; ++mt)
-                        acc[mt][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[dy][nb], a[mt + dy], acc[mt][nb], 0, 0, 0);
-        }
+                        for (int mt = 0; mt < 4; ++mt)
+                            acc[mt][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                bw[dy][nb], a[UP ? (mt + dy + 1) >> 1 : mt + dy], acc[mt][nb], 0, 0, 0);
+            }
+        };
+        if ((FUSE & kFuseUp) != 0 && HALF && c * CBK >= csplit) mma(std::true_type());
+        else mma(std::false_type());
         if (c == nchunk - 1)
-            conv_store<BN, FUSE>(acc, (const float*)(Ws + SH::kWUnits * 8), cur.n, cur.y0, cur.x0, cur.co0, wv, lane, H,
-                                 W, Y, ldy, Yf, ldyf, cstore, nullptr, 0, relu, P);
+            conv_store<BN, FUSE>(acc, Bsm, tr + wv * kTrans, mk, cur.n, cur.y0, cur.x0,
+                                 cur.co0, wv, lane, H, W, Y, ldy, Yf, ldyf, cstore, M, ldm, relu, P);
         if (!has_next) return false;
         i = ni;
         c = nc;
@@ -553,7 +658,7 @@ __global__ __launch_bounds__(TB2) void k_conv2(const uint16_t* __restrict__ X, i
 // (raw, two buffers: the next tile's loads run while this one is packed and
 // convolved); the threads pack them into the BF16 halo (channels 0-8; the
 // zero channel groups 2 and 3 are written once), then the MFMAs and the
-// epilogue are k_conv's: each output pixel gets the same MFMA sequence, so
+// epilogue are k_conv2's: each output pixel gets the same MFMA sequence, so
 // the outputs do not depend on the tiling.
 // Rows of the first layer's tiles.  16: one 8-wave block per CU (1.07 ms on
 // 128 x 512x512); 8 rows fit two 4-wave blocks per CU and were slower (1.31 ms).
@@ -577,6 +682,7 @@ __global__ __launch_bounds__(PackShape<TYP>::kThreads) void k_conv2_pack(const u
     __shared__ __attribute__((aligned(16))) float4 raw0[3 * kRawUnits];
     __shared__ __attribute__((aligned(16))) float4 raw1[3 * kRawUnits];
     __shared__ __attribute__((aligned(16))) uint16_t Hs[NH * CCLD];
+    __shared__ __attribute__((aligned(16))) uint16_t tr[PS::kWaves * kTrans];
     __shared__ __attribute__((aligned(16))) uint16_t Ws[SH::kWUnits * 8 + 2 * 64];  // + 64 FP32 biases (one per lane)
     const int tiles_x = (W + TX - 1) / TX, tiles_y = (H + TYP - 1) / TYP;
     const int n_tiles = N * tiles_x * tiles_y;
@@ -669,7 +775,7 @@ __global__ __launch_bounds__(PackShape<TYP>::kThreads) void k_conv2_pack(const u
         // __syncthreads' fence, which would wait for the loads into B too.
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (have_prev)
-            conv_store<BN, 0>(acc, Bsm, prev.n, prev.y0, prev.x0, 0, wv, lane, H, W, Y, ldy, nullptr, 0, cstore,
+            conv_store<BN, 0>(acc, Bsm, tr + wv * kTrans, nullptr, prev.n, prev.y0, prev.x0, 0, wv, lane, H, W, Y, ldy, nullptr, 0, cstore,
                               nullptr, 0, relu, nullptr);
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
@@ -706,7 +812,7 @@ __global__ __launch_bounds__(PackShape<TYP>::kThreads) void k_conv2_pack(const u
     };
     while (step(raw0, raw1) && step(raw1, raw0)) {
     }
-    conv_store<BN, 0>(acc, Bsm, prev.n, prev.y0, prev.x0, 0, wv, lane, H, W, Y, ldy, nullptr, 0, cstore, nullptr, 0,
+    conv_store<BN, 0>(acc, Bsm, tr + wv * kTrans, nullptr, prev.n, prev.y0, prev.x0, 0, wv, lane, H, W, Y, ldy, nullptr, 0, cstore, nullptr, 0,
                       relu, nullptr);
 }
 
@@ -1110,29 +1216,16 @@ template <class T> T* dalloc(size_t n) {
 // ---------------------------------------------------------------- launchers
 // One 3x3 convolution: output tiles of 16 channels when at most 16 are
 // stored (the RGB output layer), 64 when 64 divides them, else 32.
-// Persistent grid of k_conv<BN>: the blocks that are resident at once (from
-// its LDS and registers), or fewer when there are fewer items.
-template <int BN, int FUSE>
-unsigned conv_grid(unsigned n_items) {
-    static unsigned resident = 0;
-    if (!resident) {
-        int dev = 0, cus = 256, nb = 0;
-        KF_CHECK(hipGetDevice(&dev));
-        KF_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        KF_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_conv<BN, FUSE>, TB, 0));
-        resident = (unsigned)std::max(nb, 1) * (unsigned)cus;
-    }
-    return std::min(n_items, resident);
-}
-
-template <int BN, int FUSE>
+// Persistent grid of k_conv2: the blocks that are resident at once (from its
+// LDS and registers), or fewer when there are fewer items.
+template <int BN, int FUSE, bool RES>
 unsigned conv2_grid(unsigned n_items) {
     static unsigned resident = 0;
     if (!resident) {
         int dev = 0, cus = 256, nb = 0;
         KF_CHECK(hipGetDevice(&dev));
         KF_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        KF_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_conv2<BN, FUSE>, TB2, 0));
+        KF_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, (k_conv2<BN, FUSE, RES>), TB2, 0));
         resident = (unsigned)std::max(nb, 1) * (unsigned)cus;
     }
     return std::min(n_items, resident);
@@ -1169,7 +1262,7 @@ void conv_launch(const uint16_t* X, int ldx, int Cin, const uint16_t* Wt, const 
         throw Error("conv: bad upsampled input");
     if (fz.P && (H % 2 || W % 2 || !Y || Yf || cstore != Cout || cstore % 16))
         throw Error("conv: bad pooled output");
-    const unsigned tiles = (unsigned)N * blocks(H, TY) * blocks(W, TX);
+    const unsigned tiles = (unsigned)N * blocks(H, 8) * blocks(W, TX);  // a bound twice the kernel's tiles
     if ((uint64_t)tiles * blocks(cstore, 16) >= (1u << 31)) throw Error("conv: too many tiles");
     // the kernel indexes pixels, weights and rows of a tile with 32-bit integers
     const uint64_t ld_max = std::max<uint64_t>(std::max(ldy, ldyf), std::max(ldm, ldx));
@@ -1181,59 +1274,47 @@ void conv_launch(const uint16_t* X, int ldx, int Cin, const uint16_t* Wt, const 
     if (fuse && (M || Yf || cstore <= 16)) throw Error("conv: fusions write plain BF16 outputs of > 16 channels");
     if (fz.pk.rgba && (Cin != CBK || Cout > 32 || fz.pk.h > H || fz.pk.w > W || fz.pk.h < 1 || fz.pk.w < 1))
         throw Error("conv: bad packed input");
-    const int flags = fuse | (Yf ? kOutF32 : 0) | (M ? kMask : 0);
-    auto go = [&](auto bn, auto fl) {
-        constexpr int BN = decltype(bn)::value, F = decltype(fl)::value;
-        const unsigned n = tiles * blocks(cstore, BN);
-        k_conv<BN, F><<<conv_grid<BN, F>(n), TB, 0, st>>>(X, ldx, Cin, Wt, bias, Cout, N, H, W, Y, ldy, Yf, ldyf,
-                                                         cstore, M, ldm, relu, (int)n, fz.X2, fz.ldx2, fz.csplit,
-                                                         fz.P);
-    };
     using I16 = std::integral_constant<int, 16>;
     using I32 = std::integral_constant<int, 32>;
     using I64 = std::integral_constant<int, 64>;
-    auto outs = [&](auto bn) {  // the output kinds of an unfused convolution
-        switch (flags) {
-            case 0: go(bn, std::integral_constant<int, 0>()); break;
-            case kOutF32: go(bn, std::integral_constant<int, kOutF32>()); break;
-            case kMask: go(bn, std::integral_constant<int, kMask>()); break;
-            default: go(bn, std::integral_constant<int, kOutF32 | kMask>()); break;
-        }
-    };
     auto go2 = [&](auto bn, auto fl) {
         constexpr int BN = decltype(bn)::value, F = decltype(fl)::value;
-        const unsigned n = (unsigned)N * blocks(H, TY2) * blocks(W, TX) * blocks(cstore, BN);
-        k_conv2<BN, F><<<conv2_grid<BN, F>(n), TB2, 0, st>>>(X, ldx, Cin, Wt, bias, Cout, N, H, W, Y, ldy, Yf, ldyf,
-                                                            cstore, relu, (int)n, fz.X2, fz.ldx2, fz.csplit, fz.P);
+        const unsigned tiles2 = (unsigned)N * blocks(H, TY2) * blocks(W, TX), n = tiles2 * blocks(cstore, BN);
+        const ConvDiv div{FastDiv(tiles2), FastDiv(blocks(W, TX)), FastDiv(blocks(H, TY2))};
+        auto run = [&](auto res) {
+            constexpr bool RES = decltype(res)::value;
+            k_conv2<BN, F, RES><<<conv2_grid<BN, F, RES>(n), TB2, 0, st>>>(X, ldx, Cin, Wt, bias, Cout, H, W, Y, ldy, Yf,
+                                                                          ldyf, cstore, M, ldm, relu, (int)n, fz.X2,
+                                                                          fz.ldx2, fz.csplit, fz.P, (int)tiles2, div);
+        };
+        if constexpr (BN == 32) {
+            if (Cin <= kRes2 * CBK) run(std::true_type());
+            else run(std::false_type());
+        } else {
+            run(std::false_type());
+        }
     };
-    // k_conv2 takes the plain, upsampled-input and pooled-output layers of
-    // more than 16 output channels, 64 per item where they divide the output
-    // (twice the MFMAs per staged halo), and the FP32 output layer (16 per
-    // item); k_conv2_pack the packed first layer; k_conv the masked data
-    // gradients and the BF16 layers of at most 16 outputs.  (Keeping the
-    // 32-channel full-resolution layers on k_conv, which had looked faster
-    // for two of them under the profiler, made the whole denoise of
-    // 128 x 512x512 slower: 14.16-14.18 against 13.96-14.07 ms.)
-    if (!Yf && !M && !fz.pk.rgba && cstore > 16) {
-        const bool wide = cstore % 64 == 0;
+    // 64 output channels per item where they divide the output (twice the
+    // MFMAs per staged halo), but 32 for masked data gradients, whose mask
+    // needs the registers; 16 for the FP32 output layer.
+    if (fuse == kFusePack) {  // 32 inputs, at most 32 outputs: one weight set
+        constexpr int TYP = kPackRows;
+        const unsigned n = (unsigned)N * blocks(H, TYP) * blocks(W, TX);
+        k_conv2_pack<TYP><<<conv2_pack_grid<TYP>(n), PackShape<TYP>::kThreads, 0, st>>>(Wt, bias, Cout, N, H, W, Y, ldy,
+                                                                                      cstore, relu, (int)n, fz.pk);
+    } else if (Yf) {
+        if (cstore > 16 || M) throw Error("conv: FP32 output of at most 16 channels, unmasked");
+        go2(I16(), std::integral_constant<int, kOutF32>());
+    } else if (M) {
+        go2(I32(), std::integral_constant<int, kMask>());
+    } else {
         auto pick = [&](auto fl) {
-            if (wide) go2(I64(), fl);
+            if (cstore % 64 == 0) go2(I64(), fl);
             else go2(I32(), fl);
         };
         if (fuse == kFuseUp) pick(std::integral_constant<int, kFuseUp>());
         else if (fuse == kFusePool) pick(std::integral_constant<int, kFusePool>());
         else pick(std::integral_constant<int, 0>());
-    } else if (cstore <= 16 && flags == kOutF32) {
-        go2(I16(), std::integral_constant<int, kOutF32>());
-    } else if (cstore <= 16) {
-        outs(I16());
-    } else if (fuse == kFusePack) {  // 32 inputs, at most 32 outputs: one weight set
-        constexpr int TYP = kPackRows;
-        const unsigned n = (unsigned)N * blocks(H, TYP) * blocks(W, TX);
-        k_conv2_pack<TYP><<<conv2_pack_grid<TYP>(n), PackShape<TYP>::kThreads, 0, st>>>(Wt, bias, Cout, N, H, W, Y, ldy,
-                                                                                      cstore, relu, (int)n, fz.pk);
-    } else {
-        outs(I32());  // masked data gradient
     }
     KF_CHECK(hipGetLastError());
 }

@@ -56,6 +56,28 @@ def test_conv_backward(gpu, cin, cout, h, w):
     assert np.allclose(db, rdb, rtol=1e-5, atol=1e-4)
 
 
+# Tiles of the 8-wave kernel, 32 x 16 pixels: whole ones stored 16 bytes per
+# lane, inside ones loaded without bounds tests, ragged ones of each; one to
+# five input chunks (the weights of up to three stay in LDS), several blocks
+# of output channels, a ragged one among them.  Small integers, so that every
+# sum is exact and the outputs are the reference's, rounded once.
+@pytest.mark.parametrize("cin,cout,n,h,w", [(32, 32, 3, 16, 32), (96, 32, 1, 49, 97), (128, 32, 1, 33, 65),
+                                            (64, 64, 2, 48, 96), (96, 96, 1, 50, 100), (32, 40, 2, 20, 40),
+                                            (160, 128, 1, 34, 66), (32, 32, 5, 17, 33)])
+def test_conv_tiles(gpu, cin, cout, n, h, w):
+    rng = np.random.default_rng(cin + cout + h)
+    x = rng.integers(-2, 3, (n, h, w, cin)).astype(np.float64)
+    wt = rng.integers(-1, 2, (9, cout, cin)).astype(np.float64)
+    b = rng.integers(-3, 4, cout).astype(np.float32)
+    y = conv_forward(x, wt, b, relu=True)
+    assert np.array_equal(y, U.round_bf16(np.maximum(U.conv_fwd(x, wt, b.astype(np.float64)), 0)))
+    if cout % 32 == 0:
+        dy = rng.integers(-2, 3, (n, h, w, cout)).astype(np.float64)
+        dx, _, _ = conv_backward(x, wt, dy, mask_by_x=True)
+        rdx, _, _ = U.conv_bwd(x, wt, dy)
+        assert np.array_equal(dx, U.round_bf16(rdx * (x > 0)))
+
+
 # Strips of the weight-gradient kernel: 32 pixels wide and at least 4 rows
 # high, two pixels per register.  Widths around a strip and a pixel pair,
 # heights around one strip, and (last) a layer whose waves take several strips.
