@@ -116,6 +116,8 @@ Scene::~Scene() {
     if (h_vstage) (void)hipHostFree(h_vstage);
     if (vstage_ev) (void)hipEventDestroy(vstage_ev);
     if (h_stage) (void)hipHostFree(h_stage);
+    if (trace.h_pin) (void)hipHostFree(trace.h_pin);
+    release(trace.d_cnt); release(trace.d_buf);
     if (stage_ev) (void)hipEventDestroy(stage_ev);
     d_env_info = nullptr;  // points into d_tex_info, not an allocation of its own
     release(d_inst_src); release(d_ilo); release(d_ihi); release(d_glo); release(d_ghi); release(d_refit); release(d_tex); release(d_tex_info); release(d_srgb);

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -226,6 +227,14 @@ struct Scene {
     kf_active_lights al{};
     float build_ms = 0.f;
     std::vector<hipEvent_t> events;
+    // Workspace of the fixed ray batches (trace.hip), one call at a time
+    struct Trace {
+        std::mutex mu;
+        unsigned long long* d_cnt = nullptr;
+        uint8_t* d_buf = nullptr;   // rays and results of larger batches
+        uint8_t* h_pin = nullptr;   // pinned: overflow flag, rays and results of small batches
+        size_t dev_cap = 0, pin_cap = 0;
+    } trace;
 
     SceneView view() const;
     ~Scene();

@@ -7,6 +7,7 @@
 #include "traverse.h"
 
 #include <algorithm>
+#include <cstring>
 #include <mutex>
 #include <string>
 
@@ -37,7 +38,7 @@ KF_DEV void ray_of(const SceneView& S, const kf_ray& r, uint32_t q, TRay& t) {
 template <bool COUNT>
 __global__ __launch_bounds__(TB) void k_closest(SceneView S, const kf_ray* __restrict__ rays, uint32_t n,
                                                 kf_hit* __restrict__ hits, unsigned long long* __restrict__ cnt,
-                                                uint32_t refill) {
+                                                unsigned long long* __restrict__ flag, uint32_t refill) {
     uint32_t ovf = 0;
     TCount tot{0, 0, 0, 0};
     auto load = [&](uint32_t q, TRay& t) __attribute__((always_inline)) { ray_of(S, rays[q], q, t); };
@@ -56,28 +57,36 @@ __global__ __launch_bounds__(TB) void k_closest(SceneView S, const kf_ray* __res
         atomicAdd(&cnt[0], (unsigned long long)tot.nodes);
         atomicAdd(&cnt[1], (unsigned long long)tot.tris);
     }
-    if (ovf) atomicAdd(&cnt[2], 1ull);
+    if (ovf) *flag = 1ull;
 }
 
 __global__ __launch_bounds__(TB) void k_any(SceneView S, const kf_ray* __restrict__ rays, uint32_t n,
                                             uint8_t* __restrict__ occ, unsigned long long* __restrict__ cnt,
-                                            uint32_t refill) {
+                                            unsigned long long* __restrict__ flag, uint32_t refill) {
     uint32_t ovf = 0;
     TCount tot{0, 0, 0, 0};
     auto load = [&](uint32_t q, TRay& t) __attribute__((always_inline)) { ray_of(S, rays[q], q, t); };
     auto store = [&](uint32_t q, THit, bool found) __attribute__((always_inline)) { occ[q] = found ? 1 : 0; };
     trace_persistent<true, false>(S, n, cnt + kTraceChunks, refill, kGrab, false, load, store, ovf, tot);
-    if (ovf) atomicAdd(&cnt[2], 1ull);
+    if (ovf) *flag = 1ull;
 }
 
 // Persistent grid: exactly the blocks of `kernel` that are resident at once.
 template <class Kernel>
-unsigned trace_grid(Kernel kernel) {
+unsigned resident_blocks(Kernel kernel) {
     int dev = 0, cus = 256, nb = 0;
     KF_CHECK(hipGetDevice(&dev));
     KF_CHECK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
     KF_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, TB, 0));
     return (unsigned)std::max(nb, 1) * (unsigned)cus;
+}
+unsigned closest_grid() {
+    static const unsigned g = resident_blocks(k_closest<false>);
+    return g;
+}
+unsigned any_grid() {
+    static const unsigned g = resident_blocks(k_any);
+    return g;
 }
 
 // Streaming copy for the achievable-bandwidth figure: each block copies one
@@ -141,10 +150,82 @@ extern "C" int kf_bench_copy(uint64_t bytes, int iters, float* gbps) {
 }
 
 namespace {
-unsigned long long* trace_counters() {
-    static unsigned long long* c = nullptr;
-    if (!c) KF_CHECK(hipMalloc((void**)&c, kTraceCnt * sizeof(unsigned long long)));
-    return c;
+// A fixed batch through the scene's workspace (Scene::trace), one call at a
+// time per scene.  Up to kDirectRays rays the kernel reads the rays from and
+// writes the results to pinned host memory itself: the copies of a batch of
+// 4096 rays took as long as its traversal (whole calls 145 -> 105 us, 72 of
+// them the kernel).  With copies and with direct access, closest hits: 32768
+// rays 206 and 139 us, 131072 rays 478 and 395, 262144 rays 836 and 702; any
+// hit 162 and 117, 272 and 237, 414 and 407.  The line bounds a scene's pinned
+// memory at 7 MB.  Beyond it the device buffers are kept up to kKeepBytes, and
+// allocated for the call above that.
+constexpr uint32_t kDirectRays = 131072;
+constexpr size_t kKeepBytes = (size_t)64 << 20;
+constexpr size_t kCntBytes = (kTraceCnt * sizeof(unsigned long long) + 255) / 256 * 256;
+
+struct Temp {  // device memory of one call
+    uint8_t* p = nullptr;
+    ~Temp() {
+        if (p) (void)hipFree(p);
+    }
+};
+
+unsigned long long* trace_counters(Scene& s) {
+    if (!s.trace.d_cnt) KF_CHECK(hipMalloc((void**)&s.trace.d_cnt, kCntBytes));
+    return s.trace.d_cnt;
+}
+
+template <class Out, class Launch>
+void trace_batch(const char* name, Scene& s, const kf_ray* rays, uint32_t n, Out* out, Launch launch) {
+    hipStream_t st = stream();
+    std::lock_guard<std::mutex> lk(s.trace.mu);
+    const size_t rb = ((size_t)n * sizeof(kf_ray) + 255) / 256 * 256, ob = (size_t)n * sizeof(Out);
+    unsigned long long* c = trace_counters(s);
+    KF_CHECK(hipMemsetAsync(c, 0, kTraceCnt * sizeof(unsigned long long), st));
+    unsigned long long failed = 0;
+    if (n <= kDirectRays) {
+        const size_t need = 256 + rb + ob;
+        if (need > s.trace.pin_cap) {
+            if (s.trace.h_pin) KF_CHECK(hipHostFree(s.trace.h_pin));
+            s.trace.h_pin = nullptr;
+            s.trace.pin_cap = 0;
+            KF_CHECK(hipHostMalloc((void**)&s.trace.h_pin, need, hipHostMallocDefault));
+            s.trace.pin_cap = need;
+        }
+        unsigned long long* flag = (unsigned long long*)s.trace.h_pin;
+        kf_ray* r = (kf_ray*)(s.trace.h_pin + 256);
+        Out* o = (Out*)(s.trace.h_pin + 256 + rb);
+        *flag = 0ull;
+        std::memcpy(r, rays, (size_t)n * sizeof(kf_ray));
+        launch(r, o, c, flag, st);
+        KF_CHECK(hipGetLastError());
+        KF_CHECK(hipStreamSynchronize(st));
+        failed = *(volatile unsigned long long*)flag;
+        std::memcpy(out, o, ob);
+    } else {
+        Temp tmp;
+        uint8_t* d = nullptr;
+        if (rb + ob > kKeepBytes) {
+            KF_CHECK(hipMalloc((void**)&tmp.p, rb + ob));
+            d = tmp.p;
+        } else {
+            if (rb + ob > s.trace.dev_cap) {
+                if (s.trace.d_buf) KF_CHECK(hipFree(s.trace.d_buf));
+                s.trace.d_buf = nullptr;
+                s.trace.dev_cap = 0;
+                KF_CHECK(hipMalloc((void**)&s.trace.d_buf, rb + ob));
+                s.trace.dev_cap = rb + ob;
+            }
+            d = s.trace.d_buf;
+        }
+        KF_CHECK(hipMemcpyAsync(d, rays, (size_t)n * sizeof(kf_ray), hipMemcpyHostToDevice, st));
+        launch((const kf_ray*)d, (Out*)(d + rb), c, c + 2, st);
+        KF_CHECK(hipGetLastError());
+        KF_CHECK(hipMemcpyAsync(out, d + rb, ob, hipMemcpyDeviceToHost, st));
+        KF_CHECK(hipMemcpyAsync(&failed, c + 2, sizeof(failed), hipMemcpyDeviceToHost, st));
+        KF_CHECK(hipStreamSynchronize(st));
+    }
+    if (failed) throw Error(std::string(name) + ": traversal stack overflow");
 }
 }  // namespace
 
@@ -152,23 +233,10 @@ extern "C" int kf_trace_closest(kf_scene* s, const kf_ray* rays, uint32_t n, kf_
     try {
         if (!s || (n && (!rays || !hits))) throw Error("kf_trace_closest: null argument");
         if (n == 0) return 0;
-        hipStream_t st = stream();
-        kf_ray* d_r = nullptr;
-        kf_hit* d_h = nullptr;
-        KF_CHECK(hipMalloc((void**)&d_r, n * sizeof(kf_ray)));
-        KF_CHECK(hipMalloc((void**)&d_h, n * sizeof(kf_hit)));
-        unsigned long long* c = trace_counters();
-        KF_CHECK(hipMemsetAsync(c, 0, kTraceCnt * sizeof(unsigned long long), st));
-        KF_CHECK(hipMemcpyAsync(d_r, rays, n * sizeof(kf_ray), hipMemcpyHostToDevice, st));
-        k_closest<false><<<trace_grid(k_closest<false>), TB, 0, st>>>(s->view(), d_r, n, d_h, c, traversal_refill());
-        KF_CHECK(hipGetLastError());
-        unsigned long long h[4];
-        KF_CHECK(hipMemcpyAsync(hits, d_h, n * sizeof(kf_hit), hipMemcpyDeviceToHost, st));
-        KF_CHECK(hipMemcpyAsync(h, c, sizeof(h), hipMemcpyDeviceToHost, st));
-        KF_CHECK(hipStreamSynchronize(st));
-        KF_CHECK(hipFree(d_r));
-        KF_CHECK(hipFree(d_h));
-        if (h[2]) throw Error("kf_trace_closest: traversal stack overflow");
+        trace_batch("kf_trace_closest", *s, rays, n, hits,
+                    [&](const kf_ray* r, kf_hit* h, unsigned long long* c, unsigned long long* flag, hipStream_t st) {
+                        k_closest<false><<<closest_grid(), TB, 0, st>>>(s->view(), r, n, h, c, flag, traversal_refill());
+                    });
         return 0;
     } catch (const std::exception& e) {
         set_error(e.what());
@@ -180,23 +248,10 @@ extern "C" int kf_trace_any(kf_scene* s, const kf_ray* rays, uint32_t n, uint8_t
     try {
         if (!s || (n && (!rays || !occluded))) throw Error("kf_trace_any: null argument");
         if (n == 0) return 0;
-        hipStream_t st = stream();
-        kf_ray* d_r = nullptr;
-        uint8_t* d_o = nullptr;
-        KF_CHECK(hipMalloc((void**)&d_r, n * sizeof(kf_ray)));
-        KF_CHECK(hipMalloc((void**)&d_o, n));
-        unsigned long long* c = trace_counters();
-        KF_CHECK(hipMemsetAsync(c, 0, kTraceCnt * sizeof(unsigned long long), st));
-        KF_CHECK(hipMemcpyAsync(d_r, rays, n * sizeof(kf_ray), hipMemcpyHostToDevice, st));
-        k_any<<<trace_grid(k_any), TB, 0, st>>>(s->view(), d_r, n, d_o, c, traversal_refill());
-        KF_CHECK(hipGetLastError());
-        unsigned long long h[4];
-        KF_CHECK(hipMemcpyAsync(occluded, d_o, n, hipMemcpyDeviceToHost, st));
-        KF_CHECK(hipMemcpyAsync(h, c, sizeof(h), hipMemcpyDeviceToHost, st));
-        KF_CHECK(hipStreamSynchronize(st));
-        KF_CHECK(hipFree(d_r));
-        KF_CHECK(hipFree(d_o));
-        if (h[2]) throw Error("kf_trace_any: traversal stack overflow");
+        trace_batch("kf_trace_any", *s, rays, n, occluded,
+                    [&](const kf_ray* r, uint8_t* o, unsigned long long* c, unsigned long long* flag, hipStream_t st) {
+                        k_any<<<any_grid(), TB, 0, st>>>(s->view(), r, n, o, c, flag, traversal_refill());
+                    });
         return 0;
     } catch (const std::exception& e) {
         set_error(e.what());
@@ -264,7 +319,7 @@ extern "C" int kf_trace_closest_noalloc(kf_scene* s, const kf_ray* rays, uint32_
         kf_hit* d_h = (kf_hit*)(base + kNoAllocCntBytes + kNoAllocRayBytes);
         k_zero_u64<<<1, 64, 0, st>>>(c, kTraceCnt);  // the last call's counters stay in the scratch
         KF_CHECK(hipMemcpyAsync(d_r, rays, n * sizeof(kf_ray), hipMemcpyHostToDevice, st));
-        k_closest<false><<<trace_grid(k_closest<false>), TB, 0, st>>>(s->view(), d_r, n, d_h, c, traversal_refill());
+        k_closest<false><<<closest_grid(), TB, 0, st>>>(s->view(), d_r, n, d_h, c, c + 2, traversal_refill());
         KF_CHECK(hipGetLastError());
         unsigned long long h[4];
         KF_CHECK(hipMemcpyAsync(hits, d_h, n * sizeof(kf_hit), hipMemcpyDeviceToHost, st));
@@ -284,13 +339,14 @@ extern "C" int kf_trace_closest_device(kf_scene* s, const kf_ray* d_rays, uint32
         if (!s) throw Error("kf_trace_closest_device: null scene");
         if (n == 0) return 0;
         hipStream_t st = stream();
-        unsigned long long* c = trace_counters();
+        std::lock_guard<std::mutex> lk(s->trace.mu);
+        unsigned long long* c = trace_counters(*s);
         KF_CHECK(hipMemsetAsync(c, 0, kTraceCnt * sizeof(unsigned long long), st));
         hipEvent_t e0, e1;
         KF_CHECK(hipEventCreate(&e0));
         KF_CHECK(hipEventCreate(&e1));
         KF_CHECK(hipEventRecord(e0, st));
-        k_closest<false><<<trace_grid(k_closest<false>), TB, 0, st>>>(s->view(), d_rays, n, d_hits, c, traversal_refill());
+        k_closest<false><<<closest_grid(), TB, 0, st>>>(s->view(), d_rays, n, d_hits, c, c + 2, traversal_refill());
         KF_CHECK(hipEventRecord(e1, st));
         KF_CHECK(hipGetLastError());
         KF_CHECK(hipEventSynchronize(e1));

@@ -10,6 +10,7 @@
   expected); rgba running mean, albedo and normal targets likewise.
 """
 import math
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -83,6 +84,32 @@ def test_batch_sizes_give_the_same_hits(gpu, n):
     if n == 65:
         ref = oracle.Scene(scenes.config1().data).trace_closest(base)
         assert np.array_equal(hits["inst"], ref["inst"]) and np.array_equal(hits["prim"], ref["prim"])
+
+
+# Batches around the size up to which rays and hits stay in pinned memory, and
+# beyond what a scene keeps on the device, in an order that grows, shrinks and
+# skips its workspace; from several threads at once the same hits.
+@pytest.mark.parametrize("sizes", [(131072, 131073, 100, 131072), (1250000, 200000, 5), (3, 131073, 4096, 1)])
+def test_trace_workspace(gpu, sizes):
+    gs = GpuScene(scenes.config1().data)
+    rng = np.random.default_rng(len(sizes))
+    base = np.zeros(997, abi.RAY_DTYPE)
+    base["org"] = rng.uniform(-3, 3, (997, 3)) + (0.0, 3.0, 0.0)
+    d = rng.normal(size=(997, 3))
+    base["dir"] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    base["tmin"], base["tmax"] = 0.001, 1e4
+    hits, occ = gs.trace_closest(base), gs.trace_any(base)
+    for n in sizes:
+        idx = np.arange(n) % 997
+        assert gs.trace_closest(base[idx]).tobytes() == hits[idx].tobytes()
+        assert np.array_equal(gs.trace_any(base[idx]), occ[idx])
+
+    def some(k):
+        idx = (np.arange(min(sizes[k % len(sizes)], 20000)) + 31 * k) % 997
+        return gs.trace_closest(base[idx]).tobytes() == hits[idx].tobytes() and np.array_equal(gs.trace_any(base[idx]), occ[idx])
+
+    with ThreadPoolExecutor(4) as pool:
+        assert all(pool.map(some, range(24)))
 
 
 # Triangles one behind the other whose boxes every ray meets: three children
