@@ -944,9 +944,11 @@ KF_DEV bool shade_path(const SceneView& S, const Frame& F, const DevLights* __re
 // the vertices and the material, one after another), so it is held to 128
 // registers for 4 waves per SIMD: 12 spilled registers cost less than the
 // fourth wave gains (489 -> 464 us per launch on the 1080p frame).  With
-// inline shadow rays it keeps its registers (2 waves).
+// inline shadow rays it takes 182 registers or, with 4 spilled, the 168 of
+// three waves: 4 spp of 640x360 with a soft light, k_tail the same, 2.16 ->
+// 1.89 ms (four waves, 72 spilled: 1.91).
 template <bool NEE_INLINE>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(NEE_INLINE ? 1 : 4))) void k_shade(SceneView S, Frame F, const DevLights* __restrict__ LT, int bounce,
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(NEE_INLINE ? 3 : 4))) void k_shade(SceneView S, Frame F, const DevLights* __restrict__ LT, int bounce,
                                               const uint32_t* __restrict__ queue, float4* __restrict__ ray_o,
                                               float4* __restrict__ ray_d, const float4* __restrict__ thr,
                                               const float4* __restrict__ hit, const uint32_t* __restrict__ hit_prim,
@@ -1129,7 +1131,12 @@ __global__ __launch_bounds__(TB) void k_connect(Frame F, int bounce, const uint3
 // for the slowest ray of each launch; here a launch lasts as long as the
 // longest remaining path.  The random streams and light order are those of
 // the wavefront kernels, so the radiance is the same.
-__global__ __launch_bounds__(TB) void k_tail(SceneView S, Frame F, const DevLights* __restrict__ LT, int b0,
+// Bound by latency, so held to three waves per SIMD (168 registers instead of
+// 178, nothing spilled; four waves spill 35 and take 1-2 % longer on a 256x256
+// frame), with the traversal's stack in LDS: in private memory every step's
+// stack access was a memory access as well (256x256 frame at 4 spp 884 -> 864
+// us, 640x360 with a soft light 2.22 -> 2.16 ms).
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(3))) void k_tail(SceneView S, Frame F, const DevLights* __restrict__ LT, int b0,
                                              const uint32_t* __restrict__ queue, float4* __restrict__ ray_o,
                                              float4* __restrict__ ray_d, float4* __restrict__ thr,
                                              float4* __restrict__ col, float4* __restrict__ hit,

@@ -590,13 +590,22 @@ struct Trav {
     }
 };
 
+// This thread's column of the block's stack ring (blocks of kRingThreads).
+KF_DEV lds_u32* ring_column() {
+    __shared__ uint32_t ring[kRing * kRingThreads];
+    return (lds_u32*)(ring + threadIdx.x);
+}
+
 // Whole query for one lane (used where rays are generated inside a kernel).
 template <bool ANY, bool COUNT>
 KF_DEV bool traverse(const SceneView& S, uint32_t root, v3 o, v3 d, float tmin, float tmax, bool use_alpha,
                      uint32_t alpha_seed, THit& best, TCount& cnt, uint32_t& overflow) {
     const TravScene TS(S);
     Trav<ANY, COUNT> T;
-    PrivStack stk;
+    uint32_t spill[kStack];
+    RingStack stk;
+    stk.ring = ring_column();
+    stk.spill = spill;
     T.reset();
     TRay r;
     r.o = o;
@@ -657,10 +666,9 @@ KF_DEV void trace_persistent(const SceneView& S, uint32_t n, unsigned long long*
     const TravScene TS(S);
     Trav<ANY, COUNT> T;
     T.reset();
-    __shared__ uint32_t ring[kRing * kRingThreads];
     uint32_t spill[kStack];
     RingStack stk;
-    stk.ring = (lds_u32*)(ring + threadIdx.x);
+    stk.ring = ring_column();
     stk.spill = spill;
     uint64_t live = 0;  // lanes that hold a query
     uint32_t payload = 0;
