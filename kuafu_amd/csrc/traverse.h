@@ -404,7 +404,7 @@ struct Trav {
         // of an instance record's root node; lines 7-9 of an instance record,
         // its transform.  Each lane loads only its record's lines: the vector
         // L1 serves one lane's line per cycle, so that ten loads by all 64
-        // lanes kept it busy 81 % of the time beside vector ALUs at 76 % (2 M
+        // lanes kept it busy 87 % of the time beside vector ALUs at 82 % (2 M
         // rays, 256 icospheres).  The empty asm needs all results, which keeps the
         // compiler from sinking parts of the fetch into the kind-specific
         // code below (each sunk load would cost the wave another memory round
