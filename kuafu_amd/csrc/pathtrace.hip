@@ -1518,19 +1518,23 @@ uint32_t default_batch(uint32_t spp, uint32_t WH) {
 // They run each path as one chain of rays, so they win where a bounce's
 // launches cannot fill the chip and last as long as their slowest ray, and
 // where Russian roulette has thinned the paths; measured over three scenes
-// at 16 k - 30 M paths per batch, never / from bounce 1 / 2 / 3 / 5:
-//   262 k paths, 256 icospheres   2.25 / 1.45 / 1.69 / 1.83 / 2.23 ms
-//   1 M paths, projector          2.31 / 2.43 / 2.03 / 2.02 / 2.18 ms
-//   4 M paths, 256 icospheres     4.57 / 5.08 / 3.98 / 3.77 / 4.25 ms
-//   17 M paths, 256 icospheres    8.60 / 14.7 / 10.4 / 8.56 / 8.04 ms
+// at 16 k - 13 M paths per batch, from bounce 1 / 2 / 3 / 5:
+//   512 k paths, 256 icospheres    1.56 / 1.70 / 1.82 / 2.15 ms
+//   786 k paths, 256 icospheres    1.93 / 1.96 / 2.09 / 2.45 ms, projector 1.88 / 1.81
+//   922 k paths, projector         1.99 / 1.83 / 1.93 / 2.22 ms
+//   2.6 M paths, 256 icospheres    3.25 / 2.78 / 2.92 / 3.36 ms
+//   4.1 M paths, 256 icospheres    5.32 / 4.26 / 4.12 / 4.62 ms, 9 spheres 5.12 / 3.80 / 3.94 / 4.07
+//   6.3 M paths, projector         9.12 / 6.46 / 6.17 / 6.46 ms
+//   17 M paths, 256 icospheres     14.7 / 10.4 / 8.56 / 8.04 ms
 // The shadow rays of all lights are part of a path's chain.  256 k paths on
-// the config-1 spheres, never / from bounce 1 / 2: 1.48 / 1.07 / 1.09 ms with
-// 2 lights, 1.63 / 1.38 / 1.33 with 3, 1.69 / 1.71 / 1.61 with 4, 1.99 / 2.47
-// / 2.23 with 8, 3.18 / 7.84 / 7.48 with 32.
+// the config-1 spheres, never / from bounce 1 / 2 (before the tail ran three
+// waves per SIMD): 1.48 / 1.07 / 1.09 ms with 2 lights, 1.63 / 1.38 / 1.33 with
+// 3, 1.69 / 1.71 / 1.61 with 4, 1.99 / 2.47 / 2.23 with 8, 3.18 / 7.84 / 7.48
+// with 32; the lines for three and four lights are those of that time.
 uint32_t default_tail(const kf_push_constants& pc, uint64_t paths, uint32_t lights, uint32_t nb) {
     if (lights > 4) return nb;
-    if (paths <= (3u << 17) && lights <= 3) return 1;
-    if (paths <= (3u << 19)) return 2;
+    if (paths <= (lights <= 2 ? 3u << 18 : 3u << 17) && lights <= 3) return 1;
+    if (paths <= (lights <= 2 ? 1u << 22 : 3u << 19)) return 2;
     if (!pc.russian_roulette) return nb;
     return paths <= (8u << 20) ? 3 : pc.rr_min_bounces + 1;
 }
