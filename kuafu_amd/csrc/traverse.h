@@ -8,8 +8,9 @@
 //   * watertight test of Woo, Benthin & Wald (JCGT 2013), double-precision
 //     fallback when an edge function is exactly zero;
 //   * accept t in [tmin, tmax]; closest hit = smallest t, ties broken by the
-//     smaller (instance, primitive) pair, so the result does not depend on the
-//     BVH or the visiting order;
+//     smaller (instance, primitive) pair.  Hits a few roundings of t apart may
+//     cull each other (ChildOrder), so the visiting order is part of the result:
+//     it is fixed by the tree and the ray;
 //   * hit kind front-facing iff dot(d_obj, cross(v1 - v0, v2 - v0)) < 0;
 //   * the object-space ray is (W2O * (o,1), W2O * (d,0)), t is shared.
 #pragma once
@@ -276,6 +277,61 @@ KF_DEV uint32_t env_root_item(const SceneView& S, uint32_t e) {
     return S.tlas_root == kEmptyRef ? kEmptyItem : root_item(S.tlas_root);
 }
 
+// The four children of a node in the order of their keys, by the sorting
+// network (0,1)(2,3)(0,2)(1,3)(1,2).
+// Closest hits exchange two children on their distances alone, so that the
+// order follows from the ray and the children's places in the node.  Equal
+// distances are the usual case (every box around a ray's origin is entered at
+// tmin), and the order among them can decide a hit: the culling bound does not
+// cover the rounding of a triangle's own distance, so of two surfaces hit
+// within a few roundings of each other the first one found may drop the other.
+// With the item as a second key, as below, that order followed the numbering
+// of nodes and instances: 643 of 1 M rays from within 5 mm of bodies' feet got
+// another hit (distances up to 3.4e-7 m apart over a ground of 4 m).  The
+// selects cost 2 % on a 256x256 frame (866 -> 883 us), elsewhere below 1 %.
+// An any-hit query is the same in every order.  It sorts (distance, item) as
+// one 64-bit float, an exchange a min and a max instead of a comparison and
+// selects (no key is a NaN: the high word is a float).
+template <bool ANY> struct ChildOrder {
+    uint32_t item[4];
+    KF_DEV ChildOrder(const float (&k)[4], const uint32_t (&it)[4]) {
+        float key[4] = {k[0], k[1], k[2], k[3]};
+        for (int c = 0; c < 4; ++c) item[c] = it[c];
+        auto cx = [&](int i, int j) __attribute__((always_inline)) {
+            const bool sw = key[j] < key[i];
+            const float ki = key[i], kj = key[j];
+            const uint32_t ii = item[i], ij = item[j];
+            key[i] = sw ? kj : ki;
+            key[j] = sw ? ki : kj;
+            item[i] = sw ? ij : ii;
+            item[j] = sw ? ii : ij;
+        };
+        cx(0, 1);
+        cx(2, 3);
+        cx(0, 2);
+        cx(1, 3);
+        cx(1, 2);
+    }
+};
+template <> struct ChildOrder<true> {
+    uint32_t item[4];
+    KF_DEV ChildOrder(const float (&k)[4], const uint32_t (&it)[4]) {
+        double key[4];
+        for (int c = 0; c < 4; ++c) key[c] = __hiloint2double((int)__float_as_uint(k[c]), (int)it[c]);
+        auto cx = [&](int i, int j) __attribute__((always_inline)) {
+            const double a = key[i], b = key[j];
+            asm("v_min_f64 %0, %1, %2" : "=v"(key[i]) : "v"(a), "v"(b));
+            asm("v_max_f64 %0, %1, %2" : "=v"(key[j]) : "v"(a), "v"(b));
+        };
+        cx(0, 1);
+        cx(2, 3);
+        cx(0, 2);
+        cx(1, 3);
+        cx(1, 2);
+        for (int c = 0; c < 4; ++c) item[c] = (uint32_t)__double2loint(key[c]);
+    }
+};
+
 // ANY: shadow-ray query (opaque, stop at the first hit in [tmin, tmax]).
 // Closest-hit queries with use_alpha run the any-hit alpha test
 // (PathTrace.rahit:30-48) for non-opaque instances, with an order-independent
@@ -284,8 +340,8 @@ KF_DEV uint32_t env_root_item(const SceneView& S, uint32_t e) {
 // kinds with the same steps.
 // What bounds it: the vector ALUs (about 340 instructions per step) and the
 // vector L1 about equally.  Each lane loading its own record's lines only, the
-// shear axes as scalar logic, the sort on 64-bit keys and a stack without a
-// cached top took 19 % of the vector instructions and 26 % of the L1 accesses:
+// shear axes as scalar logic and a stack without a cached top took 17 % of the
+// vector instructions and 26 % of the L1 accesses:
 // 2 M rays 1.05 -> 0.97 ms, 1080p frame at 16 spp 18.7 -> 17.2 ms, 128
 // environments of 512x512 at 8 spp 137.7 -> 129 ms.
 template <bool ANY, bool COUNT, bool MIXED = false>
@@ -529,16 +585,12 @@ struct Trav {
         found = found || take;
 
         // node: four child boxes (lines lox, loy, loz, hix, hiy, hiz, ref)
-        // against the level's ray.  A child's sort key is its entry distance
-        // with its item below it, as one 64-bit float whose order is that of
-        // the distances (equal ones by item): an exchange of the sorting
-        // network is then a 64-bit min and max instead of a comparison and
-        // four selects.  No key is a NaN (the high word is a float).
+        // against the level's ray, nearest first.
         const float hix[4] = {r3.x, r3.y, r3.z, r3.w};
         const float hiy[4] = {r4.x, r4.y, r4.z, r4.w};
         const float hiz[4] = {r5.x, r5.y, r5.z, r5.w};
         const uint32_t item[4] = {__float_as_uint(r6.x), __float_as_uint(r6.y), __float_as_uint(r6.z), __float_as_uint(r6.w)};
-        double key[4];
+        float key[4];
         uint32_t n = 0;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -551,22 +603,11 @@ struct Trav {
             // Nearer child first; any-hit queries take leaf children
             // (triangles, instances: kinds 2 and 3) before inner ones, which
             // finds occluders sooner.
-            const float k = h ? (((ANY || (MIXED && any_q)) && (item[c] >> 31)) ? -INFINITY : tn) : INFINITY;
-            key[c] = __hiloint2double((int)__float_as_uint(k), (int)item[c]);
+            key[c] = h ? (((ANY || (MIXED && any_q)) && (item[c] >> 31)) ? -INFINITY : tn) : INFINITY;
             n += h ? 1u : 0u;
         }
-        auto cx = [&](int i, int j) __attribute__((always_inline)) {
-            const double a = key[i], b = key[j];
-            asm("v_min_f64 %0, %1, %2" : "=v"(key[i]) : "v"(a), "v"(b));
-            asm("v_max_f64 %0, %1, %2" : "=v"(key[j]) : "v"(a), "v"(b));
-        };
-        cx(0, 1);
-        cx(2, 3);
-        cx(0, 2);
-        cx(1, 3);
-        cx(1, 2);
-        const uint32_t c0 = (uint32_t)__double2loint(key[0]), c1 = (uint32_t)__double2loint(key[1]);
-        const uint32_t c2 = (uint32_t)__double2loint(key[2]), c3 = (uint32_t)__double2loint(key[3]);
+        const ChildOrder<ANY> order(key, item);
+        const uint32_t c0 = order.item[0], c1 = order.item[1], c2 = order.item[2], c3 = order.item[3];
 
         if (COUNT) {
             cnt.nodes += (kind <= kBlasNode && on) ? 1u : 0u;

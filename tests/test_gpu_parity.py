@@ -255,6 +255,62 @@ def test_blas_boxes_are_the_unions_of_their_triangles(gpu, counts):
             gs.update_geometry(len(counts) - 1, moved)
 
 
+def contact_rays(data, n, seed):
+    """Rays from within 5 mm of the lines where the bodies of a scene stand on
+    its ground (instance 0), half of them from the ground itself."""
+    rng = np.random.default_rng(seed)
+    inst = data.arrays()["inst"]
+    ends = []
+    for i in range(1, len(inst)):
+        m = inst[i]["transform"].reshape(4, 4)
+        p = data.geoms[int(inst[i]["geometry_index"])][0]["pos"] @ m[:3, :3] + m[3, :3]
+        foot = p[p[:, 2] < p[:, 2].min() + 1e-4]
+        ends += [foot[rng.integers(len(foot), size=2)] for _ in range(8)]
+    a, b = np.array(ends)[rng.integers(len(ends), size=n)].transpose(1, 0, 2)
+    org = a + rng.uniform(size=(n, 1)) * (b - a) + rng.uniform(-0.005, 0.005, (n, 3))
+    org[:, 2] = np.where(np.arange(n) % 2 == 0, 0.0, np.abs(org[:, 2]))
+    d = rng.uniform(-1, 1, (n, 3))
+    rays = np.zeros(n, abi.RAY_DTYPE)
+    rays["org"], rays["dir"] = org, d / np.linalg.norm(d, axis=1, keepdims=True)
+    rays["tmin"], rays["tmax"] = 0.001, 1e4
+    return rays
+
+
+@pytest.mark.parametrize("seed", [0, 1, 2, 3])
+def test_hits_do_not_follow_the_numbering_of_instances(gpu, seed):
+    """Children entered at the same distance are visited in the order of their
+    places in the node, so the same instances in another order give the same
+    hits, also where two surfaces are hit within a rounding of each other."""
+    w = scenes.config3(seed=seed)
+    inst = w.data.arrays()["inst"].copy()
+    rays = contact_rays(w.data, 1 << 18, seed)
+    gs = GpuScene(w.data)
+    hits = gs.trace_closest(rays)
+    for order in (np.arange(len(inst))[::-1], np.random.default_rng(seed).permutation(len(inst))):
+        gs.update_instances(np.ascontiguousarray(inst[order]))
+        assert gs.trace_closest(rays)["t"].tobytes() == hits["t"].tobytes()
+
+
+# (seed, ray of contact_rays, instance, primitive, distance): hits that turn on
+# the order of children entered at the same distance.  closest: whether that
+# order finds the closest one; the other hits lie within 5e-7 m of it, a few
+# roundings of a distance over the 4 m ground.
+@pytest.mark.parametrize("seed,ray,inst,prim,t,closest", [
+    (0, 5399, 0, 0, "0x1.1648460000000p-10", True), (2, 27307, 58, 57, "0x1.f301880000000p-10", True),
+    (3, 9363, 19, 11, "0x1.c2e5e60000000p-10", False), (0, 959, 23, 49, "0x1.99dd400000000p-6", False),
+    (1, 151, 54, 43, "0x1.0cabb40000000p-7", False), (3, 10955, 34, 10, "0x1.28a4e60000000p-5", False)])
+def test_hits_at_contact_lines(gpu, seed, ray, inst, prim, t, closest):
+    w = scenes.config3(seed=seed)
+    rays = contact_rays(w.data, 1 << 18, seed)[ray:ray + 1]
+    (hit,) = GpuScene(w.data).trace_closest(rays)
+    assert (hit["inst"], hit["prim"], float(hit["t"])) == (inst, prim, float.fromhex(t))
+    (ref,) = oracle.Scene(w.data).trace_closest(rays, brute=True)
+    if closest:
+        assert (ref["inst"], ref["prim"], ref["t"]) == (hit["inst"], hit["prim"], hit["t"])
+    else:
+        assert 0.0 < hit["t"] - ref["t"] < 5e-7
+
+
 EMPTY_ITEM = 0xFFFFFFFF
 
 
