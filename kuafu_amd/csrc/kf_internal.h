@@ -274,9 +274,8 @@ struct Renderer {
     uint32_t W = 0, H = 0;
     float4 *d_rgba = nullptr, *d_albedo = nullptr, *d_normal = nullptr;
     uint8_t* d_bgra = nullptr;
-    // wavefront state, sized for `cap` paths and `slots` NEE slots per path
-    size_t cap = 0;
-    uint32_t slots = 0;
+    // wavefront state, sized for `cap` paths and `slot_cap` NEE slots in all
+    size_t cap = 0, slot_cap = 0;
     float4 *ray_o = nullptr, *ray_d = nullptr, *thr = nullptr, *col = nullptr, *rw = nullptr;
     float4* hit = nullptr;
     uint32_t* hit_prim = nullptr;

@@ -1439,44 +1439,54 @@ Renderer::~Renderer() {
         if (p) (void)hipFree(p);
 }
 
-// Buffers for `paths` paths; false when they do not fit the free memory
-// (nothing is held then).
+// Buffers for `paths` paths of nslots NEE slots each; false when they do not
+// fit the free memory (nothing is held then).  Paths and slots have capacities
+// of their own: a renderer that has drawn many paths with few lights and then
+// draws few paths with many holds the larger of each, not their product
+// (4.2 M paths with 2 lights, then 0.26 M with 41: 1.3 GB instead of 12.4).
 bool Renderer::ensure(size_t paths, uint32_t nslots, uint32_t spp) {
-    if (paths > cap || nslots > slots) {
-        const size_t want = std::max(cap, paths);
-        const uint32_t wslots = std::max(slots, std::max<uint32_t>(nslots, 1));
-        struct Buf {
-            void** p;
-            size_t bytes;
-        };
-        const size_t f4 = want * sizeof(float4), u4 = want * sizeof(uint32_t), s4 = wslots * f4;
-        const Buf bufs[] = {{(void**)&ray_o, f4},   {(void**)&ray_d, f4},   {(void**)&thr, f4},
-                            {(void**)&col, f4},     {(void**)&rw, f4},
-                            {(void**)&hit, f4},     {(void**)&hit_prim, u4}, {(void**)&seed, u4},
-                            {(void**)&queue_a, u4}, {(void**)&queue_b, u4}, {(void**)&queue_e, u4},
-                            {(void**)&sh_o, s4},    {(void**)&sh_d, s4},    {(void**)&sh_root, wslots * u4},
-                            {(void**)&nee_a, s4},   {(void**)&nee_b, s4},   {(void**)&vis, wslots * want},
-                        {(void**)&d_out, f4}};
-        auto drop = [&] {
-            for (const Buf& b : bufs) {
-                if (*b.p) KF_CHECK(hipFree(*b.p));
-                *b.p = nullptr;
-            }
-            cap = 0;
-            slots = 0;
-        };
-        drop();
+    const size_t want_slots = paths * std::max<uint32_t>(nslots, 1);
+    struct Buf {
+        void** p;
+        size_t bytes;
+    };
+    auto grow = [](const auto& bufs, size_t want, size_t& have) {
         for (const Buf& b : bufs) {
-            const hipError_t e = hipMalloc(b.p, b.bytes);
+            if (*b.p) KF_CHECK(hipFree(*b.p));
+            *b.p = nullptr;
+        }
+        have = 0;
+        if (!want) return true;
+        for (const Buf& b : bufs) {
+            const hipError_t e = hipMalloc(b.p, want * b.bytes);
             if (e == hipSuccess) continue;
             *b.p = nullptr;
             (void)hipGetLastError();
-            drop();
             if (e == hipErrorOutOfMemory) return false;
             throw Error(std::string("kf_render: hipMalloc: ") + hipGetErrorString(e));
         }
-        cap = want;
-        slots = wslots;
+        have = want;
+        return true;
+    };
+    const Buf per_path[] = {{(void**)&ray_o, 16},  {(void**)&ray_d, 16},  {(void**)&thr, 16},    {(void**)&col, 16},
+                            {(void**)&rw, 16},     {(void**)&hit, 16},    {(void**)&d_out, 16},  {(void**)&hit_prim, 4},
+                            {(void**)&seed, 4},    {(void**)&queue_a, 4}, {(void**)&queue_b, 4}, {(void**)&queue_e, 4}};
+    const Buf per_slot[] = {{(void**)&sh_o, 16},  {(void**)&sh_d, 16}, {(void**)&nee_a, 16},
+                            {(void**)&nee_b, 16}, {(void**)&sh_root, 4}, {(void**)&vis, 1}};
+    auto fits = [&] {
+        return (paths <= cap || grow(per_path, paths, cap)) &&
+               (want_slots <= slot_cap || grow(per_slot, want_slots, slot_cap));
+    };
+    auto drop = [&] {
+        (void)grow(per_path, 0, cap);
+        (void)grow(per_slot, 0, slot_cap);
+    };
+    if (!fits()) {  // without what earlier frames left
+        drop();
+        if (!fits()) {
+            drop();
+            return false;
+        }
     }
     size_t sneed = (size_t)spp * W * H * 3;
     if (spp && sneed > samples_cap) {

@@ -1,0 +1,48 @@
+"""Memory of a renderer's path state (marked gpu): what a sequence of frames
+makes it hold, and frames and tuning where the state does not fit.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from kuafu_amd import abi, scenes
+from kuafu_amd.api import GpuScene, Renderer
+
+pytestmark = pytest.mark.gpu
+
+GIB = 1 << 30
+
+
+def free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert abi.lib().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def with_lights(w, n):
+    """The workload under n lights of all kinds, none of them soft."""
+    w.data.point_lights, w.data._n_point = abi.PointLights(), 0
+    for k in range(min(n - 1, 32)):
+        w.data.add_point_light((4.0 * np.cos(k), 2.0 + 0.05 * k, 4.0 * np.sin(k)), (1, 0.9, 0.8), 3.0, radius=0.0)
+    for k in range(n - 33):
+        view = scenes.look_at((3.0 * np.cos(2 * k), 4.0, 3.0 * np.sin(2 * k)), (0.0, 0.3, 0.0), (0, 1, 0))
+        w.data.add_active_light(view, (0.8, 0.9, 1.0), fov=0.9, strength=20.0)
+    return w
+
+
+def test_paths_and_slots_have_capacities_of_their_own(gpu):
+    """4.2 M paths with two lights, then 0.26 M with 41, hold 132 bytes per
+    path of the first frame and 69 per path and light of the second: 1.3 GB
+    (the product of both, 41 lights for 4.2 M paths, is 12.4)."""
+    many, few = scenes.config1(512, 512, spp=16, path_depth=3), with_lights(scenes.config1(512, 512, spp=1, path_depth=3), 41)
+    a, b = GpuScene(many.data), GpuScene(few.data)
+    r, alone = Renderer(512, 512), Renderer(512, 512)
+    alone.render(b, few.cam, few.pc, seed=1)
+    want = alone.read(0)
+    alone.close()
+    before = free_bytes()
+    r.render(a, many.cam, many.pc, seed=1, samples_per_batch=16)
+    r.render(b, few.cam, few.pc, seed=1)
+    assert before - free_bytes() < 2 * GIB
+    assert np.array_equal(r.read(0), want)
