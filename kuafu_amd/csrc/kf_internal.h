@@ -276,6 +276,7 @@ struct Renderer {
     uint8_t* d_bgra = nullptr;
     // wavefront state, sized for `cap` paths and `slot_cap` NEE slots in all
     size_t cap = 0, slot_cap = 0;
+    size_t state_limit = SIZE_MAX;             // bytes of path state that fitted after a default batch had not
     float4 *ray_o = nullptr, *ray_d = nullptr, *thr = nullptr, *col = nullptr, *rw = nullptr;
     float4* hit = nullptr;
     uint32_t* hit_prim = nullptr;
@@ -321,6 +322,8 @@ struct Renderer {
     uint32_t n_env_last = 1;                   // environments of the last frame (the denoiser's batch)
     ~Renderer();
     bool ensure(size_t paths, uint32_t nslots, uint32_t spp);
+    bool holds(size_t paths, uint32_t nslots) const { return paths <= cap && paths * nslots <= slot_cap; }
+    size_t state_held() const;
 };
 
 }  // namespace kf

@@ -1439,6 +1439,10 @@ Renderer::~Renderer() {
         if (p) (void)hipFree(p);
 }
 
+// Path state: bytes per path, and per path and NEE slot (Renderer::ensure).
+constexpr size_t kPathBytes = 132, kSlotBytes = 69;
+size_t Renderer::state_held() const { return cap * kPathBytes + slot_cap * kSlotBytes; }
+
 // Buffers for `paths` paths of nslots NEE slots each; false when they do not
 // fit the free memory (nothing is held then).  Paths and slots have capacities
 // of their own: a renderer that has drawn many paths with few lights and then
@@ -1468,6 +1472,7 @@ bool Renderer::ensure(size_t paths, uint32_t nslots, uint32_t spp) {
         have = want;
         return true;
     };
+    // kPathBytes and kSlotBytes are the sums of these
     const Buf per_path[] = {{(void**)&ray_o, 16},  {(void**)&ray_d, 16},  {(void**)&thr, 16},    {(void**)&col, 16},
                             {(void**)&rw, 16},     {(void**)&hit, 16},    {(void**)&d_out, 16},  {(void**)&hit_prim, 4},
                             {(void**)&seed, 4},    {(void**)&queue_a, 4}, {(void**)&queue_b, 4}, {(void**)&queue_e, 4}};
@@ -1515,11 +1520,14 @@ uint32_t resident_grid(Kernel kernel, int n_cu) {
 
 constexpr uint32_t kLastShadowGrab = 32;  // queries per wave reservation, last wavefront bounce's shadow rays
 
+size_t state_bytes(size_t paths, uint32_t nslots) { return paths * (kPathBytes + kSlotBytes * (size_t)nslots); }
+
 // Default batch: up to 64M paths (2 spp of 128 environments of 512x512).
 // Each batch ends every bounce's launch on its slowest rays, about 3 ms in
 // all on that frame (batches of 32M, 64M, 128M, 256M paths: 175, 162, 156,
 // 153 ms); the state costs 200-300 B per path, 13-19 GB at 64M paths, and a
-// default that does not fit the free memory is halved (render_frame).
+// default that does not leave a quarter of the free memory is halved
+// (render_frame).
 uint32_t default_batch(uint32_t spp, uint32_t WH) {
     return std::max<uint32_t>(1, std::min<uint32_t>(spp, (64u << 20) / std::max<uint32_t>(WH, 1)));
 }
@@ -1612,13 +1620,24 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     build_light_list(*s, L, inline_nee);
     uint32_t WH = r->W * r->H;
     uint32_t spb = o.samples_per_batch ? o.samples_per_batch : r->tune_spb;
+    const uint32_t K = inline_nee ? 1u : (uint32_t)std::max(L.n_slots, 1);
     if (spb == 0) spb = default_batch(pc->spp, WH);
     spb = std::min(spb, pc->spp);
-    uint32_t K = inline_nee ? 1u : (uint32_t)std::max(L.n_slots, 1);
+    // A default batch that the buffers held do not take already leaves a quarter
+    // of the free memory to others, and is halved where it does not fit after
+    // all; state_limit keeps later frames from trying again (a frame that gave
+    // its buffers back, failed and allocated anew took 313 ms instead of 16).
     const bool spb_default = !o.samples_per_batch && !r->tune_spb;
+    if (spb_default && !r->holds((size_t)WH * spb, K)) {
+        size_t free_mem = 0, total = 0;
+        KF_CHECK(hipMemGetInfo(&free_mem, &total));
+        const size_t room = std::min((free_mem + r->state_held()) / 4 * 3, r->state_limit);
+        while (spb > 1 && state_bytes((size_t)WH * spb, K) > room && !r->holds((size_t)WH * spb, K)) spb = (spb + 1) / 2;
+    }
     while (!r->ensure((size_t)WH * spb, K, o.keep_samples ? pc->spp : 0)) {
         if (!spb_default || spb == 1) throw Error("kf_render: out of GPU memory for the path state");
         spb = (spb + 1) / 2;
+        r->state_limit = state_bytes((size_t)WH * spb, K);
     }
     r->samples_spp = o.keep_samples ? pc->spp : 0;
     // device light list (per frame, like the UBO upload)

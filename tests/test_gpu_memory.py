@@ -2,6 +2,7 @@
 makes it hold, and frames and tuning where the state does not fit.
 """
 import ctypes as C
+import time
 
 import numpy as np
 import pytest
@@ -46,3 +47,53 @@ def test_paths_and_slots_have_capacities_of_their_own(gpu):
     r.render(b, few.cam, few.pc, seed=1)
     assert before - free_bytes() < 2 * GIB
     assert np.array_equal(r.read(0), want)
+
+
+@pytest.fixture
+def scarce(gpu):
+    """scarce(n): leaves n bytes of GPU memory free until the test ends."""
+    L, held = abi.lib(), []
+    small = scenes.config1(32, 32, spp=1, path_depth=6)
+    gs, r = GpuScene(small.data), Renderer(32, 32)
+    for tail in (1, 2, 7):  # code and scratch of the kernels, while there is room
+        r.set_schedule(tail_bounce=tail)
+        r.render(gs, small.cam, small.pc)
+
+    def leave(n):
+        p = C.c_void_p()
+        assert L.hipMalloc(C.byref(p), C.c_size_t(free_bytes() - n)) == 0
+        held.append(p)
+
+    yield leave
+    for p in held:
+        assert L.hipFree(p) == 0
+
+
+def test_default_batch_in_scarce_memory(scarce):
+    """A default batch leaves a quarter of the free memory to others, also on
+    the frames after the first, which allocate nothing.  33.5 M paths with two
+    lights are 9.1 GB: less than three quarters of what is free, more than
+    that, and more than is free."""
+    w = scenes.config1(2048, 1024, spp=16, path_depth=2)
+    gs, ref = GpuScene(w.data), Renderer(2048, 1024)
+    ref.render(gs, w.cam, w.pc, seed=1, samples_per_batch=1)
+    want = ref.read(0)
+    ref.close()
+    for free, halved in ((16, False), (10, True), (6, True)):
+        scarce(free * GIB)
+        r = Renderer(2048, 1024)
+        before = free_bytes()
+        launches, ms = [], []
+        for _ in range(4):
+            t = time.perf_counter()
+            launches.append(r.render(gs, w.cam, w.pc, seed=1).extend_launches)
+            ms.append(time.perf_counter() - t)
+            assert free_bytes() >= before // 4 - GIB // 2  # targets, camera rays' tree
+        assert len(set(launches)) == 1
+        assert np.array_equal(r.read(0), want)
+        t = time.perf_counter()
+        st = r.render(gs, w.cam, w.pc, seed=1, samples_per_batch=8)
+        t = time.perf_counter() - t
+        assert (launches[0] > st.extend_launches // 2) == halved
+        assert min(ms[1:]) < 5 * t  # 313 ms against 16 where every frame allocated
+        r.close()
