@@ -21,6 +21,9 @@ struct Error : std::exception {
     explicit Error(std::string m) : msg(std::move(m)) {}
     const char* what() const noexcept override { return msg.c_str(); }
 };
+struct OutOfMemory : Error {
+    using Error::Error;
+};
 
 void set_error(const std::string& m);
 hipStream_t stream();
@@ -277,6 +280,7 @@ struct Renderer {
     // wavefront state, sized for `cap` paths and `slot_cap` NEE slots in all
     size_t cap = 0, slot_cap = 0;
     size_t state_limit = SIZE_MAX;             // bytes of path state that fitted after a default batch had not
+    uint32_t last_spb = 0;                     // samples per batch of the last frame
     float4 *ray_o = nullptr, *ray_d = nullptr, *thr = nullptr, *col = nullptr, *rw = nullptr;
     float4* hit = nullptr;
     uint32_t* hit_prim = nullptr;
@@ -317,8 +321,10 @@ struct Renderer {
     uint32_t graph_ext = 0, graph_sh = 0;      // traversal launches in the graph
     uint64_t graph_captures = 0;               // frame graphs captured by this renderer so far
     // Schedule picked by kf_renderer_autotune (0: built-in default).
-    uint32_t tune_spb = 0, tune_refill = 0, tune_grab = 0, tune_tail = 0, tune_grab0 = 0, tune_grabs = 0;
-    uint32_t tune_pairs = 1;  // 1: k_tail2 may carry the tail bounces of few paths, 0: k_tail only
+    struct Schedule {
+        uint32_t spb = 0, refill = 0, grab = 0, tail = 0, grab0 = 0, grabs = 0;
+        uint32_t pairs = 1;  // 1: k_tail2 may carry the tail bounces of few paths, 0: k_tail only
+    } tune;
     uint32_t n_env_last = 1;                   // environments of the last frame (the denoiser's batch)
     ~Renderer();
     bool ensure(size_t paths, uint32_t nslots, uint32_t spp);

@@ -1619,7 +1619,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     bool inline_nee = false;
     build_light_list(*s, L, inline_nee);
     uint32_t WH = r->W * r->H;
-    uint32_t spb = o.samples_per_batch ? o.samples_per_batch : r->tune_spb;
+    uint32_t spb = o.samples_per_batch ? o.samples_per_batch : r->tune.spb;
     const uint32_t K = inline_nee ? 1u : (uint32_t)std::max(L.n_slots, 1);
     if (spb == 0) spb = default_batch(pc->spp, WH);
     spb = std::min(spb, pc->spp);
@@ -1627,7 +1627,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     // of the free memory to others, and is halved where it does not fit after
     // all; state_limit keeps later frames from trying again (a frame that gave
     // its buffers back, failed and allocated anew took 313 ms instead of 16).
-    const bool spb_default = !o.samples_per_batch && !r->tune_spb;
+    const bool spb_default = !o.samples_per_batch && !r->tune.spb;
     if (spb_default && !r->holds((size_t)WH * spb, K)) {
         size_t free_mem = 0, total = 0;
         KF_CHECK(hipMemGetInfo(&free_mem, &total));
@@ -1635,10 +1635,11 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
         while (spb > 1 && state_bytes((size_t)WH * spb, K) > room && !r->holds((size_t)WH * spb, K)) spb = (spb + 1) / 2;
     }
     while (!r->ensure((size_t)WH * spb, K, o.keep_samples ? pc->spp : 0)) {
-        if (!spb_default || spb == 1) throw Error("kf_render: out of GPU memory for the path state");
+        if (!spb_default || spb == 1) throw OutOfMemory("kf_render: out of GPU memory for the path state");
         spb = (spb + 1) / 2;
         r->state_limit = state_bytes((size_t)WH * spb, K);
     }
+    r->last_spb = spb;
     r->samples_spp = o.keep_samples ? pc->spp : 0;
     // device light list (per frame, like the UBO upload)
     if (!r->d_lights) KF_CHECK(hipMalloc(&r->d_lights, sizeof(DevLights)));
@@ -1742,15 +1743,15 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     // connect passes carry two lights per path, that is 5 % faster than 2
     // blocks per CU; on the 1080p frame the two are within noise
     const uint32_t grid_conn = (uint32_t)n_cu * 8;
-    const uint32_t refill = std::min<uint32_t>(64u, std::max<uint32_t>(1u, r->tune_refill ? r->tune_refill
+    const uint32_t refill = std::min<uint32_t>(64u, std::max<uint32_t>(1u, r->tune.refill ? r->tune.refill
                                                                                          : traversal_refill()));
     // largest reservation per wave
-    const uint32_t grab = std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grab ? r->tune_grab : kGrab));
+    const uint32_t grab = std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune.grab ? r->tune.grab : kGrab));
     // camera rays (bounce 0): one long, coherent queue that may want another
     // reservation than the scattered later bounces
-    const uint32_t grab0 = r->tune_grab0 ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grab0)) : grab;
+    const uint32_t grab0 = r->tune.grab0 ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune.grab0)) : grab;
     // shadow rays: short any-hit queries, which favour smaller reservations
-    const uint32_t grabs = r->tune_grabs ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune_grabs)) : grab;
+    const uint32_t grabs = r->tune.grabs ? std::min<uint32_t>(4096u, std::max<uint32_t>(16u, r->tune.grabs)) : grab;
     // Persistent traversal kernels: the blocks that fit at once.
     static const uint32_t grid_ext0 = std::min(resident_grid(k_extend<false>, n_cu), kExtendBlocks * (uint32_t)n_cu);
     static const uint32_t grid_ext1 = resident_grid(k_extend<true>, n_cu);
@@ -1758,7 +1759,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     const uint32_t nb = pc->path_depth + 1;
     // bounces from b_tail on run in k_tail (not in counting frames, whose
     // node counts come from the wavefront kernels)
-    const uint32_t tail = r->tune_tail ? r->tune_tail
+    const uint32_t tail = r->tune.tail ? r->tune.tail
                                        : std::max(1u, default_tail(*pc, (uint64_t)WH * spb, (uint32_t)L.n_slots, nb));
     const uint32_t b_tail = o.count_traversal ? nb : std::min(tail, nb);
 
@@ -1810,7 +1811,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
                 // k_tail beyond, and the other launch returns at once (up to
                 // a quarter, 4 M paths from bounce 3 are 4 % slower: the
                 // pairs then compete for the same SIMDs)
-                const uint32_t pair_max = (inline_nee || !r->tune_pairs) ? 0u : grid * TB / 8u;
+                const uint32_t pair_max = (inline_nee || !r->tune.pairs) ? 0u : grid * TB / 8u;
                 if (!inline_nee)
                     k_tail2<<<grid, TB, 0, st>>>(S, F, d_lights, (int)b, qa, r->ray_o, r->ray_d, r->thr, r->col,
                                                  r->hit, r->hit_prim, r->rw, r->seed, r->nee_a, r->nee_b,
@@ -1879,7 +1880,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
             key.insert(key.end(), b, b + n);
         };
         const uint32_t sched[12] = {spb, K, nb, refill, grab, grid, (uint32_t)o.count_traversal,
-                                    (uint32_t)o.keep_samples, b_tail, grab0, grabs, r->tune_pairs};
+                                    (uint32_t)o.keep_samples, b_tail, grab0, grabs, r->tune.pairs};
         const void* bufs[] = {r->ray_o, r->ray_d, r->thr, r->col, r->rw, r->hit, r->hit_prim, r->seed,
                               r->queue_a, r->queue_b, r->queue_e, r->sh_o, r->sh_d, r->sh_root, r->nee_a,
                               r->nee_b, r->vis, r->samples, r->counters, d_lights, d_jump, d_acc, d_out,
@@ -1989,6 +1990,7 @@ extern "C" int kf_render_envs(kf_renderer* r, kf_scene* s, uint32_t num_envs, co
 
 extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_envs, const kf_camera_ubo* cams,
                                     const kf_push_constants* pc, kf_tune_result* out) {
+    const Renderer::Schedule before = r ? r->tune : Renderer::Schedule();
     try {
         if (!r || !s || !cams || !pc || !out) throw Error("kf_renderer_autotune: null argument");
         kf_push_constants p = *pc;
@@ -1999,17 +2001,22 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
         // of three (of one for frames over 50 ms)
         uint32_t b_tail = 0, b_grab0 = 0, b_grabs = 0, b_pairs = 1;
         auto run = [&](uint32_t spb, uint32_t refill, uint32_t grab) {
-            r->tune_spb = spb;
-            r->tune_refill = refill;
-            r->tune_grab = grab;
-            r->tune_tail = b_tail;
-            r->tune_grab0 = b_grab0;
-            r->tune_grabs = b_grabs;
-            r->tune_pairs = b_pairs;
+            r->tune.spb = spb;
+            r->tune.refill = refill;
+            r->tune.grab = grab;
+            r->tune.tail = b_tail;
+            r->tune.grab0 = b_grab0;
+            r->tune.grabs = b_grabs;
+            r->tune.pairs = b_pairs;
             float best = INFINITY;
             for (int k = 0; k < 3; ++k) {
                 kf_render_stats st{};
-                render_frame(r, s, num_envs, cams, &p, &o, &st);
+                try {
+                    render_frame(r, s, num_envs, cams, &p, &o, &st);
+                } catch (const OutOfMemory&) {
+                    if (!spb) throw;
+                    return INFINITY;  // a batch that no longer fits
+                }
                 ++trials;
                 best = std::min(best, st.trace_ms);
                 if (st.trace_ms > 50.0f) break;
@@ -2019,7 +2026,6 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
         run(0, 0, 0);  // warm-up: buffers, code objects, clocks
         run(0, 0, 0);
         const float t_def = run(0, 0, 0);
-        const uint32_t WH = r->W * r->H;
         uint32_t b_spb = 0, b_refill = 0, b_grab = 0;
         float t_best = t_def;
         // One parameter at a time.  Every candidate is timed in a forward
@@ -2048,13 +2054,11 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
             best = cand[kb];
             t_best = t[kb];
         };
+        // powers of two up to the batch the default frames had, and that one
+        const uint32_t spb_def = r->last_spb;
         std::vector<uint32_t> spbs;
-        for (uint32_t spb = 1; spb <= p.spp; spb *= 2) {
-            if ((uint64_t)WH * spb > (64ull << 20)) break;  // path state stays within ~13 GB
-            spbs.push_back(spb);
-        }
-        const uint32_t spb_def = default_batch(p.spp, WH);
-        if (std::find(spbs.begin(), spbs.end(), spb_def) == spbs.end()) spbs.push_back(spb_def);
+        for (uint32_t spb = 1; spb < spb_def; spb *= 2) spbs.push_back(spb);
+        spbs.push_back(spb_def);
         b_refill = std::min<uint32_t>(64u, std::max<uint32_t>(1u, traversal_refill()));
         b_grab = kGrab;
         // the best refill threshold depends on the reservation size: the
@@ -2097,13 +2101,13 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
         uint32_t best_grabs = 0;
         sweep(grabss, best_grabs, 5);
         b_grabs = best_grabs;
-        r->tune_spb = b_spb;
-        r->tune_refill = b_refill;
-        r->tune_grab = b_grab;
-        r->tune_tail = b_tail;
-        r->tune_grab0 = b_grab0;
-        r->tune_grabs = b_grabs;
-        r->tune_pairs = b_pairs;
+        r->tune.spb = b_spb;
+        r->tune.refill = b_refill;
+        r->tune.grab = b_grab;
+        r->tune.tail = b_tail;
+        r->tune.grab0 = b_grab0;
+        r->tune.grabs = b_grabs;
+        r->tune.pairs = b_pairs;
         out->tail_pairs = b_pairs;
         out->tail_bounce = b_tail;
         out->grab0 = b_grab0;
@@ -2116,6 +2120,7 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
         out->trials = trials;
         return 0;
     } catch (const std::exception& e) {
+        if (r) r->tune = before;
         set_error(e.what());
         return -1;
     }
@@ -2127,13 +2132,13 @@ extern "C" int kf_renderer_set_schedule(kf_renderer* r, uint32_t samples_per_bat
         set_error("kf_renderer_set_schedule: null renderer");
         return -1;
     }
-    r->tune_spb = samples_per_batch;
-    r->tune_refill = refill;
-    r->tune_grab = grab;
-    r->tune_tail = tail_bounce;
-    r->tune_grab0 = grab0;
-    r->tune_grabs = grab_shadow;
-    r->tune_pairs = 1;
+    r->tune.spb = samples_per_batch;
+    r->tune.refill = refill;
+    r->tune.grab = grab;
+    r->tune.tail = tail_bounce;
+    r->tune.grab0 = grab0;
+    r->tune.grabs = grab_shadow;
+    r->tune.pairs = 1;
     return 0;
 }
 
@@ -2146,7 +2151,7 @@ extern "C" int kf_renderer_set_tail_pairs(kf_renderer* r, uint32_t tail_pairs) {
         set_error("kf_renderer_set_tail_pairs: tail_pairs must be 0 or 1");
         return -1;
     }
-    r->tune_pairs = tail_pairs;
+    r->tune.pairs = tail_pairs;
     return 0;
 }
 

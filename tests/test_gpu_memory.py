@@ -7,7 +7,7 @@ import time
 import numpy as np
 import pytest
 
-from kuafu_amd import abi, scenes
+from kuafu_amd import KuafuError, abi, scenes
 from kuafu_amd.api import GpuScene, Renderer
 
 pytestmark = pytest.mark.gpu
@@ -97,3 +97,28 @@ def test_default_batch_in_scarce_memory(scarce):
         assert (launches[0] > st.extend_launches // 2) == halved
         assert min(ms[1:]) < 5 * t  # 313 ms against 16 where every frame allocated
         r.close()
+
+
+def test_autotune_in_scarce_memory(scarce):
+    """Tuning passes over batches that do not fit (16 samples: 9.1 GB of 6
+    GiB), and the renderer draws with what it picked."""
+    w = scenes.config1(2048, 1024, spp=16, path_depth=2)
+    gs = GpuScene(w.data)
+    scarce(6 * GIB)
+    r = Renderer(2048, 1024)
+    want = r.render(gs, w.cam, w.pc, seed=1, samples_per_batch=1) and r.read(0)
+    t = r.autotune(gs, w.cam, w.pc)
+    assert 1 <= t["samples_per_batch"] < 16 and t["frame_ms"] < np.inf
+    r.render(gs, w.cam, w.pc, seed=1)
+    assert np.array_equal(r.read(0), want)
+
+
+def test_failed_autotune_keeps_the_schedule(gpu):
+    w = scenes.config1(64, 64, spp=8, path_depth=4)
+    gs, r = GpuScene(w.data), Renderer(64, 64)
+    r.set_schedule(samples_per_batch=2, tail_bounce=3)
+    before = r.render(gs, w.cam, w.pc).extend_launches
+    deep = scenes.config1(64, 64, spp=8, path_depth=70)
+    with pytest.raises(KuafuError, match="depth"):
+        r.autotune(gs, deep.cam, deep.pc)
+    assert r.render(gs, w.cam, w.pc).extend_launches == before == 4 * 3
