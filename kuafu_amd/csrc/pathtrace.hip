@@ -1522,14 +1522,19 @@ constexpr uint32_t kLastShadowGrab = 32;  // queries per wave reservation, last 
 
 size_t state_bytes(size_t paths, uint32_t nslots) { return paths * (kPathBytes + kSlotBytes * (size_t)nslots); }
 
-// Default batch: up to 64M paths (2 spp of 128 environments of 512x512).
-// Each batch ends every bounce's launch on its slowest rays, about 3 ms in
-// all on that frame (batches of 32M, 64M, 128M, 256M paths: 175, 162, 156,
-// 153 ms); the state costs 200-300 B per path, 13-19 GB at 64M paths, and a
-// default that does not leave a quarter of the free memory is halved
-// (render_frame).
-uint32_t default_batch(uint32_t spp, uint32_t WH) {
-    return std::max<uint32_t>(1, std::min<uint32_t>(spp, (64u << 20) / std::max<uint32_t>(WH, 1)));
+// Default batch: 64M paths while their state stays within 32 GiB (up to five
+// lights), fewer for more lights, but not below 32M (98 GB at 41 lights).
+// Each batch ends every bounce's launch on its slowest rays, about 3 ms in all
+// on 128 environments of 512x512 at 8 spp, which counts for less the more
+// shadow rays a path has.  Batches of 32M and 64M paths:
+//   lights   environments     1080p at 32 spp   720p projector at 64 spp
+//   2        144 / 132 ms     32.3 / 30.6       42.7 / 40.8
+//   5        210 / 193        54.8 / 51.6       60.5 / 58.6
+//   13       486 / 468        124 / 121         147 / 145
+//   25       981 / 958        237 / 232         304 / 298
+uint32_t default_batch(uint32_t spp, uint32_t WH, uint32_t nslots) {
+    const size_t paths = std::clamp<size_t>(((size_t)32 << 30) / state_bytes(1, nslots), 32u << 20, 64u << 20);
+    return (uint32_t)std::max<size_t>(1, std::min<size_t>(spp, paths / std::max<uint32_t>(WH, 1)));
 }
 
 // Default bounce from which the tail kernels carry the paths (nb: never).
@@ -1621,7 +1626,7 @@ void render_frame(Renderer* r, Scene* s, uint32_t n_env, const kf_camera_ubo* ca
     uint32_t WH = r->W * r->H;
     uint32_t spb = o.samples_per_batch ? o.samples_per_batch : r->tune.spb;
     const uint32_t K = inline_nee ? 1u : (uint32_t)std::max(L.n_slots, 1);
-    if (spb == 0) spb = default_batch(pc->spp, WH);
+    if (spb == 0) spb = default_batch(pc->spp, WH, K);
     spb = std::min(spb, pc->spp);
     // A default batch that the buffers held do not take already leaves a quarter
     // of the free memory to others, and is halved where it does not fit after

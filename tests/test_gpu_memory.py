@@ -49,6 +49,20 @@ def test_paths_and_slots_have_capacities_of_their_own(gpu):
     assert np.array_equal(r.read(0), want)
 
 
+# 4.2 M pixels at 16 samples: 67 M paths of 270 bytes, and, with 684 bytes
+# each, as many as stay within 32 GiB.
+@pytest.mark.parametrize("lights,batches", [(2, 1), (8, 2)])
+def test_default_batch_by_the_state_of_its_paths(gpu, lights, batches):
+    w = with_lights(scenes.config1(2048, 2048, spp=16, path_depth=1), lights)
+    gs, r = GpuScene(w.data), Renderer(2048, 2048)
+    r.render(gs, w.cam, w.pc, samples_per_batch=1)  # targets, camera rays' tree
+    before = free_bytes()
+    st = r.render(gs, w.cam, w.pc)
+    assert before - free_bytes() < 32 * GIB
+    assert st.shadow_launches == 2 * batches
+    r.close()
+
+
 @pytest.fixture
 def scarce(gpu):
     """scarce(n): leaves n bytes of GPU memory free until the test ends."""
