@@ -400,12 +400,13 @@ int kf_render_envs(kf_renderer* r, kf_scene* s, uint32_t num_envs, const kf_came
  * in a forward and a backward sweep; keeps the fastest for later frames
  * rendered with samples_per_batch = 0.  Images do not depend on the
  * schedule.  Renders into r's targets (frame_count 0). */
+#define KF_TAIL_NEVER 64 /* a tail_bounce beyond the last bounce of any frame */
 typedef struct kf_tune_result {
     uint32_t samples_per_batch, refill, grab; /* grab: largest reservation per wave (smaller once its queue runs short) */
     float frame_ms;    /* kernel time of a frame with the picked schedule */
     float default_ms;  /* ... with the built-in default */
     uint32_t trials;   /* frames timed */
-    uint32_t tail_bounce; /* bounce from which one thread carries each path to its end (path_depth + 1: never) */
+    uint32_t tail_bounce; /* bounce from which one thread carries each path to its end (KF_TAIL_NEVER: never) */
     uint32_t grab0;       /* queries reserved per wave for the camera rays (0: grab) */
     uint32_t grab_shadow; /* ... for the shadow rays (0: grab) */
     uint32_t tail_pairs;  /* 1: two lanes per path carry the tail bounces while few paths remain (at most an
@@ -415,8 +416,9 @@ int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_envs, const k
                          const kf_push_constants* pc, kf_tune_result* out);
 /* Set the schedule directly (e.g. one kf_renderer_autotune picked earlier);
  * 0 keeps the built-in default of that parameter (for tail_bounce: chosen by
- * the number of paths and lights; a value beyond the last bounce runs every
- * bounce in the wavefront; for grab0 and grab_shadow, the camera rays' and
+ * the number of paths and lights, as for a renderer without a schedule; a
+ * value beyond the frame's last bounce runs every bounce in the wavefront,
+ * KF_TAIL_NEVER does so at any path depth; for grab0 and grab_shadow, the camera rays' and
  * the shadow rays' largest reservations: grab).  refill is clamped to [1, 64],
  * the reservations to [16, 4096]. */
 int kf_renderer_set_schedule(kf_renderer* r, uint32_t samples_per_batch, uint32_t refill, uint32_t grab,

@@ -42,6 +42,7 @@ static_assert(TB == (int)kRingThreads, "traversal kernels index their LDS stack 
 // rays).  Then, per bounce, the work chunks of k_extend and of k_shadow (8
 // each, kChunkStride apart).
 constexpr int kMaxBounces = 64;
+static_assert(KF_TAIL_NEVER >= kMaxBounces, "beyond the last bounce of any frame");
 constexpr int kCntFields = 3;
 constexpr int kCntPerBounce = kCntFields * (int)kChunkStride;
 constexpr int kCntPaths = 0, kCntShadow = (int)kChunkStride, kCntExtQueue = 2 * (int)kChunkStride;
@@ -2072,10 +2073,10 @@ extern "C" int kf_renderer_autotune(kf_renderer* r, kf_scene* s, uint32_t num_en
         std::vector<uint32_t> refills = {8u, 16u, 32u, 48u};
         if (std::find(refills.begin(), refills.end(), b_refill) == refills.end()) refills.push_back(b_refill);
         // the bounce from which k_tail finishes the paths: never (beyond the
-        // last bounce), or from bounce 1 up to the first bounces after Russian roulette starts (few
-        // paths per frame favour an early tail: at 1 spp of the 1080p scene
-        // bounce 3 beats bounce 5 by 8 %)
-        std::vector<uint32_t> tails = {p.path_depth + 1u};
+        // last bounce of any frame), or from bounce 1 up to the first bounces
+        // after Russian roulette starts (few paths per frame favour an early
+        // tail: at 1 spp of the 1080p scene bounce 3 beats bounce 5 by 8 %)
+        std::vector<uint32_t> tails = {KF_TAIL_NEVER};
         for (uint32_t tb = 1u; tb < std::min<uint32_t>(p.path_depth + 1u, p.rr_min_bounces + 4u); ++tb)
             tails.push_back(tb);
         sweep(spbs, b_spb, 0);

@@ -307,3 +307,20 @@ def test_default_schedule_equals_wavefront(gpu, w, h, spp, extra, rr):
     for t in range(3):
         assert np.array_equal(ra.read(t), rb.read(t))
     assert (sa.primary_rays, sa.extension_rays, sa.shadow_rays) == (sb.primary_rays, sb.extension_rays, sb.shadow_rays)
+
+
+@pytest.mark.parametrize("depth", [2, 8])
+def test_tail_bounce_of_a_schedule(gpu, depth):
+    """In a schedule 0 leaves the tail bounce to the renderer, and never is a
+    value beyond the last bounce; the tuner's (all that it can pick for frames
+    of one bounce) is never for deeper frames too."""
+    w = scenes.config1(64, 48, spp=2, path_depth=depth)
+    gs, r = GpuScene(w.data), Renderer(64, 48)
+    for schedule, used in ((None, True), (0, True), (2, True), (depth + 1, False), (64, False)):
+        if schedule is not None:
+            r.set_schedule(tail_bounce=schedule)
+        assert (r.render(gs, w.cam, w.pc).tail_rays > 0) == used
+    w.pc.path_depth = 0
+    assert r.autotune(gs, w.cam, w.pc)["tail_bounce"] == 64
+    w.pc.path_depth = depth
+    assert r.render(gs, w.cam, w.pc).tail_rays == 0
