@@ -619,14 +619,17 @@ int kf_scene_read_bvh4(kf_scene* s, int which, float* nodes, uint32_t max_nodes,
         if (nodes && nn) {
             if (max_nodes < nn) throw Error("kf_scene_read_bvh4: node buffer too small");
             KF_CHECK(hipMemcpy(nodes, src, nn * sizeof(Node4), hipMemcpyDeviceToHost));
-            // lox, loy, loz, hix, hiy, hiz on the device; lox, hix, loy, hiy, loz, hiz here
-            float4* q = (float4*)nodes;
-            for (uint32_t i = 0; i < nn; ++i, q += 8) {
-                const float4 ly = q[1], lz = q[2], hx = q[3], hy = q[4];
-                q[1] = hx;
-                q[2] = ly;
-                q[3] = hy;
-                q[4] = lz;
+            // lox, loy, loz, hix, hiy, hiz on the device; lox, hix, loy, hiy,
+            // loz, hiz here.  Single floats: the caller's buffer is aligned
+            // for nothing wider.
+            float* q = nodes;
+            for (uint32_t i = 0; i < nn; ++i, q += sizeof(Node4) / sizeof(float)) {
+                float line[16];
+                std::memcpy(line, q + 4, sizeof(line));
+                std::memcpy(q + 4, line + 8, 16);
+                std::memcpy(q + 8, line, 16);
+                std::memcpy(q + 12, line + 12, 16);
+                std::memcpy(q + 16, line + 4, 16);
             }
         }
         if (roots) {

@@ -9,6 +9,7 @@
   required within 1e-4 relative for >= 99.9 % of samples (bit equality is
   expected); rgba running mean, albedo and normal targets likewise.
 """
+import ctypes as C
 import math
 from concurrent.futures import ThreadPoolExecutor
 
@@ -349,6 +350,21 @@ def walk_bvh4(nodes, root, leaf_box_check, inner_kind):
                 leaves.append(idx)
                 leaf_box_check(idx, lo[c], hi[c])
     return seen, leaves
+
+
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_bvh4_into_a_buffer_aligned_for_floats(gpu, shift):
+    """The nodes arrive whole in a buffer that starts 4, 8 or 12 bytes off a
+    16-byte line."""
+    gs = GpuScene(scenes.config1().data)
+    for which in (0, 1):
+        want, _ = gs.read_bvh4(which)
+        raw = np.zeros(want.size + 8, np.float32)
+        at = (-raw.ctypes.data // 4) % 4 + shift
+        n = C.c_uint32()
+        abi.check(abi.lib().kf_scene_read_bvh4(gs.h, which, raw.ctypes.data + 4 * at, len(want), C.byref(n), None, 0))
+        assert (raw.ctypes.data + 4 * at) % 16 == 4 * shift and n.value == len(want)
+        assert raw[at:at + want.size].tobytes() == want.tobytes()
 
 
 def check_blas4(gs, s):
