@@ -1496,6 +1496,9 @@ void refit_blas(Scene& s, uint32_t g) {
     const uint32_t n = s.h_toff[g + 1] - s.h_toff[g];
     if (n == 0) return;
     // the slots' boxes and their pyramid, in a workspace that the scene keeps
+    // (96 bytes per triangle, half of what the geometry's own arrays take;
+    // allocated per call an update of 1.3 M triangles takes 1.91 ms instead of
+    // 1.58)
     const size_t need = 2 * (size_t)n * sizeof(float4) + pyramid_size(n) * sizeof(Box);
     if (need > s.refit_cap) {
         dfree(s.d_refit);

@@ -174,7 +174,7 @@ struct Scene {
     uint32_t* d_node_off = nullptr;          // h_node_off on the device
     uint32_t* d_blas_cnt = nullptr;          // 2 collapse counters per geometry: [2g] = next free BVH4 slot
     std::vector<kf_instance> h_inst;         // instances of the last TLAS build (for rebuilds after a refit)
-    uint8_t* d_refit = nullptr;              // workspace of refits (the largest geometry refitted so far)
+    uint8_t* d_refit = nullptr;              // workspace of refits: 96 B per triangle of the largest geometry refitted so far
     size_t refit_cap = 0;
     uint8_t* h_vstage = nullptr;             // pinned staging of geometry vertex updates
     size_t vstage_cap = 0;
@@ -234,7 +234,7 @@ struct Scene {
     struct Trace {
         std::mutex mu;
         unsigned long long* d_cnt = nullptr;
-        uint8_t* d_buf = nullptr;   // rays and results of larger batches
+        uint8_t* d_buf = nullptr;   // rays and results of larger batches (kKeepBytes at most)
         uint8_t* h_pin = nullptr;   // pinned: overflow flag, rays and results of small batches
         size_t dev_cap = 0, pin_cap = 0;
     } trace;

@@ -158,9 +158,12 @@ namespace {
 // rays 206 and 139 us, 131072 rays 478 and 395, 262144 rays 836 and 702; any
 // hit 162 and 117, 272 and 237, 414 and 407.  The line bounds a scene's pinned
 // memory at 7 MB.  Beyond it the device buffers are kept up to kKeepBytes, and
-// allocated for the call above that.
+// allocated for the call above that, where the 45 us count for less (131073,
+// 262144, 524288 and 1048576 rays kept 470, 775, 1420 and 2830 us, allocated
+// 515, 825, 1460 and 2900): a scene holds on to 16 MiB at most, not to what
+// its largest batch took.
 constexpr uint32_t kDirectRays = 131072;
-constexpr size_t kKeepBytes = (size_t)64 << 20;
+constexpr size_t kKeepBytes = (size_t)16 << 20;
 constexpr size_t kCntBytes = (kTraceCnt * sizeof(unsigned long long) + 255) / 256 * 256;
 
 struct Temp {  // device memory of one call

@@ -136,3 +136,18 @@ def test_failed_autotune_keeps_the_schedule(gpu):
     with pytest.raises(KuafuError, match="depth"):
         r.autotune(gs, deep.cam, deep.pc)
     assert r.render(gs, w.cam, w.pc).extend_launches == before == 4 * 3
+
+
+def test_a_scene_does_not_keep_its_largest_ray_batch(gpu):
+    """A batch of 1 M rays (59 MB of rays and hits) leaves a scene with the 16
+    MiB at most that smaller batches keep."""
+    gs = GpuScene(scenes.config1().data)
+    rng = np.random.default_rng(3)
+    rays = np.zeros(1 << 20, abi.RAY_DTYPE)
+    rays["org"], rays["tmax"] = rng.uniform(-2, 2, (len(rays), 3)), 10.0
+    rays["dir"] = rng.normal(size=(len(rays), 3))
+    few = gs.trace_closest(rays[:1000])  # pinned memory, counters
+    before = free_bytes()
+    for n in (1 << 20, 1 << 18, 400000):
+        assert gs.trace_closest(rays[:n])[:1000].tobytes() == few.tobytes()
+        assert before - free_bytes() <= 16 << 20
