@@ -324,3 +324,63 @@ def test_tail_bounce_of_a_schedule(gpu, depth):
     assert r.autotune(gs, w.cam, w.pc)["tail_bounce"] == 64
     w.pc.path_depth = depth
     assert r.render(gs, w.cam, w.pc).tail_rays == 0
+
+
+def _against_wavefront(wl, tail, pairs):
+    """Frames with a renderer's own schedule (tail None) or a pinned tail bounce
+    against the wavefront for every bounce: targets and ray counts.  Returns
+    the launches of the closest-hit wavefront, one per bounce before the tail
+    and batch."""
+    gs = GpuScene(wl.data)
+    ra, rb = Renderer(wl.width, wl.height), Renderer(wl.width, wl.height)
+    if tail is not None:
+        ra.set_schedule(tail_bounce=tail, tail_pairs=pairs)
+    rb.set_schedule(tail_bounce=64)
+    sa = ra.render(gs, wl.cam, wl.pc, seed=3)
+    sb = rb.render(gs, wl.cam, wl.pc, seed=3)
+    assert sb.tail_rays == 0
+    for t in range(3):
+        assert np.array_equal(ra.read(t), rb.read(t))
+    assert (sa.primary_rays, sa.extension_rays, sa.shadow_rays) == (sb.primary_rays, sb.extension_rays, sb.shadow_rays)
+    ra.close(), rb.close()
+    return sa.extend_launches
+
+
+# The lines of the default tail bounce: 786432 and 4194304 paths with up to two
+# lights, 393216 and 1572864 with three, the latter with four, 8388608 (up to
+# which it is 3, beyond which one after Russian roulette may first end paths),
+# more than four lights, no Russian roulette.  On each line and one column
+# beyond it.
+@pytest.mark.parametrize("w,h,spp,lights,rr,tail", [
+    (1024, 768, 1, 2, True, 1), (1025, 768, 1, 2, True, 2), (2048, 2048, 1, 2, True, 2), (2049, 2048, 1, 2, True, 3),
+    (2048, 2048, 2, 2, True, 3), (2049, 2048, 2, 2, True, 4), (2049, 2048, 1, 2, False, 7), (768, 512, 1, 3, True, 1),
+    (769, 512, 1, 3, True, 2), (1024, 768, 2, 3, True, 2), (1025, 768, 2, 3, True, 3), (768, 512, 1, 4, True, 2),
+    (1024, 768, 2, 4, True, 2), (1025, 768, 2, 4, True, 3), (64, 64, 1, 5, True, 7)])
+def test_default_tail_at_its_lines(gpu, w, h, spp, lights, rr, tail):
+    wl = scenes.config1(w, h, spp=spp, path_depth=6)  # a directional and a point light
+    for k in range(lights - 2):
+        wl.data.add_point_light((k - 1.0, 3.0, 2.0), (1, 1, 1), 4.0, radius=0.0)
+    wl.pc.russian_roulette, wl.pc.rr_min_bounces = int(rr), 3
+    assert _against_wavefront(wl, None, 1) == tail
+
+
+def test_tail_kernels_around_the_pair_capacity(gpu):
+    """k_tail2 takes the paths while every eighth thread of the launch can have
+    one (65536 on 256 CUs), k_tail beyond: frames whose paths at bounce 1, 145
+    per column, are the most that fit and the fewest that do not."""
+    def live(w):
+        wl = scenes.config1(w, 256, spp=1, path_depth=1)
+        r = Renderer(w, 256)
+        r.set_schedule(tail_bounce=64)
+        n = r.render(GpuScene(wl.data), wl.cam, wl.pc, seed=3).extension_rays
+        r.close()
+        return n
+
+    lo, hi = 400, 560
+    assert live(lo) <= 65536 < live(hi)
+    while hi - lo > 1:
+        mid = (lo + hi) // 2
+        lo, hi = (mid, hi) if live(mid) <= 65536 else (lo, mid)
+    assert 65000 < live(lo) <= 65536 < live(hi) < 66000
+    for w in (lo, hi):
+        assert _against_wavefront(scenes.config1(w, 256, spp=1, path_depth=6), 1, 1) == 1
