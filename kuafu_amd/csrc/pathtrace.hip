@@ -1560,7 +1560,7 @@ uint32_t default_tail(const kf_push_constants& pc, uint64_t paths, uint32_t ligh
     if (paths <= (lights <= 2 ? 3u << 18 : 3u << 17) && lights <= 3) return 1;
     if (paths <= (lights <= 2 ? 1u << 22 : 3u << 19)) return 2;
     if (!pc.russian_roulette) return nb;
-    return paths <= (8u << 20) ? 3 : pc.rr_min_bounces + 1;
+    return paths <= (8u << 20) ? 3 : std::min(pc.rr_min_bounces, nb) + 1;
 }
 
 void build_light_list(const Scene& s, DevLights& L, bool& inline_nee) {

@@ -384,3 +384,11 @@ def test_tail_kernels_around_the_pair_capacity(gpu):
     assert 65000 < live(lo) <= 65536 < live(hi) < 66000
     for w in (lo, hi):
         assert _against_wavefront(scenes.config1(w, 256, spp=1, path_depth=6), 1, 1) == 1
+
+
+def test_default_tail_without_an_end_to_the_first_bounces(gpu):
+    """Russian roulette after 2^32 - 1 bounces is none: beyond 8 M paths the
+    wavefront runs every bounce."""
+    wl = scenes.config1(2049, 2048, spp=2, path_depth=6)
+    wl.pc.rr_min_bounces = 0xFFFFFFFF
+    assert _against_wavefront(wl, None, 1) == 7
