@@ -1550,11 +1550,15 @@ uint32_t default_batch(uint32_t spp, uint32_t WH, uint32_t nslots) {
 //   4.1 M paths, 256 icospheres    5.32 / 4.26 / 4.12 / 4.62 ms, 9 spheres 5.12 / 3.80 / 3.94 / 4.07
 //   6.3 M paths, projector         9.12 / 6.46 / 6.17 / 6.46 ms
 //   17 M paths, 256 icospheres     14.7 / 10.4 / 8.56 / 8.04 ms
-// The shadow rays of all lights are part of a path's chain.  256 k paths on
-// the config-1 spheres, never / from bounce 1 / 2 (before the tail ran three
-// waves per SIMD): 1.48 / 1.07 / 1.09 ms with 2 lights, 1.63 / 1.38 / 1.33 with
-// 3, 1.69 / 1.71 / 1.61 with 4, 1.99 / 2.47 / 2.23 with 8, 3.18 / 7.84 / 7.48
-// with 32; the lines for three and four lights are those of that time.
+// The shadow rays of all lights are part of a path's chain.  From bounce 1 / 2 /
+// 3 / never, with three lights (four are 0.1-0.3 ms slower, in the same order):
+//   393 k paths  256 icospheres 1.70 / 1.63 / 1.78 / 2.24 ms, 9 spheres 1.15 / 1.29 / 1.37 / 1.59,
+//                projector 1.39 / 1.39 / 1.48 / 1.79
+//   786 k paths  2.08 / 2.12 / 2.03 / 2.56, 1.76 / 1.67 / 1.77 / 1.95, 1.97 / 1.72 / 1.79 / 2.12
+//   1.57 M paths 2.92 / 2.54 / 2.55 / 3.03, 2.49 / 2.02 / 2.16 / 2.41, 3.22 / 2.43 / 2.45 / 2.76
+//   2.62 M paths 3.87 / 3.35 / 3.23 / 3.63, 3.51 / 2.74 / 2.76 / 2.98, 4.80 / 3.33 / 3.30 / 3.64
+// 256 k paths, 9 spheres, never / from bounce 1 / 2 (before the tail ran three
+// waves per SIMD): 1.99 / 2.47 / 2.23 ms with 8 lights, 3.18 / 7.84 / 7.48 with 32.
 uint32_t default_tail(const kf_push_constants& pc, uint64_t paths, uint32_t lights, uint32_t nb) {
     if (lights > 4) return nb;
     if (paths <= (lights <= 2 ? 3u << 18 : 3u << 17) && lights <= 3) return 1;
