@@ -1053,7 +1053,8 @@ KF_DEV bool connect_path(const Frame& F, int bounce, uint32_t p, float4* __restr
     float4 t4 = first ? kPathStart : thr[p];
     v3 weight = xyz(t4);
     uint32_t depth = __float_as_uint(t4.w);
-    v3 color = first ? splat(0.0f) : xyz(col[p]);
+    const float4 c4 = first ? make_float4(0.f, 0.f, 0.f, 0.f) : col[p];
+    v3 color = xyz(c4);
     const float4 r4 = rw[p];  // BSDF weight, or the emission that ends the path
     const bool term = __float_as_uint(r4.w) != 0u;
     uint32_t rs = seed[p];
@@ -1076,9 +1077,14 @@ KF_DEV bool connect_path(const Frame& F, int bounce, uint32_t p, float4* __restr
             shadow = (sd + sp) + sa;
         }
     }
-    // rgen:109-138; without emission the product still adds 0 x weight
+    // rgen:109-138; without emission the product still adds 0 x weight, and at
+    // the end of a path the shadow term 0 x (weight x the last BSDF weight),
+    // which is no zero where that product overflows: bits 2:0 of col.w say
+    // where it does
     color = color + (term ? xyz(r4) : splat(0.0f)) * weight;
-    weight = weight * (term ? splat(first ? 0.0f : 1.0f) : xyz(r4));
+    const uint32_t over = __float_as_uint(c4.w);
+    if (term) weight = mk(over & 1u ? INFINITY : 0.0f, over & 2u ? INFINITY : 0.0f, over & 4u ? INFINITY : 0.0f);
+    else weight = weight * xyz(r4);
     color = color + shadow * weight;
     uint32_t d2 = term ? maxDepth + 1 : depth;
     cont = true;
@@ -1093,8 +1099,11 @@ KF_DEV bool connect_path(const Frame& F, int bounce, uint32_t p, float4* __restr
     uint32_t nd = d2 + 1;
     if (nd > maxDepth) cont = false;
     if (cont) {
+        const v3 last = weight * xyz(r4);
+        const uint32_t o = (__builtin_isfinite(last.x) ? 0u : 1u) | (__builtin_isfinite(last.y) ? 0u : 2u) |
+                           (__builtin_isfinite(last.z) ? 0u : 4u);
         thr[p] = f4(weight, __uint_as_float(nd));
-        col[p] = f4(color, 0.0f);
+        col[p] = f4(color, __uint_as_float(o));
         seed[p] = rs;
     } else {
         out[p] = f4(color, 0.0f);

@@ -263,3 +263,20 @@ def test_render_parity_light_counts(gpu, points, active):
     full.set_schedule(tail_bounce=w.pc.path_depth + 1)
     full.render(GpuScene(w.data), w.cam, w.pc, seed=0, keep_samples=True)
     assert full.read_samples(w.pc.spp).tobytes() == res[1].tobytes()
+
+
+@pytest.mark.parametrize("diffuse,depth", [(1e19, 4), (1e13, 4), (1e10, 6)])
+def test_render_parity_where_weights_overflow(gpu, diffuse, depth):
+    """At the end of a path the shader still adds 0 x (throughput x the last
+    BSDF weight): NaN where that overflows, per sample as in the oracle."""
+    w = scenes.config1(48, 32, spp=3, path_depth=depth)
+    for m in w.data.materials[:3]:
+        m["diffuse"][:3] = (diffuse, 0.5, 0.7)
+    gs, ref = GpuScene(w.data), oracle.Scene(w.data).render(w.cam, w.pc, w.width, w.height, seed=0, keep_samples=True)
+    for tail in (0, 1, 64):
+        rd = Renderer(w.width, w.height)
+        rd.set_schedule(tail_bounce=tail)
+        rd.render(gs, w.cam, w.pc, seed=0, keep_samples=True)
+        got = rd.read_samples(w.pc.spp)
+        assert np.array_equal(np.isnan(got), np.isnan(ref["samples"]))
+        assert np.isnan(got[..., 0]).any()
