@@ -295,7 +295,11 @@ __global__ __launch_bounds__(TB) void k_tile_roots(SceneView S, Frame F, const N
                     const float4 lo = ilo[ci], hi = ihi[ci];
                     const DV m = {0.5 * ((double)lo.x + hi.x), 0.5 * ((double)lo.y + hi.y),
                                   0.5 * ((double)lo.z + hi.z)};
-                    const double key = dv_dot(dv_sub(m, o), ctr);
+                    // a box without a centre (infinite vertices) comes last:
+                    // among NaN keys the ranks would not be a permutation, and
+                    // the list below would hold indices that nobody wrote
+                    const double depth = dv_dot(dv_sub(m, o), ctr);
+                    const double key = depth == depth ? depth : INFINITY;
                     rank = 0;
                     for (uint32_t j = 0; j < k; ++j) {
                         const double kj = __shfl(key, (int)j);

@@ -131,3 +131,16 @@ def test_tile_roots_graph_replays(gpu):
         for k in range(3):
             assert same(rg.read(k), re_.read(k)), "frame %d target %d" % (f, k)
     assert rg.render(gs, base, pc, seed=9, use_graph=True).graph_captures == 1
+
+
+def test_tile_roots_with_infinite_boxes(gpu):
+    """Boxes without a centre among a tile's 5 to 16 candidates: geometries
+    with an infinite vertex, whose boxes reach from -infinity to infinity once
+    they are turned."""
+    w = scenes.config2(width=96, height=56, spp=2, path_depth=3, n_inst=30, subdiv=2)
+    for k in (0, 3, 11, 12, 20, 29):
+        v, *rest = w.data.geoms[k]
+        v = v.copy()
+        v["pos"][7 * k % len(v)] = np.inf
+        w.data.geoms[k] = (v, *rest)
+    _assert_same_frames(w, expect_fewer=False)
