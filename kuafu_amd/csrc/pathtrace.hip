@@ -125,12 +125,11 @@ __global__ void k_zero(unsigned long long* c, int nb, int globals) {
 // meet the pyramid and gives the tile a root item over just those: none ->
 // the empty item, one -> the instance, 2-4 -> one node, 5-16 -> a node over
 // up to four groups in depth order; more, or a camera with an aperture (rays
-// from a disc), -> the environment's TLAS root.  The closest hit does not
-// depend on the order in which records are visited (smallest t, ties by
-// instance and primitive), each instance keeps its TLAS leaf box, and a node
-// box here is the exact union of its children's, so camera rays find the hits
-// they find through the full TLAS.  Later bounces and shadow rays start from
-// the environment's root.
+// from a disc), -> the environment's TLAS root.  Each instance keeps its TLAS
+// leaf box, and a node box here is the exact union of its children's, so camera
+// rays find the hits they find through the full TLAS, up to the order of
+// surfaces a few roundings of t apart (ChildOrder in traverse.h).  Later
+// bounces and shadow rays start from the environment's root.
 constexpr uint32_t kTile = 8, kTileNodes = 5, kTileMax = 16;
 // The pyramid's planes pass half a pixel outside the tile, and each of the
 // tile's rays must lie at least this angle (radians) inside every plane, far
