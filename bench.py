@@ -7,10 +7,12 @@ HBM before timing starts.
 
 value = rays traced (primary + extension + shadow, counted on the device) /
 wall time of the K timed frames / 1e6  [Mrays/s].
-roofline = the closest-hit traversal kernel (k_extend): algorithmic bytes per
-ray = 32 (ray) + 20 (hit) + 128 * BVH4 node visits + 192 * instance records
-(each with its BLAS root node) + 48 * triangle tests, counted by the
-instrumented traversal on the same frame, / the kernel's HIP-event time.
+roofline = the closest-hit traversal kernel (k_extend): what it moves to and
+from memory (rocprofv3 counters of the same schedule, profiles/) / its HIP-event
+time, against HBM; vector ALUs and the vector L1 bound it.  record_gbs prices
+every record it reads, most of them from caches: per ray 32 (ray) + 20 (hit) +
+128 * BVH4 node visits + 192 * instance records (each with its BLAS root node)
++ 48 * triangle tests, counted by the instrumented traversal on the same frame.
 cpu_baseline = the FP32 CPU oracle on a bounded band of rows of the same frame.
 """
 import argparse
@@ -455,7 +457,7 @@ def main():
     insts_per_ray = cst.instance_visits / max(closest, 1)
     tris_per_ray = cst.tri_tests / max(closest, 1)
     bytes_per_ray = 32 + 20 + 128 * nodes_per_ray + 192 * insts_per_ray + 48 * tris_per_ray
-    achieved = bytes_per_ray * ext_rays / (ext_ms * 1e-3) / 1e9
+    record_gbs = bytes_per_ray * ext_rays / (ext_ms * 1e-3) / 1e9
     # HBM traffic per launch is not measurable from inside the process: it
     # comes from the committed rocprofv3 counter profile of this kernel on
     # this scene and schedule (FETCH_SIZE and WRITE_SIZE, each scaled by what
@@ -469,11 +471,11 @@ def main():
         tsrc = ("profiles/extend_traffic_config2.json (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE of k_extend<false>, "
                 "schedule %s, build %s, %s)" % (tj.get("schedule", "?"), tj.get("build", "?"), tj.get("date", "?")))
     avg_ms = ext_ms / max(launches, 1)
+    # without the counters: the ray and hit records alone
+    achieved = (traffic if traffic else 52 * ext_rays / max(launches, 1)) / (avg_ms * 1e-3) / 1e9
     roof = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": tsrc,
-            "dram_gbs": round(traffic / (avg_ms * 1e-3) / 1e9, 1) if traffic else None,
-            "dram_frac": round(traffic / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
-            "kernel": "k_extend (closest-hit traversal)",
+            "record_gbs": round(record_gbs, 1), "kernel": "k_extend (closest-hit traversal)",
             "bytes_per_ray": round(bytes_per_ray, 1), "node_visits_per_ray": round(nodes_per_ray, 2),
             "instance_visits_per_ray": round(insts_per_ray, 2), "tri_tests_per_ray": round(tris_per_ray, 2),
             "tlas_node_visits_per_ray": round(cst.tlas_node_visits / max(closest, 1), 2),

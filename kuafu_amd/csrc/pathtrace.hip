@@ -449,7 +449,7 @@ __global__ __launch_bounds__(TB) void k_raygen(SceneView S, Frame F, const uint2
 // fits when it is alone and keeps them out: 1080p frame 18.0 ms against 17.0
 // (kExtendBlocks; within 1 % for the camera rays, which have none beside
 // them).  At 80 VGPRs (40 spilled) the frame took 37 ms.
-// Bound by the vector ALUs (1080p frame: busy 74 % of the SIMD cycles, with 25 %
+// Bound by the vector ALUs (1080p frame: busy 75 % of the SIMD cycles, with 24 %
 // less instructions than before) and by the vector L1, one lane's line per
 // cycle and CU (0.72 of it).  amdgpu_num_vgpr counts in units of two registers on gfx950 (the
 // unified VGPR/AGPR file).

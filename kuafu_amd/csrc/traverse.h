@@ -338,7 +338,7 @@ template <> struct ChildOrder<true> {
 // coin (alpha_coin).  MIXED (with ANY false): each lane's query is a shadow
 // query or a closest-hit one (any_q), so that lanes of one wave trace both
 // kinds with the same steps.
-// What bounds it: the vector ALUs (about 340 instructions per step) and the
+// What bounds it: the vector ALUs (about 345 instructions per step) and the
 // vector L1 about equally.  Each lane loading its own record's lines only, the
 // shear axes as scalar logic and a stack without a cached top took 17 % of the
 // vector instructions and 26 % of the L1 accesses:
