@@ -415,6 +415,7 @@ class Renderer:
     def set_schedule(self, samples_per_batch=0, refill=0, grab=0, tail_bounce=0, grab0=0, grab_shadow=0,
                      tail_pairs=1):
         """grab0 / grab_shadow: reservation per wave for the camera / shadow rays (0: grab);
+        tail_bounce 0: chosen by the number of paths and lights, 64 (KF_TAIL_NEVER): never;
         tail_pairs 1: two lanes per path may carry the tail bounces, 0: one lane."""
         check(lib().kf_renderer_set_schedule(self.h, samples_per_batch, refill, grab, tail_bounce, grab0,
                                              grab_shadow))
